@@ -171,8 +171,9 @@ WC_API int wc_density(wc_ctx* ctx);
 /* Fluid::runUpdateProg(buffer2, buffer1, dt) (src/core/Fluid.cpp:294-321): update.comp:134-232.
  * `dt` is the integration step itself (the reference passes frame time * time_scale_).  Reads
  * the densities and pressures of the preceding wc_density on the same sort, as the reference's
- * pass order does.  The sort and the density pass also check that every position, velocity,
- * density and pressure is 0 or within [2^-40, 2^40] in magnitude; when they are, the pass forms
+ * pass order does.  The sort and the density pass also check that every position is 0 or within
+ * [2^-20, 2^20] in magnitude, and every velocity, density and pressure 0 or within [2^-40, 2^40];
+ * when they are, the pass forms
  * each neighbour's quotients from shared reciprocals (same bits as IEEE division), otherwise,
  * and when no density pass followed the last sort, it divides as IEEE does. */
 WC_API int wc_update(wc_ctx* ctx, float dt);
@@ -271,9 +272,12 @@ WC_API const char* wc_pass_name(int k);
 
 /* Tuning of the two neighbour passes (density, force).  Variant v in [0, wc_num_variants()) is
  * a (threads per workgroup, LDS list entries per lane, neighbour slots in flight per lane, drain
- * the list after every dx plane or only when full) choice; every variant computes bit-identical
- * results, only speed differs.  No reference
- * counterpart: the reference dispatches fixed 128-invocation work groups (src/core/util.h:18). */
+ * the list after every dx plane or only when full) choice of a particle per lane; the last variant
+ * stages boxes of cells in LDS instead (both passes of it run together; without the memory for it,
+ * or on a grid of more than 64 cells a particle, it stands for variant 2).  Every variant computes
+ * bit-identical results, only speed differs.  Contexts of 50,000 particles and more start with the
+ * last variant, smaller ones with variant 2.  No reference counterpart: the reference dispatches
+ * fixed 128-invocation work groups (src/core/util.h:18). */
 typedef struct wc_tuning {
     int32_t density_variant;
     int32_t update_variant;

@@ -1,0 +1,94 @@
+"""The tile passes (the last tuning variant) against the oracle, bit for bit, at the edges of their boxes."""
+import numpy as np
+import pytest
+
+from watercube_amd import Fluid
+from watercube_amd import _lib as L
+from watercube_amd.scenes import scaled_block
+
+pytestmark = pytest.mark.gpu
+
+
+
+def _clustered(oracle_params, parts, cells, seed):
+    """`parts` and clusters of m particles inside the grid cells `cells` = [(cell, m)], shuffled."""
+    rng = np.random.default_rng(seed)
+    b = float(oracle_params.bin_size)
+    add = []
+    for cell, m in cells:
+        rec = np.zeros(m, L.PARTICLE_DTYPE)
+        lo = np.array(cell, np.float64) * b
+        rec["position"] = rng.uniform(lo + 0.05 * b, lo + 0.95 * b, (m, 3)).astype(np.float32)
+        add.append(rec)
+    out = np.concatenate([parts] + add)
+    return out[rng.permutation(len(out))]
+
+
+def _case(name):
+    if name == "4x2x2, 12 a cell":  # sides that no box divides
+        return scaled_block((23, 17, 19), 0.027, 1, 2.3)
+    if name == "2x2x2, 51 a cell":  # more neighbours than the context's lists hold
+        return scaled_block((23, 17, 19), 0.027, 1, 3.5)
+    if name == "4x4x2":
+        return scaled_block((47, 43, 47), 0.017, 2)
+    if name == "4x4x3":
+        return scaled_block((53, 57, 59), 0.0151, 3)
+    if name == "one cell":  # a grid that is a single box
+        p, parts = scaled_block((4, 5, 4), 0.2, 4)
+        p.grid_res = 1
+        p.bin_size = p.size
+        return p, parts
+    small = name.startswith("small")
+    p, parts = scaled_block((20, 20, 20) if small else (53, 57, 59), 0.03 if small else 0.0151, 5)
+    if "split" in name:    # boxes over the records that LDS holds: parts of 2x2x2, single cells
+        cells = [((3, 3, 2), 900), ((6, 4, 4), 700), ((7, 7, 7), 500)]
+    elif "long" in name:   # lists at and over their 512 entries, a cell that fits LDS
+        cells = [((5, 5, 5), 513), ((2, 9, 3), 514), ((9, 2, 9), 800)]
+    else:                  # a cell over them, searched directly; its neighbours too
+        cells = [((5, 5, 5), 2600), ((8, 2, 3), 2305)]
+    parts = _clustered(p, parts, cells, 7)
+    if "odd positions" in name:  # a box with a position outside the shared arithmetic's range, NaN among them
+        parts["position"][11] = (1e-12, 0.2, 0.2)
+        parts["position"][12] = (np.nan, 0.1, 0.1)
+        parts["position"][13] = (5.0, -3.0, 0.4)
+    p.num_particles = len(parts)
+    return p, parts
+
+
+CASES = ["4x2x2, 12 a cell", "2x2x2, 51 a cell", "4x4x2", "4x4x3", "one cell", "small, split", "small, long", "small, direct",
+         "small, split, odd positions", "4x4x3, split", "4x4x3, direct"]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_tile_passes_bit_exact(case, oracle):
+    """Two steps by the tile passes, then one with their density pass writing the context's lists for the
+    per-particle force pass: the oracle's bits (NaN where it has NaN), and its cells."""
+    p, parts = _case(case)
+    print(f"case {case}: n={p.num_particles} R={p.grid_res}", flush=True)
+    dt = 2e-6
+    st = oracle.OracleState(p, parts)
+    tile = L.lib().wc_num_variants() - 1
+    with Fluid(p, parts) as f:
+        for steps, tuning in ((1, (tile, tile, 0)), (1, (tile, tile, 1)), (1, (tile, 2, 1))):
+            f.set_tuning(*tuning)
+            st.step(dt, steps)
+            f.step(dt, steps)
+            f.synchronize()
+            got = f.particles(1)
+            for k in ("density", "pressure", "velocity", "position"):
+                x, y = got[k], st.buf1[k]
+                assert np.array_equal(np.isnan(x), np.isnan(y)), f"{case} {tuning}: {k} NaN"
+                bad = (x.view(np.uint32) != y.view(np.uint32)) & ~np.isnan(y)
+                assert not bad.any(), f"{case} {tuning}: {k} differs at {int(bad.sum())} places"
+            assert np.array_equal(f.sort_.getCountBuffer(), st.counts)
+            assert np.array_equal(f.sort_.getOffsetBuffer(), st.offsets)
+        # the lists that the two kinds of density pass write agree
+        counts = []
+        for variant in (tile, 2):
+            f.set_tuning(variant, 2, 1)
+            f.sort_.run()
+            f.runDensityProg()
+            counts.append(f.neighbour_counts())
+        assert np.array_equal(counts[0], counts[1])
+        if case == "2x2x2, 51 a cell":
+            assert (counts[0] == 0xFFFFFFFF).any()

@@ -115,8 +115,9 @@ using wc::SceneDesc;
 struct wc_ctx {
     std::vector<wc_params> params;   // per scene
     std::vector<SceneDesc> desc;     // per scene, mirrored in d_desc
-    std::vector<uint32_t> tables;    // blk64 | blk128 | blk256 | tiles, each num_scenes + 1
-    std::vector<uint32_t> scene_tab;  // several scenes: scene of each 64/128/256-thread block and tile
+    std::vector<uint32_t> tables;    // blk64 | blk128 | blk256 | tiles | tblk, each num_scenes + 1
+    // several scenes: scene of each 64/128/256-thread block, scan tile and block of base boxes
+    std::vector<uint32_t> scene_tab;
     uint32_t num_scenes = 0;
     uint32_t total_particles = 0;
     uint32_t total_cells = 0;        // padded to scan tiles per scene
@@ -135,9 +136,22 @@ struct wc_ctx {
     hipGraph_t graph[2] = {nullptr, nullptr};
     hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
     bool graph_valid = false;
-    int density_variant = 2;  // (64 threads, 32 list entries, 4 in flight, per-plane drain) until tuned
+    // until tuned: the tile passes where they can run, else (64 threads, 32 list entries, 4 in flight,
+    // per-plane drain)
+    int density_variant = 2;
     int update_variant = 2;
     bool neighbour_list = false;  // density writes neighbour lists, the force pass reads them
+    // tile passes: their base box (choose_tile_shape()), and whether the context may use them
+    wc::TileShape tile_shape{};
+    uint32_t tile_per = 1;  // base boxes per classification workgroup
+    bool tile_ok = false;
+    uint32_t tile_entries = 0;  // entries the work list needs at most
+    void* tile_mem = nullptr;   // the tile passes' buffers, one allocation
+    // What the last queued passes left in the buffers; a host upload or a parameter change clears all.
+    bool sorted_ok = false;  // buffer 2 holds the last sort's output, every slot in its cell's range
+    bool tiles_ok = false;   // ... and the work list is that sort's
+    bool llist_ok = false;   // the tiles' lists and counts are those of a density pass on that sort
+    bool nlist_ok = false;   // nlist and ncount likewise
     double clock_khz = 100000.0;  // wall_clock64 rate
     // learned-closure workspace (allocated on first use)
     uint16_t* cl_x = nullptr;       // features, n x 208 bf16
@@ -168,16 +182,57 @@ int check_params(const wc_params* p) {
     return WC_OK;
 }
 
-// Lays the scenes out (particle and cell offsets, block and tile tables) from c->params.
-int layout_scenes(wc_ctx* c) {
+constexpr uint64_t kTileMaxCellsPerParticle = 64;
+
+// Base box of the tile passes.  Larger boxes stage less halo per particle; they have to fit LDS at rest
+// density (a denser one is split) and leave the chip's 256 CUs some boxes each: the largest shape of which
+// the particles fill 350.  At 8 particles a cell the whole step took, by 4x3x4 / 4x2x4 / 2x2x4 (us):
+// 16,384 particles 75 / 71 / 70, 91,125 118 / 108 / 112, 125,000 125 / 117 / 133, 262,144 152 / 164 / 187;
+// at 12 a cell 4x2x4 / 2x2x4: 125,000 155 / 149, 2,048,000 1,144 / 1,175.  Below that 2x2x4 unless a box
+// has more particles than threads: the 80,000-particle scene (20 a cell) 225 by 2x2x4, 181 by 2x2x2.
+wc::TileShape choose_tile_shape(const std::vector<wc_params>& scenes) {
+    double n = 0.0, cell = 0.0;  // particles; those a cell holds at rest density
+    for (const wc_params& p : scenes) {
+        n += p.num_particles;
+        const double rest = (double)p.rest_density / (double)p.particle_mass * pow((double)p.bin_size, 3.0);
+        if (rest > 0.0 && rest < 1e6) cell += rest * p.num_particles;
+    }
+    cell = n > 0.0 ? cell / n : 0.0;
+    for (const wc::TileShape& t : {wc::TileShape{4, 3, 4, wc::kTileLargeBlock, wc::kTileLargeCap},
+                                   wc::TileShape{4, 2, 4, wc::kTileLargeBlock, wc::kTileLargeCap},
+                                   wc::TileShape{2, 2, 4, wc::kTileSmallBlock, wc::kTileSmallCap}})
+        if ((t.x + 2) * (t.y + 2) * (t.z + 2) * cell * 1.05 <= t.cap && n >= 350.0 * (t.x * t.y * t.z) * cell) return t;
+    return {2, 2, 16.0 * cell <= wc::kTileSmallBlock ? 4 : 2, wc::kTileSmallBlock, wc::kTileSmallCap};
+}
+
+// Base boxes classified per workgroup: about 2,000 workgroups, at least 8 boxes each (fewer workgroups
+// leave the chip idle, more queue on the work list's counter).
+uint32_t tiles_per_block(const std::vector<wc_params>& scenes, const wc::TileShape& t) {
+    uint64_t boxes = 0;
+    for (const wc_params& p : scenes) {
+        const uint32_t R = (uint32_t)p.grid_res;
+        boxes += (uint64_t)ceil_div(R, t.x) * ceil_div(R, t.y) * ceil_div(R, t.z);
+    }
+    uint32_t per = 8;
+    while (per < wc::kTileBlock && boxes / per > 2000) per *= 2;
+    return per;
+}
+
+// Lays the scenes out (particle and cell offsets, block and tile tables) from c->params.  max_entries: what
+// the tile passes' work list may hold.
+int layout_scenes(wc_ctx* c, uint64_t max_entries) {
     const uint32_t S = c->num_scenes;
     c->desc.assign(S, SceneDesc{});
-    c->tables.assign(4 * (size_t)(S + 1), 0u);
+    c->tables.assign(5 * (size_t)(S + 1), 0u);
     uint32_t* blk64 = &c->tables[0];
     uint32_t* blk128 = blk64 + (S + 1);
     uint32_t* blk256 = blk128 + (S + 1);
     uint32_t* tiles = blk256 + (S + 1);
-    uint64_t p_off = 0, c_off = 0;
+    uint32_t* tblk = tiles + (S + 1);
+    uint64_t p_off = 0, c_off = 0, boxes = 0, cells = 0;
+    c->tile_shape = choose_tile_shape(c->params);
+    const wc::TileShape shape = c->tile_shape;
+    c->tile_per = tiles_per_block(c->params, shape);
     for (uint32_t s = 0; s < S; ++s) {
         const wc_params& p = c->params[s];
         SceneDesc& d = c->desc[s];
@@ -189,6 +244,13 @@ int layout_scenes(wc_ctx* c) {
         blk128[s + 1] = blk128[s] + ceil_div(d.c.n, 128);
         blk256[s + 1] = blk256[s] + ceil_div(d.c.n, 256);
         tiles[s + 1] = tiles[s] + nt;
+        const uint32_t R = (uint32_t)d.c.R;
+        d.tnx = ceil_div(R, shape.x);
+        d.tny = ceil_div(R, shape.y);
+        d.ntiles = d.c.n ? d.tnx * d.tny * ceil_div(R, shape.z) : 0u;
+        tblk[s + 1] = tblk[s] + ceil_div(d.ntiles, c->tile_per);
+        boxes += d.ntiles;
+        cells += d.c.ncells;
         p_off += d.c.n;
         c_off += (uint64_t)nt * wc::kScanTile;
         if (p_off > 0xFFFFFF00ull || c_off > 0xFFFFFF00ull)
@@ -196,9 +258,14 @@ int layout_scenes(wc_ctx* c) {
     }
     c->total_particles = (uint32_t)p_off;
     c->total_cells = (uint32_t)c_off;
+    // The tile passes look at every base box: on a grid with far more cells than particles that costs
+    // more than they gain.
+    const uint64_t entries = wc::tile_capacity(boxes, p_off);
+    c->tile_ok = p_off > 0 && cells <= kTileMaxCellsPerParticle * p_off && entries <= max_entries;
+    c->tile_entries = c->tile_ok ? (uint32_t)entries : 0u;
     c->scene_tab.clear();
     if (S > 1) {
-        for (const uint32_t* first : {blk64, blk128, blk256, tiles})
+        for (const uint32_t* first : {blk64, blk128, blk256, tiles, tblk})
             for (uint32_t s = 0; s < S; ++s) c->scene_tab.insert(c->scene_tab.end(), first[s + 1] - first[s], s);
     }
     return WC_OK;
@@ -212,12 +279,14 @@ void fill_scene_views(wc_ctx* c) {
     v.blk128 = c->d_tables + (S + 1);
     v.blk256 = c->d_tables + 2 * (S + 1);
     v.tiles = c->d_tables + 3 * (S + 1);
-    v.scene64 = v.scene128 = v.scene256 = v.scene_tile = nullptr;
+    v.tblk = c->d_tables + 4 * (S + 1);
+    v.scene64 = v.scene128 = v.scene256 = v.scene_tile = v.scene_tblk = nullptr;
     if (S > 1 && c->d_scene_tab) {
         v.scene64 = c->d_scene_tab;
         v.scene128 = v.scene64 + c->tables[S];
         v.scene256 = v.scene128 + c->tables[2 * (size_t)(S + 1) - 1];
         v.scene_tile = v.scene256 + c->tables[3 * (size_t)(S + 1) - 1];
+        v.scene_tblk = v.scene_tile + c->tables[4 * (size_t)(S + 1) - 1];
     }
     v.num_scenes = S;
     v.total_particles = c->total_particles;
@@ -225,6 +294,12 @@ void fill_scene_views(wc_ctx* c) {
     v.blocks64 = c->tables[S];
     v.blocks128 = c->tables[2 * (size_t)(S + 1) - 1];
     v.blocks256 = c->tables[3 * (size_t)(S + 1) - 1];
+    v.tblocks = c->tables[5 * (size_t)(S + 1) - 1];
+    const wc::TileShape& shape = c->tile_shape;
+    v.tper = c->tile_per;
+    v.bx = (uint32_t)shape.x;
+    v.by = (uint32_t)shape.y;
+    v.bz = (uint32_t)shape.z;
 }
 
 int upload_tables(wc_ctx* c) {
@@ -247,7 +322,7 @@ void free_ctx_buffers(wc_ctx* c) {
                     c->d_tables,   b.rho_max,     b.ids[0],      b.ids[1],      c->cl_x,     c->cl_y,
                     c->cl_backup[0][0], c->cl_backup[0][1], c->cl_backup[1][0], c->cl_backup[1][1],
                     c->cl_backup_ids[0], c->cl_backup_ids[1], c->cl_rows, b.nlist, b.ncount, c->d_scene_tab,
-                    b.crowd,      b.crowd_count, c->cl_long};
+                    b.crowd,      b.crowd_count, c->cl_long,      c->tile_mem};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (c->cl_host_rho) (void)hipHostFree(c->cl_host_rho);
@@ -263,6 +338,7 @@ void free_ctx_buffers(wc_ctx* c) {
     c->cl_backup[0][0] = c->cl_backup[0][1] = c->cl_backup[1][0] = c->cl_backup[1][1] = nullptr;
     c->cl_backup_ids[0] = c->cl_backup_ids[1] = nullptr;
     c->cl_rows = nullptr;
+    c->tile_mem = nullptr;
 }
 
 void drop_graph(wc_ctx* c) {
@@ -300,19 +376,77 @@ int ensure_neighbour_lists(wc_ctx* c) {
     return WC_OK;
 }
 
+bool density_by_tiles(const wc_ctx* c) { return c->tile_ok && c->density_variant == wc::tile_variant(); }
+bool update_by_tiles(const wc_ctx* c) { return density_by_tiles(c) && c->update_variant == wc::tile_variant(); }
+// the per-particle variant of a pass whose tile form cannot run
+int particle_variant(int v) { return v == wc::tile_variant() ? 2 : v; }
+
+// What the buffers hold after a sort, and after the whole step of the current tuning.
+void note_sort(wc_ctx* c, bool tiles) {
+    c->sorted_ok = true;
+    c->tiles_ok = tiles;
+    c->llist_ok = c->nlist_ok = false;
+}
+void note_step(wc_ctx* c) {
+    note_sort(c, density_by_tiles(c));
+    c->llist_ok = density_by_tiles(c);
+    c->nlist_ok = c->neighbour_list && !update_by_tiles(c);
+}
+
+// The kernels of a sort, in order, each followed by after(k) (k-th of the passes wc_pass_name names).
+template <typename After>
+hipError_t launch_sort(wc_ctx* c, bool tiles, After after) {
+    hipError_t e = wc::launch_hash(c->b, c->stream);
+    if (e == hipSuccess) e = after(0);
+    if (e == hipSuccess) e = wc::launch_scan(c->b, c->stream);
+    if (e == hipSuccess) e = after(1);
+    if (e == hipSuccess) e = wc::launch_place(c->b, tiles ? &c->tile_shape : nullptr, c->stream);
+    if (e == hipSuccess) e = after(2);
+    if (e == hipSuccess) e = wc::launch_gather(c->b, tiles ? &c->tile_shape : nullptr, c->stream);
+    if (e == hipSuccess) e = after(3);
+    note_sort(c, tiles);
+    return e;
+}
+
 int enqueue_sort(wc_ctx* c) {
-    WC_HIP(wc::launch_hash(c->b, c->stream));
-    WC_HIP(wc::launch_scan(c->b, c->stream));
-    WC_HIP(wc::launch_place(c->b, c->stream));
-    WC_HIP(wc::launch_gather(c->b, c->stream));
+    WC_HIP(launch_sort(c, density_by_tiles(c), [](int) { return hipSuccess; }));
     return WC_OK;
+}
+
+// Density pass of the current tuning.  `lists`: the caller reads nlist and ncount; the tile passes keep
+// lists of their own, so in list mode they write these only then, or when the force pass reads them.
+hipError_t launch_density_pass(wc_ctx* c, bool lists) {
+    if (density_by_tiles(c) && c->tiles_ok) {
+        const bool write = c->neighbour_list && (lists || !update_by_tiles(c));
+        const hipError_t e = wc::launch_density_tile(c->b, c->tile_shape, write, c->stream);
+        c->llist_ok = true;
+        c->nlist_ok = write;
+        return e;
+    }
+    c->llist_ok = false;
+    c->nlist_ok = c->neighbour_list;
+    return wc::launch_density(c->b, particle_variant(c->density_variant), c->neighbour_list, c->stream);
+}
+
+hipError_t launch_update_pass(wc_ctx* c) {
+    if (update_by_tiles(c) && c->llist_ok) return wc::launch_update_tile(c->b, c->tile_shape, wc::TileUpdate{}, c->stream);
+    return wc::launch_update(c->b, particle_variant(c->update_variant), c->neighbour_list && c->nlist_ok, c->stream);
+}
+
+// nlist and ncount of the last density pass, for readers in list mode: a density pass by tiles that
+// left them out runs again and writes them (and the same densities).  After an upload the counts are
+// marked overflowed and every reader searches.
+hipError_t refresh_lists(wc_ctx* c) {
+    if (!c->llist_ok || c->nlist_ok || !c->b.nlist || !c->b.ncount) return hipSuccess;
+    c->nlist_ok = true;
+    return wc::launch_density_tile(c->b, c->tile_shape, true, c->stream);
 }
 
 int enqueue_step(wc_ctx* c) {
     int rc = enqueue_sort(c);
     if (rc) return rc;
-    WC_HIP(wc::launch_density(c->b, c->density_variant, c->neighbour_list, c->stream));
-    WC_HIP(wc::launch_update(c->b, c->update_variant, c->neighbour_list, c->stream));
+    WC_HIP(launch_density_pass(c, false));
+    WC_HIP(launch_update_pass(c));
     return WC_OK;
 }
 
@@ -335,14 +469,14 @@ int create_context(const wc_params* scenes, uint32_t num, wc_ctx** out) {
     if (!c) return fail(WC_ERR_NO_MEMORY, "host allocation failed");
     c->num_scenes = num;
     c->params.assign(scenes, scenes + num);
-    int rc = layout_scenes(c);
+    int rc = layout_scenes(c, 0xFFFFFFFFu);
     if (rc) {
         delete c;
         return rc;
     }
     c->particle_cap = c->total_particles;
     c->cell_cap = c->total_cells;
-    c->tile_cap = c->tables.back();
+    c->tile_cap = c->tables[4 * (size_t)(num + 1) - 1];
     if (hipGetDevice(&c->device) != hipSuccess) {
         delete c;
         return fail(WC_ERR_NO_DEVICE, "hipGetDevice failed");
@@ -391,6 +525,35 @@ int create_context(const wc_params* scenes, uint32_t num, wc_ctx** out) {
         return fail(WC_ERR_NO_MEMORY, "device allocation failed (%u particles, %u cells)", c->total_particles,
                     c->total_cells);
     }
+    if (c->tile_ok) {
+        // Only with room left for what a caller may ask for later, about 1 KB a particle (neighbour lists, a
+        // learned step's workspace): else the context keeps the per-particle passes.
+        const size_t list_cap = wc::tile_list_cap(n), chunks = wc::tile_list_chunks(n);
+        const size_t tables = n / 128 + 1024 < c->tile_entries ? n / 128 + 1024 : c->tile_entries;
+        const size_t bytes[6] = {c->tile_entries * sizeof(uint4), 256, tables * wc::kTileTableBytes, n * 4,
+                                 chunks * 64 * list_cap * sizeof(uint16_t), chunks * 64 * sizeof(uint16_t)};
+        void** const ptr[6] = {(void**)&b.tiles,  (void**)&b.tile_count, &b.tables,
+                               (void**)&b.sparse, (void**)&b.llist,      (void**)&b.lcount};
+        size_t free_bytes = 0, total_bytes = 0, all = 0;
+        for (size_t v : bytes) all += (v + 255) / 256 * 256;
+        c->tile_ok = hipMemGetInfo(&free_bytes, &total_bytes) == hipSuccess && all + n * 1024 <= free_bytes &&
+                     hipMalloc(&c->tile_mem, all) == hipSuccess;
+        if (c->tile_ok) {
+            char* at = static_cast<char*>(c->tile_mem);
+            for (int k = 0; k < 6; ++k) {
+                *ptr[k] = at;
+                at += (bytes[k] + 255) / 256 * 256;
+            }
+            b.tile_cap = c->tile_entries;
+            b.table_cap = (uint32_t)tables;
+            b.list_cap = (uint32_t)list_cap;
+            b.list_chunks = (uint32_t)chunks;
+            if (n >= wc::kTileMinParticles) c->density_variant = c->update_variant = wc::tile_variant();
+        } else {
+            c->tile_mem = nullptr;
+            (void)hipGetLastError();
+        }
+    }
     hipError_t e = hipSuccess;
     auto zero = [&](void* p, size_t bytes) {
         if (e == hipSuccess) e = hipMemsetAsync(p, 0, bytes, c->stream);
@@ -403,6 +566,7 @@ int create_context(const wc_params* scenes, uint32_t num, wc_ctx** out) {
     zero(b.step_start, 64);
     zero(b.rho_max, 64);
     zero(b.crowd_count, 64);
+    if (c->tile_ok) zero(b.tile_count, 256);
     // rho_max[1] = 2: no density pass has checked the force pass's division operands yet
     if (e == hipSuccess) e = hipMemsetAsync(reinterpret_cast<char*>(b.rho_max) + 4, 2, 1, c->stream);
     zero(b.sorted, n * 4);
@@ -471,6 +635,7 @@ int run_steps(wc_ctx* c, uint32_t nsteps) {
     uint32_t left = nsteps;
     for (; left >= kStepsPerGraph; left -= kStepsPerGraph) WC_HIP(hipGraphLaunch(c->graph_exec[1], c->stream));
     for (; left > 0; --left) WC_HIP(hipGraphLaunch(c->graph_exec[0], c->stream));
+    note_step(c);
     return WC_OK;
 }
 
@@ -504,6 +669,7 @@ int copy_records_in(wc_ctx* c, uint32_t first, const wc_particle* host, uint32_t
         WC_HIP(wc::launch_split_records(c->staging + first, c->b.posrho[b] + first, c->b.velp[b] + first, n,
                                         c->stream));
     // buffer 2 changed under the last sort: its cell keys, neighbour lists and division check
+    c->sorted_ok = c->tiles_ok = c->llist_ok = c->nlist_ok = false;
     WC_HIP(wc::launch_invalidate(c->b, c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
     return WC_OK;
@@ -727,13 +893,14 @@ WC_API int wc_set_params(wc_ctx* c, const wc_params* p) {
     WC_HIP(hipStreamSynchronize(c->stream));
     const float dt = c->desc[0].dt;
     c->params[0] = *p;
-    rc = layout_scenes(c);
+    rc = layout_scenes(c, c->b.tile_cap);
     if (rc) return rc;
     c->desc[0].dt = dt;
     drop_graph(c);
     rc = upload_tables(c);
     if (rc) return rc;
     // keys, lists and the division check of buffer 2 were formed with the old constants
+    c->sorted_ok = c->tiles_ok = c->llist_ok = c->nlist_ok = false;
     WC_HIP(wc::launch_invalidate(c->b, c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
     return WC_OK;
@@ -785,7 +952,7 @@ WC_API int wc_density(wc_ctx* c) {
     if (!c) return fail(WC_ERR_INVALID_ARG, "ctx is NULL");
     int rc = set_device(c);
     if (rc) return rc;
-    WC_HIP(wc::launch_density(c->b, c->density_variant, c->neighbour_list, c->stream));
+    WC_HIP(launch_density_pass(c, true));
     return WC_OK;
 }
 
@@ -795,7 +962,7 @@ WC_API int wc_update(wc_ctx* c, float dt) {
     if (rc) return rc;
     rc = set_device(c);
     if (rc) return rc;
-    WC_HIP(wc::launch_update(c->b, c->update_variant, c->neighbour_list, c->stream));
+    WC_HIP(launch_update_pass(c));
     return WC_OK;
 }
 
@@ -877,8 +1044,8 @@ WC_API int wc_step_noalloc(const wc_params* p, float dt, void* posrho, void* vel
     WC_HIP(wc::launch_noalloc_setup(d, tables, d_desc, d_tables, b.counts, (uint32_t)ncells, b.error_flag, s));
     WC_HIP(wc::launch_hash(b, s));
     WC_HIP(wc::launch_scan(b, s));
-    WC_HIP(wc::launch_place(b, s));
-    WC_HIP(wc::launch_gather(b, s));
+    WC_HIP(wc::launch_place(b, nullptr, s));
+    WC_HIP(wc::launch_gather(b, nullptr, s));
     WC_HIP(wc::launch_density(b, kNoAllocVariant, false, s));
     WC_HIP(wc::launch_update(b, kNoAllocVariant, false, s));
     return WC_OK;
@@ -971,17 +1138,11 @@ WC_API int wc_profile_steps(wc_ctx* c, float dt, uint32_t nsteps, double ms_tota
     for (uint32_t s = 0; s < nsteps && err == hipSuccess; ++s) {
         hipEvent_t* e = &ev[(size_t)s * (WC_NUM_PASSES + 1)];
         err = hipEventRecord(e[0], c->stream);
-        if (err == hipSuccess) err = wc::launch_hash(c->b, c->stream);
-        if (err == hipSuccess) err = hipEventRecord(e[1], c->stream);
-        if (err == hipSuccess) err = wc::launch_scan(c->b, c->stream);
-        if (err == hipSuccess) err = hipEventRecord(e[2], c->stream);
-        if (err == hipSuccess) err = wc::launch_place(c->b, c->stream);
-        if (err == hipSuccess) err = hipEventRecord(e[3], c->stream);
-        if (err == hipSuccess) err = wc::launch_gather(c->b, c->stream);
-        if (err == hipSuccess) err = hipEventRecord(e[4], c->stream);
-        if (err == hipSuccess) err = wc::launch_density(c->b, c->density_variant, c->neighbour_list, c->stream);
+        if (err == hipSuccess)
+            err = launch_sort(c, density_by_tiles(c), [&](int k) { return hipEventRecord(e[k + 1], c->stream); });
+        if (err == hipSuccess) err = launch_density_pass(c, false);
         if (err == hipSuccess) err = hipEventRecord(e[5], c->stream);
-        if (err == hipSuccess) err = wc::launch_update(c->b, c->update_variant, c->neighbour_list, c->stream);
+        if (err == hipSuccess) err = launch_update_pass(c);
         if (err == hipSuccess) err = hipEventRecord(e[6], c->stream);
     }
     if (err == hipSuccess) err = hipStreamSynchronize(c->stream);
@@ -1044,6 +1205,7 @@ WC_API int wc_get_neighbour_counts(wc_ctx* c, uint32_t* host, uint32_t n) {
     if (n != c->total_particles) return fail(WC_ERR_INVALID_ARG, "n = %u, the context holds %u", n, c->total_particles);
     int rc = set_device(c);
     if (rc) return rc;
+    WC_HIP(refresh_lists(c));
     WC_HIP(hipMemcpyAsync(host, c->b.ncount, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
     return WC_OK;
@@ -1079,16 +1241,20 @@ WC_API int wc_tune(wc_ctx* c, float dt, uint32_t reps, wc_tuning* chosen, double
             err = hipMemcpyAsync(save_pos, c->b.posrho[0], n * sizeof(float4), hipMemcpyDeviceToDevice, c->stream);
         if (err == hipSuccess)
             err = hipMemcpyAsync(save_vel, c->b.velp[0], n * sizeof(float4), hipMemcpyDeviceToDevice, c->stream);
-        if (err == hipSuccess) err = (enqueue_sort(c) == WC_OK) ? hipSuccess : hipErrorUnknown;
+        if (err == hipSuccess) err = launch_sort(c, c->tile_ok, [](int) { return hipSuccess; });
         // Both passes are idempotent on the sorted buffer: density rewrites the same densities
         // (and, with lists, the same lists), the force pass rewrites buffer 1 from buffer 2 alone.
-        // In list mode the density variants run first, so every force-pass variant reads lists.
+        // In list mode the density variants run first, so every force-pass variant reads lists; the
+        // tile variant is the last, so its force pass too.
         for (int mode = 0; mode < 2 && err == hipSuccess; ++mode) {
             for (int pass = 0; pass < 2 && err == hipSuccess; ++pass) {
                 for (int v = 0; v < nv && err == hipSuccess; ++v) {
                     auto launch = [&]() {
-                        return pass == 0 ? wc::launch_density(c->b, v, mode == 1, c->stream)
-                                         : wc::launch_update(c->b, v, mode == 1, c->stream);
+                        if (v == wc::tile_variant() && c->tile_ok)
+                            return pass == 0 ? wc::launch_density_tile(c->b, c->tile_shape, false, c->stream)
+                                             : wc::launch_update_tile(c->b, c->tile_shape, wc::TileUpdate{}, c->stream);
+                        return pass == 0 ? wc::launch_density(c->b, particle_variant(v), mode == 1, c->stream)
+                                         : wc::launch_update(c->b, particle_variant(v), mode == 1, c->stream);
                     };
                     err = launch();  // warm-up
                     if (err == hipSuccess) err = hipEventRecord(ev.start, c->stream);
@@ -1109,17 +1275,28 @@ WC_API int wc_tune(wc_ctx* c, float dt, uint32_t reps, wc_tuning* chosen, double
         (void)hipFree(save_pos);
         (void)hipFree(save_vel);
         if (err != hipSuccess) return fail(WC_ERR_HIP, "tuning failed: %s", hipGetErrorString(err));
+        c->llist_ok = c->tile_ok;
+        c->nlist_ok = true;
+        // The per-particle variants of the two passes combine freely; the tile variant's passes only with
+        // each other (its force pass reads its density pass's lists).  Those lists are the same in both
+        // modes, so a pick of the tile variant keeps neighbour lists available.
+        const int tile = wc::tile_variant();
         int best[2][2] = {{0, 0}, {0, 0}};
         for (int mode = 0; mode < 2; ++mode)
             for (int pass = 0; pass < 2; ++pass)
                 for (int v = 1; v < nv; ++v)
-                    if (t[mode][pass][v] < t[mode][pass][best[mode][pass]]) best[mode][pass] = v;
+                    if (v != tile && t[mode][pass][v] < t[mode][pass][best[mode][pass]]) best[mode][pass] = v;
         const double step0 = t[0][0][best[0][0]] + t[0][1][best[0][1]];
         const double step1 = t[1][0][best[1][0]] + t[1][1][best[1][1]];
+        const double step_tile = fmin(t[0][0][tile], t[1][0][tile]) + fmin(t[0][1][tile], t[1][1][tile]);
         const int mode = step1 < step0 ? 1 : 0;
         c->density_variant = best[mode][0];
         c->update_variant = best[mode][1];
         c->neighbour_list = mode == 1;
+        if (c->tile_ok && step_tile < fmin(step0, step1)) {
+            c->density_variant = c->update_variant = tile;
+            c->neighbour_list = true;
+        }
         drop_graph(c);
     }
     if (chosen) {
@@ -1459,6 +1636,7 @@ WC_API int wc_closure_features(wc_ctx* c, float dt_mult, const uint32_t* rows_ho
     } else {
         nrows = n;
     }
+    if (c->neighbour_list) WC_HIP(refresh_lists(c));
     WC_HIP(wc::launch_closure_features(c->b, rows, nrows, dt_mult, (uint16_t*)x_dev, c->neighbour_list,
                                        c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
@@ -1490,9 +1668,18 @@ WC_API int wc_closure_infer(wc_ctx* c, wc_mlp* net, float dt_mult, void* y_dev) 
     rc = set_device(c);
     if (rc) return rc;
     WC_HIP(hipStreamSynchronize(net->m.stream));
+    WC_HIP(refresh_lists(c));
     WC_HIP(closure_infer_from_lists(c, net, dt_mult, (float*)y_dev));
     WC_HIP(hipStreamSynchronize(c->stream));
     return WC_OK;
+}
+
+// The learned step's force pass: by tiles when their lists are there and no correction is averaged over
+// neighbours, else per particle.
+static hipError_t launch_learned_update(wc_ctx* c, const wc::TileUpdate& u, bool smooth) {
+    if (update_by_tiles(c) && c->llist_ok && !(smooth && u.corr)) return wc::launch_update_tile(c->b, c->tile_shape, u, c->stream);
+    return wc::launch_closure_update(c->b, u.dt, u.corr, u.corr_scale, u.acc_out, smooth, u.substeps,
+                                     c->neighbour_list && c->nlist_ok, c->stream, u.backup);
 }
 
 WC_API int wc_closure_update(wc_ctx* c, float dt, const void* corr_dev, float corr_scale, void* acc_dev) {
@@ -1500,8 +1687,13 @@ WC_API int wc_closure_update(wc_ctx* c, float dt, const void* corr_dev, float co
     if (c->num_scenes != 1) return fail(WC_ERR_INVALID_ARG, "the learned closure runs on single-scene contexts");
     int rc = set_device(c);
     if (rc) return rc;
-    WC_HIP(wc::launch_closure_update(c->b, dt, (const float*)corr_dev, corr_scale, (float*)acc_dev, false, 0.0f,
-                                     c->neighbour_list, c->stream));
+    wc::TileUpdate u;
+    u.learned = true;
+    u.dt = dt;
+    u.corr = (const float*)corr_dev;
+    u.corr_scale = corr_scale;
+    u.acc_out = (float*)acc_dev;
+    WC_HIP(launch_learned_update(c, u, false));
     return WC_OK;
 }
 
@@ -1552,7 +1744,7 @@ WC_API int wc_closure_run(wc_ctx* c, wc_mlp* net, float dt, uint32_t K, uint32_t
     auto sort_density = [&]() -> int {
         int r = enqueue_sort(c);
         if (r) return r;
-        WC_HIP(wc::launch_density(c->b, c->density_variant, c->neighbour_list, c->stream));
+        WC_HIP(launch_density_pass(c, net != nullptr));  // the network reads the lists
         return WC_OK;
     };
     // One macro step: form the closure inputs, run the network, take the large step (whose force
@@ -1567,12 +1759,16 @@ WC_API int wc_closure_run(wc_ctx* c, wc_mlp* net, float dt, uint32_t K, uint32_t
                                                c->stream));
             WC_HIP(wc::mlp_infer(net->m, c->cl_x, c->cl_y, n, c->stream));
         }
-        wc::RecordBackup backup;
-        backup.posrho = c->cl_backup[slot][0];
-        backup.velp = c->cl_backup[slot][1];
-        backup.ids = c->b.ids[0] ? c->cl_backup_ids[slot] : nullptr;
-        WC_HIP(wc::launch_closure_update(c->b, dt_large, net ? c->cl_y : nullptr, g, nullptr, c->cl_smooth,
-                                         c->cl_substeps ? (float)K : 0.0f, c->neighbour_list, c->stream, backup));
+        wc::TileUpdate u;
+        u.learned = true;
+        u.dt = dt_large;
+        u.corr = net ? c->cl_y : nullptr;
+        u.corr_scale = g;
+        u.substeps = c->cl_substeps ? (float)K : 0.0f;
+        u.backup.posrho = c->cl_backup[slot][0];
+        u.backup.velp = c->cl_backup[slot][1];
+        u.backup.ids = c->b.ids[0] ? c->cl_backup_ids[slot] : nullptr;
+        WC_HIP(launch_learned_update(c, u, c->cl_smooth));
         int r = sort_density();
         if (r) return r;
         WC_HIP(hipMemcpyAsync(c->cl_host_rho + slot, c->b.rho_max, 4, hipMemcpyDeviceToHost, c->stream));

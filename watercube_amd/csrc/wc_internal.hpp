@@ -68,7 +68,8 @@ struct SceneDesc {
     uint32_t p_off;  // first particle slot of the scene
     uint32_t c_off;  // first cell of the scene (a multiple of kScanTile)
     float dt;        // integration step
-    uint32_t pad;
+    uint32_t tnx, tny, ntiles;  // base tiles per x and y axis, and in all (tile passes)
+    uint32_t pad[2];
 };
 
 // Device tables of a context's scenes, passed by value to every kernel.
@@ -88,6 +89,13 @@ struct Scenes {
     uint32_t total_particles;
     uint32_t total_tiles;
     uint32_t blocks64, blocks128, blocks256;
+    // tile passes: first classification block of each scene (num_scenes + 1 entries), the
+    // scene of every such block (NULL with one scene), their number, and the base tile's cells
+    const uint32_t* tblk;
+    const uint32_t* scene_tblk;
+    uint32_t tblocks;
+    uint32_t tper;  // base boxes per classification block
+    uint32_t bx, by, bz;
 };
 
 // Device buffers of one context.  posrho/velp are the 32-byte record split in its two
@@ -111,6 +119,17 @@ struct DeviceBuffers {
     uint32_t* ids[2];                 // particle identity per slot of buffer 1 / 2 (NULL: not tracked)
     uint32_t* nlist;                  // neighbour lists (NULL until the list mode is first used)
     uint32_t* ncount;
+    uint4* tiles;                     // work list of the tile passes (NULL: they are not used)
+    uint32_t* tile_count;             // TileWork::count (reset by every sort)
+    uint32_t tile_cap;
+    uint32_t* sparse;                 // slots of the boxes with too few particles to be staged
+    void* tables;                     // cell tables of the first table_cap entries (kTileTableBytes each)
+    uint32_t table_cap;
+    uint16_t* llist;                  // tile passes: neighbours as offsets into the tile's LDS, in chunks of 64
+                                      // lanes: entry k of all of them is one 128-byte row
+    uint16_t* lcount;                 // their number (more than list_cap: none are kept)
+    uint32_t list_chunks;
+    uint32_t list_cap;                // entries of a list (a multiple of 4)
     uint2* crowd;                     // cells with more than kGatherDirectMax particles: (cell, scene)
     uint32_t* crowd_count;            // entries of `crowd` (reset by every sort)
     uint32_t crowd_cap;
@@ -150,13 +169,69 @@ struct PassVariant {
 int num_variants();
 PassVariant variant(int v);
 
+// Tile passes (the last variant): a workgroup stages one box of cells and its halo in LDS.
+struct TileShape {
+    int x, y, z;  // cells of a base box
+    int block;    // threads per workgroup: kTileLargeBlock or kTileSmallBlock
+    int cap;      // records (box and halo) its LDS holds
+};
+constexpr int kTileLargeBlock = 512, kTileLargeCap = 1920;
+constexpr int kTileSmallBlock = 256, kTileSmallCap = 2304;
+int tile_variant();
+// What the sort forms for them.
+struct TileWork {
+    uint4* tiles;     // work list
+    uint32_t* count;  // its entries; [1]: slots in `sparse`; [kListCount]: list chunks
+    uint32_t cap;
+    uint32_t rec_cap;  // records a box may stage
+    uint32_t chunk;    // particles of an entry that searches directly
+    void* tables;      // cell tables of the first table_cap entries
+    uint32_t table_cap;
+    uint32_t* sparse;  // slots of the boxes with few particles
+    uint32_t sparse_max;  // the most records of such a box and its halo
+};
+constexpr uint32_t kListCount = 32;          // in another 128-byte line: atomics on one line serialise
+constexpr uint32_t kTileBlock = 256;         // threads, and at most that many boxes, per classification workgroup
+// Neighbours a particle's list holds (16 bits each; particles with more search directly): dense clusters
+// have a few hundred; large contexts keep lists of half the size.
+inline uint32_t tile_list_cap(uint64_t particles) { return particles <= 500000 ? 512u : particles <= 4000000 ? 256u : 128u; }
+// Contexts of this many particles start with the tile passes.  Smaller ones gain while the fluid is at rest
+// density (16,384 particles, three contexts at once: 20 us a step against 33) and lose as it spreads and boxes
+// empty (44 against 36 at step 4,000); 80,000 particles gain in both (83 against 131, 84 against 122).
+// wc_tune times both whatever the size.
+constexpr uint32_t kTileMinParticles = 50000;
+// Chunks of 64 lanes that lists are kept for.  Full boxes use 1.2 lanes a particle (columns are rounded to four
+// lanes, boxes to 64), a fluid that has spread up to 1.4; boxes past the memory search directly.
+inline uint64_t tile_list_chunks(uint64_t particles) { return particles / 32 + 1024; }
+constexpr size_t kTileTableBytes = 1824;     // cell table of a box
+// Entries a sort can list.  One per base tile; a box whose halo holds more than `cap` >= 1024 records
+// becomes boxes of 2x2x2 cells, then single cells, then chunks of at least 256 particles: every
+// particle lies in the halo of at most 8 boxes of a size (27 cells' halos), so there are at most
+// 8 N / cap such base boxes of up to 8 parts, 8 N / cap boxes of 2x2x2 of 8 parts, and 27 N / cap
+// single cells, with N / 256 chunks more in all.
+inline uint64_t tile_capacity(uint64_t tiles, uint64_t particles) { return tiles + particles / 4 + 64; }
+
 // Kernel launchers (wc_kernels.hip).  Each enqueues on `stream` and returns the launch status.
 hipError_t launch_hash(const DeviceBuffers& b, hipStream_t stream);
 hipError_t launch_scan(const DeviceBuffers& b, hipStream_t stream);
-hipError_t launch_place(const DeviceBuffers& b, hipStream_t stream);
-hipError_t launch_gather(const DeviceBuffers& b, hipStream_t stream);
+// With `tiles`, the two also form the tile passes' work list and tables for that shape.
+hipError_t launch_place(const DeviceBuffers& b, const TileShape* tiles, hipStream_t stream);
+hipError_t launch_gather(const DeviceBuffers& b, const TileShape* tiles, hipStream_t stream);
 // With `list`, the density pass also writes the neighbour lists and the force pass reads them.
 hipError_t launch_density(const DeviceBuffers& b, int variant, bool list, hipStream_t stream);
+// Density pass by tiles; with `list` it also writes the context's neighbour lists (nlist, ncount).
+hipError_t launch_density_tile(const DeviceBuffers& b, const TileShape& t, bool list, hipStream_t stream);
+// Force pass by tiles, from the lists that launch_density_tile wrote for the same sort.
+struct TileUpdate {
+    bool learned = false;  // the learned step's integration (launch_closure_update without averaging)
+    float dt = 0.0f;       // learned: the step, the correction and its scale, the plain acceleration's place
+    const float* corr = nullptr;
+    float corr_scale = 0.0f;
+    float* acc_out = nullptr;
+    float substeps = 0.0f;
+    RecordBackup backup;
+};
+hipError_t launch_update_tile(const DeviceBuffers& b, const TileShape& t, const TileUpdate& u, hipStream_t stream);
 // For the single scene's particles with more than kClosureNeighbours listed neighbours (or an
 // overflowed list): the slots of the kClosureNeighbours nearest, in list order, at
 // sel[t * kClosureFeatures / 2 + k].  Other rows are left alone.

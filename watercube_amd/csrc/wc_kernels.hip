@@ -113,12 +113,14 @@ __global__ __launch_bounds__(kHashBlock) void k_hash(Scenes S, const float4* __r
                                                      unsigned long long* __restrict__ scene_done,
                                                      unsigned long long* __restrict__ step_start,
                                                      uint32_t* __restrict__ rho_max,
-                                                     uint32_t* __restrict__ crowd_count) {
+                                                     uint32_t* __restrict__ crowd_count,
+                                                     uint32_t* __restrict__ tile_count) {
     const uint32_t g = blockIdx.x * kHashBlock + threadIdx.x;
     if (g < S.total_tiles) scan_status[g] = 0ull;
     if (g < S.num_scenes) scene_done[g] = 0ull;
     if (g == 0) {
         *crowd_count = 0u;
+        if (tile_count) tile_count[0] = tile_count[1] = tile_count[kListCount] = 0u;
         *step_start = wall_clock64();
         rho_max[0] = 0u;
         rho_max[1] = kDivPending;  // the force pass's operands are unchecked until a density pass runs
@@ -295,6 +297,387 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(Scenes S, uint32_t* __res
 }
 
 // ------------------------------------------------------------------------------------------
+// The tile passes' work list and cell tables (the passes themselves follow the force pass).  They need
+// only the scan's ranges, so further workgroups of k_place form the list and further ones of k_gather
+// the tables: a launch of their own each cost 4-5 us a step.
+//
+// Listed are the base boxes that hold particles.  One whose records with its halo exceed LDS is listed
+// as boxes of 2x2x2 cells, then as single cells, then as chunks of particles that search in HBM.
+// ------------------------------------------------------------------------------------------
+// Boxes with at most this many records per cell of the box and its halo are not staged: their particles' slots go
+// to T.sparse, which is searched directly.  A fluid that has spread over the cube, us a step of three contexts at
+// once, with no such line / 1.33 / 2 / 3 / 4 records: 192,089 particles at step 4,000 140 / 98 / 97 / 98 / 103 (105
+// by the per-particle passes), a million at step 2,000 405 / 370 / 363 / 364 / 369 (467), a gas of one particle a
+// cell 278 / 75 / 74 / 74 / 75 (77), of two 161 / 147 / 134 / 109 / 108 (98).  At its start, when only the block's
+// skin is that thin, its few particles lengthen the force pass (55 us to 78 at 2, 100 at 3).
+constexpr uint32_t kSparseRecords = 2;
+constexpr uint32_t kEntryDirect = 1u << 12;                 // particles searched for directly: e.w + i
+constexpr uint32_t kEntrySparse = 1u;                       // ... their slots at sparse[e.w + i]
+constexpr int kMaxBox = 4;                                  // cells per side of a box
+constexpr int kMaxHalo = kMaxBox + 2;
+constexpr int kMaxCells = kMaxHalo * kMaxHalo * kMaxHalo;   // of a box and its halo
+
+// (first slot, count) of a cell, inside the scene whatever a failed scan left in the ranges.
+__device__ __forceinline__ uint2 cell_range_in(const uint2* __restrict__ range, uint32_t cell, uint32_t p_off,
+                                               uint32_t n) {
+    uint2 rg = range[cell];
+    if (rg.x - p_off > n) return make_uint2(p_off, 0u);
+    rg.y = min(rg.y, p_off + n - rg.x);
+    return rg;
+}
+
+// Slots of the cells [x0, x1] x {y} x {z} (consecutive cells of a row hold consecutive slots).
+__device__ __forceinline__ uint2 row_slots(const SceneDesc& d, const uint2* __restrict__ range, int x0, int x1, int y,
+                                           int z) {
+    const int R = d.c.R;
+    const uint2* row = range + d.c_off + ((size_t)z * R + y) * R;
+    const uint2 a = cell_range_in(row, (uint32_t)x0, d.p_off, d.c.n), b = cell_range_in(row, (uint32_t)x1, d.p_off, d.c.n);
+    const uint32_t end = b.x + b.y;
+    return make_uint2(a.x, end > a.x ? end - a.x : 0u);
+}
+
+__device__ __forceinline__ void list_tile(const TileWork& T, uint32_t* __restrict__ error_flag, const uint4& e) {
+    const uint32_t at = atomicAdd(T.count, 1u);
+    if (at < T.cap)
+        T.tiles[at] = e;
+    else
+        atomicOr(error_flag, 2u);  // cannot happen when the scan succeeded
+}
+
+// A box's lanes, 64 at a time, have a chunk of list memory each: the box's are e.w, e.w + 1, ...
+__device__ __forceinline__ uint32_t box_chunks(uint32_t particles, int nx, int ny) {
+    return (particles + 3u * (uint32_t)(nx * ny) + 63u) / 64u;  // columns of whole groups of four lanes
+}
+
+__device__ __forceinline__ uint4 box_entry(int x, int y, int z, int nx, int ny, int nz, uint32_t s, uint32_t chunk) {
+    return make_uint4((uint32_t)x | (uint32_t)y << 10 | (uint32_t)z << 20, (uint32_t)nx | (uint32_t)ny << 4 | (uint32_t)nz << 8,
+                      s, chunk);
+}
+
+// A box of at most 2x2x2 cells that does not fit LDS: its cells one by one, or a cell's particles in
+// chunks (one thread's work; dense clusters only).
+__device__ __forceinline__ void list_cells(const SceneDesc& d, const uint2* __restrict__ range, int x, int y, int z, int nx,
+                                           int ny, int nz, uint32_t s, const TileWork& T,
+                                           uint32_t* __restrict__ error_flag) {
+    const int R = d.c.R;
+#pragma unroll 1
+    for (int k = z; k < min(z + nz, R); ++k)
+#pragma unroll 1
+        for (int j = y; j < min(y + ny, R); ++j)
+#pragma unroll 1
+            for (int i = x; i < min(x + nx, R); ++i) {
+                const uint2 slots = row_slots(d, range, i, i, j, k);
+                if (slots.y == 0) continue;
+                uint32_t all = 0;
+                for (int r = 0; r < 9; ++r) {
+                    const int cy = j + r % 3 - 1, cz = k + r / 3 - 1;
+                    if (cy >= 0 && cz >= 0 && cy < R && cz < R)
+                        all += row_slots(d, range, max(i - 1, 0), min(i + 2, R) - 1, cy, cz).y;
+                }
+                if (all <= T.rec_cap) {
+                    list_tile(T, error_flag, box_entry(i, j, k, 1, 1, 1, s, atomicAdd(T.count + kListCount, box_chunks(slots.y, 1, 1))));
+                } else {
+                    for (uint32_t a = 0; a < slots.y; a += T.chunk)
+                        list_tile(T, error_flag,
+                                  make_uint4(0u, kEntryDirect | min(T.chunk, slots.y - a) << 13, s, slots.x + a));
+                }
+            }
+}
+
+// Records of a box and of the box with its halo, by LANES lanes: lane `row` of the group takes one halo
+// row (two dependent loads for the whole box).
+template <int LANES>
+__device__ __forceinline__ uint2 box_records_by(const SceneDesc& d, const uint2* __restrict__ range, int row, bool any,
+                                                int x, int y, int z, int nx, int ny, int nz) {
+    const int R = d.c.R, ry = row % (ny + 2), rz = row / (ny + 2), cy = y - 1 + ry, cz = z - 1 + rz;
+    uint32_t own = 0, all = 0;
+    const bool in = any && rz < nz + 2 && cy >= 0 && cz >= 0 && cy < R && cz < R;
+    if (in && ry > 0 && rz > 0 && ry <= ny && rz <= nz) own = row_slots(d, range, x, min(x + nx, R) - 1, cy, cz).y;
+#pragma unroll
+    for (int m = LANES / 2; m >= 1; m >>= 1) own += __shfl_xor(own, m);
+    if (own == 0) return make_uint2(0u, 0u);  // most boxes of a large grid: their halo is not read
+    if (in) all = row_slots(d, range, max(x - 1, 0), min(x + nx + 1, R) - 1, cy, cz).y;
+#pragma unroll
+    for (int m = LANES / 2; m >= 1; m >>= 1) all += __shfl_xor(all, m);
+    return make_uint2(own, all);
+}
+
+// Classifies S.tper base boxes per workgroup.  Boxes that hold particles are appended in order within a
+// workgroup (one atomic per workgroup: atomics on the one counter serialise at about 11 ns each); one
+// whose halo does not fit LDS is split by a wave.
+template <int LANES>
+__device__ __forceinline__ void classify_boxes(const Scenes& S, const uint2* __restrict__ range, const TileWork& T,
+                                               uint32_t* __restrict__ error_flag, uint32_t b) {
+    __shared__ uint2 s_rec[kTileBlock];  // records of the box, of the box and its halo
+    __shared__ uint3 s_wave[kTileBlock / 64], s_base;  // boxes, slots of sparse ones, list chunks
+    const uint32_t s = scene_of(S.scene_tblk, S.num_scenes, b);
+    const SceneDesc& d = S.desc[s];
+    const int R = d.c.R, bx = (int)S.bx, by = (int)S.by, bz = (int)S.bz;
+    const uint32_t first = (b - S.tblk[s]) * S.tper;
+    auto origin = [&](uint32_t t, int& x, int& y, int& z) {
+        x = (int)(t % d.tnx) * bx;
+        y = (int)(t / d.tnx % d.tny) * by;
+        z = (int)(t / (d.tnx * d.tny)) * bz;
+    };
+    int x, y, z;
+    // four boxes' loads in flight
+    for (uint32_t k0 = threadIdx.x / LANES; k0 < S.tper; k0 += 4 * (kTileBlock / LANES)) {
+        uint2 rec[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t k = k0 + u * (kTileBlock / LANES);
+            origin(first + k, x, y, z);
+            rec[u] = box_records_by<LANES>(d, range, (int)(threadIdx.x % LANES), k < S.tper && first + k < d.ntiles, x, y, z,
+                                           bx, by, bz);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t k = k0 + u * (kTileBlock / LANES);
+            if (k < S.tper && threadIdx.x % LANES == 0) s_rec[k] = rec[u];
+        }
+    }
+    __syncthreads();
+    const uint2 rec = threadIdx.x < S.tper ? s_rec[threadIdx.x] : make_uint2(0u, 0u);
+    const bool few = rec.x != 0 && rec.y <= T.sparse_max;
+    const bool fits = rec.x != 0 && !few && rec.y <= T.rec_cap;
+    const unsigned long long m = __ballot(fits);
+    const unsigned lane = lane_id(), wave = threadIdx.x >> 6;
+    const uint32_t take = few ? rec.x : 0u, lists = fits ? box_chunks(rec.x, bx, by) : 0u;
+    uint32_t incl = take, lists_incl = lists;
+#pragma unroll
+    for (int dd = 1; dd < 64; dd <<= 1) {
+        const uint32_t t = __shfl_up(incl, dd), u = __shfl_up(lists_incl, dd);
+        if ((int)lane >= dd) {
+            incl += t;
+            lists_incl += u;
+        }
+    }
+    if (lane == 63) s_wave[wave] = make_uint3((uint32_t)__popcll(m), incl, lists_incl);
+    __syncthreads();
+    uint32_t before = 0, listed = 0, sparse = 0, sparse_before = incl - take, chunk = lists_incl - lists, list_chunks = 0;
+    for (unsigned w = 0; w < kTileBlock / 64; ++w) {
+        before += w < wave ? s_wave[w].x : 0u;
+        sparse_before += w < wave ? s_wave[w].y : 0u;
+        chunk += w < wave ? s_wave[w].z : 0u;
+        listed += s_wave[w].x;
+        sparse += s_wave[w].y;
+        list_chunks += s_wave[w].z;
+    }
+    // several scenes: entries of their own (one scene's sparse particles need none, tile_item)
+    const uint32_t chunks = S.num_scenes == 1 ? 0u : (sparse + T.chunk - 1) / T.chunk;
+    if (threadIdx.x == 0) {
+        const unsigned long long add = (unsigned long long)sparse << 32 | (listed + chunks);
+        const unsigned long long old = add ? atomicAdd(reinterpret_cast<unsigned long long*>(T.count), add) : 0ull;
+        s_base.x = (uint32_t)old;
+        s_base.y = (uint32_t)(old >> 32);
+    }
+    if (threadIdx.x == 64) s_base.z = list_chunks ? atomicAdd(T.count + kListCount, list_chunks) : 0u;
+    if (threadIdx.x < S.tper) s_rec[threadIdx.x] = make_uint2(few ? 0x80000000u | sparse_before : rec.x, rec.y);
+    __syncthreads();
+    if (fits || threadIdx.x < chunks) {
+        // chunks <= S.tper: a box adds at most sparse_max <= T.chunk particles
+        if (s_base.x + listed + chunks > T.cap) {
+            atomicOr(error_flag, 2u);
+        } else {
+            if (fits) {
+                origin(first + threadIdx.x, x, y, z);
+                T.tiles[s_base.x + chunks + before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] =
+                    box_entry(x, y, z, min(bx, R - x), min(by, R - y), min(bz, R - z), s, s_base.z + chunk);
+            }
+            if (threadIdx.x < chunks)
+                T.tiles[s_base.x + threadIdx.x] =
+                    make_uint4(0u, kEntryDirect | kEntrySparse | min(T.chunk, sparse - threadIdx.x * T.chunk) << 13, s,
+                               s_base.y + threadIdx.x * T.chunk);
+        }
+    }
+    if (sparse != 0u) {
+        // a few lanes a box: lane `row` lists the particles of one row
+        for (uint32_t k = threadIdx.x / LANES; k < S.tper; k += kTileBlock / LANES) {
+            const uint32_t at = s_rec[k].x;
+            if (!(at & 0x80000000u)) continue;  // the same for the box's lanes
+            origin(first + k, x, y, z);
+            const int row = (int)(threadIdx.x % LANES), cy = y + row % by, cz = z + row / by;
+            uint2 slots = make_uint2(0u, 0u);
+            if (row < by * bz && cy < R && cz < R) slots = row_slots(d, range, x, min(x + bx, R) - 1, cy, cz);
+            uint32_t end = slots.y;
+#pragma unroll
+            for (int dd = 1; dd < LANES; dd <<= 1) {
+                const uint32_t t = __shfl_up(end, dd, LANES);
+                if (row >= dd) end += t;
+            }
+            const uint32_t to = s_base.y + (at & 0x7fffffffu) + end - slots.y;
+            for (uint32_t i = 0; i < slots.y; ++i)
+                if (to + i < S.total_particles) T.sparse[to + i] = slots.x + i;
+        }
+    }
+    const bool split = bx > 2 || by > 2 || bz > 2;
+    for (uint32_t k = split ? wave : threadIdx.x; k < S.tper; k += split ? kTileBlock / 64 : kTileBlock) {
+        const uint2 r = s_rec[k];
+        if (r.x == 0 || (r.x & 0x80000000u) || r.y <= T.rec_cap) continue;
+        origin(first + k, x, y, z);
+        if (!split) {
+            list_cells(d, range, x, y, z, bx, by, bz, s, T, error_flag);
+            continue;
+        }
+        // parts of 2x2x2, 16 lanes each (wave-uniform loop)
+        const int px = (bx + 1) / 2, py = (by + 1) / 2, parts = px * py * ((bz + 1) / 2);
+        for (int q0 = 0; q0 < parts; q0 += 4) {
+            const int q = q0 + (int)(lane / 16u);
+            const int i = x + q % px * 2, j = y + q / px % py * 2, l = z + q / (px * py) * 2;
+            // a part ends with its box
+            const int ex = min(min(2, x + bx - i), R - i), ey = min(min(2, y + by - j), R - j), ez = min(min(2, z + bz - l), R - l);
+            const bool any = q < parts && ex > 0 && ey > 0 && ez > 0;
+            const uint2 part = box_records_by<16>(d, range, (int)(lane % 16u), any, i, j, l, ex, ey, ez);
+            if (lane % 16u == 0 && part.x != 0) {
+                if (part.y <= T.rec_cap)
+                    list_tile(T, error_flag, box_entry(i, j, l, ex, ey, ez, s, atomicAdd(T.count + kListCount, box_chunks(part.x, ex, ey))));
+                else
+                    list_cells(d, range, i, j, l, ex, ey, ez, s, T, error_flag);
+            }
+        }
+    }
+}
+
+// A staged box: its halo's cells with z fastest, each cell's records consecutive in LDS.  The three cells
+// (dx, dy, -1..1) about a cell are then one window, in the reference's order (dz innermost).
+struct BoxTable {
+    uint32_t cell[kMaxCells];             // first record | end << 16
+    uint32_t slot[kMaxCells];             // slot of a cell's record r: r + slot
+    uint32_t own[kMaxBox * kMaxBox + 4];  // lanes before each of the box's columns (whole groups of four), then all
+    uint32_t records;
+    uint32_t pad[3];
+};
+static_assert(sizeof(BoxTable) == kTileTableBytes && sizeof(BoxTable) % 16 == 0, "copied in 16-byte pieces");
+
+struct BoxShared : BoxTable {
+    uint32_t wave_sum[4];
+    uint32_t rho;                    // largest density of the box
+};
+
+struct Box {
+    int x, y, z, nx, ny, nz;  // first cell and cells per side
+    int hx, hy, hz;           // with the halo
+};
+
+__device__ __forceinline__ Box box_of(const uint4& e) {
+    Box b;
+    b.x = (int)(e.x & 1023u);
+    b.y = (int)(e.x >> 10 & 1023u);
+    b.z = (int)(e.x >> 20 & 1023u);
+    b.nx = (int)(e.y & 15u);
+    b.ny = (int)(e.y >> 4 & 15u);
+    b.nz = (int)(e.y >> 8 & 15u);
+    b.hx = b.nx + 2;
+    b.hy = b.ny + 2;
+    b.hz = b.nz + 2;
+    return b;
+}
+
+// i / d for i < 256, d <= 36
+__device__ __forceinline__ int small_div(int i, int d) { return (int)((uint32_t)i * (uint32_t)((65536 + d - 1) / d) >> 16); }
+
+// Halo cell (x fastest) i of a box, as its index in the table (z fastest).
+__device__ __forceinline__ int table_cell(const Box& b, int i) {
+    const int r = small_div(i, b.hx), z = small_div(r, b.hy);
+    return ((i - r * b.hx) * b.hy + (r - z * b.hy)) * b.hz + z;
+}
+__device__ __forceinline__ int own_column(const Box& b, int q) {  // table index of column q's first halo cell
+    const int x = small_div(q, b.ny);
+    return ((x + 1) * b.hy + (q - x * b.ny + 1)) * b.hz;
+}
+
+// Lanes before each of the box's columns, columns rounded up to whole groups of four lanes (by wave 0).
+__device__ __forceinline__ void box_lanes(BoxShared& sh, const Box& b) {
+    const int lane = (int)threadIdx.x, ncol = b.nx * b.ny;
+    if (lane < 64) {
+        uint32_t n = 0;
+        if (lane < ncol) {
+            const int c = own_column(b, lane);
+            n = ((sh.cell[c + b.nz] >> 16) - (sh.cell[c + 1] & 0xffffu) + 3u) & ~3u;
+        }
+        uint32_t incl = n;
+#pragma unroll
+        for (int dd = 1; dd < 16; dd <<= 1) {
+            const uint32_t t = __shfl_up(incl, dd);
+            if (lane >= dd) incl += t;
+        }
+        const uint32_t all = (uint32_t)__shfl((int)incl, ncol - 1);
+        if (lane < kMaxBox * kMaxBox + 4) sh.own[lane] = lane < ncol ? incl - n : all;
+    }
+}
+
+// Cell table of a box: every thread takes a halo cell (out-of-grid cells are empty), a prefix sum over the
+// counts gives each its records in LDS.  BLOCK threads take ceil(216 / BLOCK) cells each, in order.
+template <int BLOCK>
+__device__ __forceinline__ void box_cells(BoxShared& sh, const Box& b, const SceneDesc& d, const uint2* __restrict__ range) {
+    constexpr int kPer = (kMaxCells + BLOCK - 1) / BLOCK;
+    const int tid = threadIdx.x, ncell = b.hx * b.hy * b.hz, R = d.c.R;
+    const unsigned lane = lane_id(), wave = threadIdx.x >> 6;
+    for (int i = tid; i < ncell; i += BLOCK) {  // read along x
+        const int r = small_div(i, b.hx), cx = b.x - 1 + (i - r * b.hx);
+        const int rz = small_div(r, b.hy), cy = b.y - 1 + (r - rz * b.hy), cz = b.z - 1 + rz;
+        uint2 rg = make_uint2(0u, 0u);
+        if (cx >= 0 && cy >= 0 && cz >= 0 && cx < R && cy < R && cz < R)
+            rg = cell_range_in(range + d.c_off, (uint32_t)((cz * R + cy) * R + cx), d.p_off, d.c.n);
+        const int at = table_cell(b, i);
+        sh.cell[at] = rg.y;
+        sh.slot[at] = rg.x;
+    }
+    __syncthreads();
+    uint32_t cnt[kPer], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int i = tid * kPer + k;
+        cnt[k] = i < ncell ? sh.cell[i] : 0u;
+        sum += cnt[k];
+    }
+    uint32_t incl = sum;
+#pragma unroll
+    for (int dd = 1; dd < 64; dd <<= 1) {
+        const uint32_t t = __shfl_up(incl, dd);
+        if ((int)lane >= dd) incl += t;
+    }
+    if (lane == 63 && wave < 4) sh.wave_sum[wave] = incl;
+    __syncthreads();
+    uint32_t base = incl - sum, total = 0;
+#pragma unroll
+    for (unsigned w = 0; w < 4 && w < BLOCK / 64; ++w) {
+        base += w < wave ? sh.wave_sum[w] : 0u;
+        total += sh.wave_sum[w];
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int i = tid * kPer + k;
+        if (i < ncell) {
+            sh.cell[i] = base | (base + cnt[k]) << 16;
+            sh.slot[i] -= base;
+        }
+        base += cnt[k];
+    }
+    if (tid == 0) sh.records = total;
+    __syncthreads();
+    box_lanes(sh, b);
+    __syncthreads();
+}
+
+// Tables of the listed boxes, one workgroup each.
+__device__ __forceinline__ void form_tables(const Scenes& S, const uint2* __restrict__ range, const TileWork& T,
+                                            uint32_t block, uint32_t nblocks) {
+    __shared__ BoxShared sh;
+    const uint32_t listed = min(min(*T.count, T.cap), T.table_cap);
+    for (uint32_t item = block; item < listed; item += nblocks) {
+        const uint4 e = T.tiles[item];
+        if (e.y & kEntryDirect) continue;
+        const Box b = box_of(e);
+        box_cells<kHashBlock>(sh, b, S.desc[e.z], range);
+        for (uint32_t k = threadIdx.x; k < sizeof(BoxTable) / 16; k += kHashBlock)
+            reinterpret_cast<uint4*>(&reinterpret_cast<BoxTable*>(T.tables)[item])[k] =
+                reinterpret_cast<const uint4*>(static_cast<const BoxTable*>(&sh))[k];
+        __syncthreads();
+    }
+}
+
+// ------------------------------------------------------------------------------------------
 // 3. place: slot = first slot of the cell + arrival rank (reorder.comp:38-43 without the copy).
 // ------------------------------------------------------------------------------------------
 // The first particle to arrive in a cell of more than kGatherDirectMax also lists the cell for the
@@ -304,8 +687,15 @@ __global__ __launch_bounds__(kHashBlock) void k_place(Scenes S, const uint32_t* 
                                                       const uint2* __restrict__ range,
                                                       uint32_t* __restrict__ slot_tmp, uint2* __restrict__ crowd,
                                                       uint32_t* __restrict__ crowd_count, uint32_t crowd_cap,
-                                                      uint32_t* __restrict__ error_flag) {
+                                                      uint32_t* __restrict__ error_flag, TileWork tiles) {
     const uint32_t b = blockIdx.x;
+    if (b >= S.blocks256) {  // the tile passes' work list
+        if ((S.by + 2) * (S.bz + 2) <= 16)
+            classify_boxes<16>(S, range, tiles, error_flag, b - S.blocks256);
+        else
+            classify_boxes<32>(S, range, tiles, error_flag, b - S.blocks256);
+        return;
+    }
     const uint32_t s = scene_of(S.scene256, S.num_scenes, b);
     const SceneDesc& d = S.desc[s];
     const uint32_t lt = (b - S.blk256[s]) * kHashBlock + threadIdx.x;
@@ -342,6 +732,26 @@ __device__ __forceinline__ float quot(float a, float b, float y) {
 __device__ __forceinline__ bool div_operand(float x) {
     const uint32_t u = __float_as_uint(x) & 0x7fffffffu;
     return u == 0u || u - 0x2b800000u <= 0x53800000u - 0x2b800000u;
+}
+
+// Correctly rounded square root and reciprocal in five and three instructions.  Both were compared
+// with sqrtf and 1 / x on gfx950 for every float in [2^-96, 2^60): no difference.  x = 0 gives 0 (the
+// clamped estimate keeps infinity out), NaN stays NaN.
+__device__ __forceinline__ float sqrt_in_range(float x) {
+    const float y = __builtin_amdgcn_rsqf(fmaxf(x, 0x1p-96f));
+    const float s = x * y;
+    return fmaf(fmaf(-s, s, x), 0.5f * y, s);
+}
+__device__ __forceinline__ float rcp_in_range(float x) {
+    const float y = __builtin_amdgcn_rcpf(x);
+    return fmaf(fmaf(-x, y, 1.0f), y, y);
+}
+
+// Positions of 0 or of [2^-20, 2^20] in magnitude differ by 0 or at least 2^-43, so their squared
+// distances are 0 or in sqrt_in_range's range.
+__device__ __forceinline__ bool pos_operand(float x) {
+    const uint32_t u = __float_as_uint(x) & 0x7fffffffu;
+    return u == 0u || u - 0x35800000u <= 0x49800000u - 0x35800000u;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -464,7 +874,8 @@ __global__ __launch_bounds__(kHashBlock) void k_gather(Scenes S, uint32_t* __res
                                                        const uint32_t* __restrict__ id_in, uint32_t* __restrict__ id_out,
                                                        uint32_t* __restrict__ div_flags,
                                                        const uint2* __restrict__ crowd,
-                                                       const uint32_t* __restrict__ crowd_count, uint32_t crowd_cap) {
+                                                       const uint32_t* __restrict__ crowd_count, uint32_t crowd_cap,
+                                                       TileWork tiles) {
     __shared__ uint32_t s_v[kCrowdChunk];
     if (blockIdx.x < kCrowdBlocks) {  // the leading workgroups take the crowded cells k_place listed
         gather_crowded_cells(S, crowd, crowd_count, crowd_cap, slot_tmp, range, posrho_in,
@@ -473,7 +884,11 @@ __global__ __launch_bounds__(kHashBlock) void k_gather(Scenes S, uint32_t* __res
         return;
     }
     // kCrowdBlocks is a multiple of the XCD count, so block b still runs on XCD b mod 8
-    const uint32_t b = xcd_block(blockIdx.x - kCrowdBlocks, gridDim.x - kCrowdBlocks);
+    if (blockIdx.x >= kCrowdBlocks + S.blocks256) {  // the listed boxes' tables
+        form_tables(S, range, tiles, blockIdx.x - kCrowdBlocks - S.blocks256, gridDim.x - kCrowdBlocks - S.blocks256);
+        return;
+    }
+    const uint32_t b = xcd_block(blockIdx.x - kCrowdBlocks, S.blocks256);
     const uint32_t s = scene_of(S.scene256, S.num_scenes, b);
     const SceneDesc& d = S.desc[s];
     const uint32_t lt = (b - S.blk256[s]) * kHashBlock + threadIdx.x;
@@ -640,7 +1055,7 @@ __global__ __launch_bounds__(BLOCK) void k_density(Scenes S, float4* __restrict_
         reinterpret_cast<float*>(posrho)[4 * (size_t)t + 3] = density;
         reinterpret_cast<float*>(velp)[4 * (size_t)t + 3] = pressure;
         // the other operands of the force pass's quotients (the sort checks the velocities)
-        const bool ok = div_operand(p.x) && div_operand(p.y) && div_operand(p.z) && div_operand(pressure) &&
+        const bool ok = pos_operand(p.x) && pos_operand(p.y) && pos_operand(p.z) && div_operand(pressure) &&
                         div_operand(density) && density != 0.0f;
         if (!ok) atomicOr(&rho_max[1], kDivUnsafe);
     }
@@ -776,6 +1191,29 @@ struct ForceSums {
             vfz = vfz + (c.m * ((qv.z - pv.z) / q.w)) * wv;
         }
         return dist;
+    }
+
+    // The same sums with the square root and the reciprocals in their short forms: every operand
+    // passes div_operand (positions pos_operand), so each step rounds as in add.  The pair pressure is
+    // half the quotient by rho_j, exactly, and the half goes into the mass (a power of two).
+    __device__ __forceinline__ void add_in_range(const StepConsts& c, const float4& p, const float4& pv, const float4& q,
+                                                 const float4& qv) {
+        const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
+        const float dist = sqrt_in_range((rx * rx + ry * ry) + rz * rz);
+        const float iw = rcp_in_range(q.w);
+        const float twice = quot(pv.w + qv.w, q.w, iw);  // twice the pair pressure
+        const float mp = twice > 0.0f ? (0.5f * c.m) * twice : 0.0f;
+        const float dd = dist + 1e-16f;
+        const float y = rcp_in_range(dd);
+        const float a = c.h - dd;
+        const float s = a * a;
+        pfx = pfx - mp * ((s * quot(rx, dd, y)) * c.spiky);
+        pfy = pfy - mp * ((s * quot(ry, dd, y)) * c.spiky);
+        pfz = pfz - mp * ((s * quot(rz, dd, y)) * c.spiky);
+        const float wv = (c.h - dist) * c.visc;
+        vfx = vfx + (c.m * quot(qv.x - pv.x, q.w, iw)) * wv;
+        vfy = vfy + (c.m * quot(qv.y - pv.y, q.w, iw)) * wv;
+        vfz = vfz + (c.m * quot(qv.z - pv.z, q.w, iw)) * wv;
     }
 };
 
@@ -1018,6 +1456,637 @@ __global__ __launch_bounds__(BLOCK) void k_update(Scenes S, const float4* __rest
     if (id_out) id_out[t] = id_sorted[t];
     // completion time of this wave's particles; the scene's latest wave ends its step
     if ((threadIdx.x & 63) == 0) atomicMax(&scene_done[s], (unsigned long long)wall_clock64());
+}
+
+// ------------------------------------------------------------------------------------------
+// Tile passes: density and forces of one box of cells per workgroup, neighbours in LDS.
+//
+// The per-particle search above spends 14 VALU instructions and a 12-byte L1 return on each of the
+// about 216 candidates of a particle, and the list-driven force pass waits on neighbour gathers
+// through a 32 KB L1.  Here a workgroup copies the records of its box of cells and of the cells
+// around it into LDS once, and
+//   - the density pass forms candidate distances on the matrix cores (tile_search), which leaves one
+//     VALU instruction per candidate and lane;
+//   - both passes read neighbours from LDS.  The density pass leaves each particle's accepted
+//     neighbours as 16-bit indices into the staged records (half the bytes of slots), and the force
+//     pass, which stages the same boxes the same way, walks them.
+// Sums are formed in the reference's order with the reference's operations, so results are the same
+// bits as those of the per-particle passes.
+//
+// Measured against those (us, density + force): the 80,000-particle scene 120 + 202 -> 92 + 64, 192,089
+// particles 90 + 125 -> 84 + 57, the million-particle block 265 + 217 -> 163 + 117, 17.8 million
+// 3,582 + 3,762 -> 2,107 + 1,710; the work list and tables cost the sort 17 us of the million's step.
+//
+// The density pass is bound by VALU issue and, below 4 boxes a CU, by its chain of dependent loads; the force
+// pass by LDS reads (32 bytes a neighbour) and arithmetic.  512 threads and 1,920 records let three density
+// workgroups into a CU's LDS and registers (80 of them), and two force workgroups; 256 threads and 2,304
+// records suit boxes of at most 256 particles and cells of up to 85, at 4 and 2.
+// ------------------------------------------------------------------------------------------
+// The box's table into sh: as k_gather formed it, or formed here for entries past its memory.
+template <int BLOCK>
+__device__ __forceinline__ void box_open(BoxShared& sh, const Box& b, const SceneDesc& d, const uint2* __restrict__ range,
+                                         const BoxTable* __restrict__ tables, uint32_t item, uint32_t table_cap) {
+    if (threadIdx.x == 0) sh.rho = 0u;
+    if (item < table_cap) {  // workgroup-uniform
+        for (uint32_t k = threadIdx.x; k < sizeof(BoxTable) / 16; k += BLOCK)
+            reinterpret_cast<uint4*>(static_cast<BoxTable*>(&sh))[k] = reinterpret_cast<const uint4*>(tables + item)[k];
+    } else {
+        box_cells<BLOCK>(sh, b, d, range);
+    }
+}
+
+// The work of a pass: a single scene's sparse particles in chunks of BLOCK first, dealt round to the XCDs, then the
+// listed boxes, neighbours on one XCD.
+struct TileItems {
+    uint32_t boxes, sparse, lead, all;  // lead: items of the chunks, a multiple of kNumXcd
+};
+template <int BLOCK>
+__device__ __forceinline__ TileItems tile_items(const Scenes& S, const uint32_t* __restrict__ count, uint32_t cap) {
+    TileItems t;
+    t.boxes = min(count[0], cap);
+    t.sparse = S.num_scenes == 1 ? min(count[1], S.total_particles) : 0u;
+    t.lead = ((t.sparse + BLOCK - 1) / BLOCK + kNumXcd - 1) / kNumXcd * kNumXcd;
+    t.all = t.lead + t.boxes;
+    return t;
+}
+template <int BLOCK>
+__device__ __forceinline__ uint4 tile_item(const TileItems& t, const uint4* __restrict__ tiles, uint32_t item,
+                                           uint32_t& at_list) {
+    at_list = 0u;
+    if (item < t.lead) {
+        const uint32_t first = min(item * BLOCK, t.sparse);
+        return make_uint4(0u, kEntryDirect | kEntrySparse | min((uint32_t)BLOCK, t.sparse - first) << 13, 0u, first);
+    }
+    at_list = item - t.lead;
+    if (t.all <= gridDim.x) at_list = xcd_block(at_list, t.boxes);
+    return tiles[at_list];
+}
+
+// Copies the box's records: store(LDS index, record, slot) for each.  Eight lanes take a cell, neighbours in
+// x side by side, with up to 16 records of kFlight cells in flight.  The table is read where box_open reads it,
+// without waiting for sh.
+template <int BLOCK, typename Load, typename Store>
+__device__ __forceinline__ void box_stage_from(const Box& b, const BoxTable* table, uint32_t cap, Load load, Store store) {
+    constexpr int kFlight = 3, kGroups = BLOCK / 8;
+    const uint32_t sub = threadIdx.x & 7u;
+    const int ncell = b.hx * b.hy * b.hz;
+    using Rec = decltype(load(0u));
+    for (int i0 = (int)(threadIdx.x >> 3); i0 < ncell; i0 += kGroups * kFlight) {
+        Rec v[kFlight][2];
+        uint32_t at[kFlight], end[kFlight], slot[kFlight];
+#pragma unroll
+        for (int k = 0; k < kFlight; ++k) {
+            const int i = i0 + k * kGroups, c = table_cell(b, min(i, ncell - 1));
+            const uint32_t e = table->cell[c];
+            slot[k] = table->slot[c];
+            at[k] = (e & 0xffffu) + sub;
+            end[k] = i < ncell ? min(e >> 16, cap) : 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < kFlight; ++k) {
+            if (at[k] < end[k]) v[k][0] = load(at[k] + slot[k]);
+            if (at[k] + 8u < end[k]) v[k][1] = load(at[k] + 8u + slot[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < kFlight; ++k) {
+            if (at[k] < end[k]) store(at[k], v[k][0], at[k] + slot[k]);
+            if (at[k] + 8u < end[k]) store(at[k] + 8u, v[k][1], at[k] + 8u + slot[k]);
+        }
+        for (int k = 0; k < kFlight; ++k)  // cells of more than 16 records
+            for (uint32_t a = at[k] + 16u; a < end[k]; a += 8u) store(a, load(a + slot[k]), a + slot[k]);
+    }
+}
+
+template <int BLOCK, typename Load, typename Store>
+__device__ __forceinline__ void box_stage(const BoxShared& sh, const Box& b, const BoxTable* __restrict__ tables,
+                                          uint32_t item, uint32_t table_cap, uint32_t cap, Load load, Store store) {
+    if (item < table_cap)
+        box_stage_from<BLOCK>(b, tables + item, cap, load, store);
+    else
+        box_stage_from<BLOCK>(b, &sh, cap, load, store);
+}
+
+// The lane's particle: lane `at` of the box's `sh.own` numbering (lanes past a column's or the box's last
+// particle repeat it).
+struct BoxLane {
+    uint32_t idx;   // its record in LDS
+    uint32_t slot;
+    int cell;       // its halo cell
+    bool valid;
+};
+__device__ __forceinline__ BoxLane box_lane(const BoxShared& sh, const Box& b, uint32_t at, const SceneDesc& d) {
+    const uint32_t all = sh.own[kMaxBox * kMaxBox];
+    const uint32_t a = min(at, all - 1u);
+    int q = -1;  // the last column that starts at or before `a` (empty ones after it start past it or hold no lane)
+#pragma unroll
+    for (int k = 0; k < kMaxBox * kMaxBox; ++k) q += a >= sh.own[k] ? 1 : 0;
+    const int c0 = own_column(b, q);
+    const uint32_t st = sh.cell[c0 + 1] & 0xffffu, n = (sh.cell[c0 + b.nz] >> 16) - st;
+    uint32_t li = a - sh.own[q];
+    BoxLane L;
+    L.valid = at < all && li < n;
+    li = min(li, n - 1u);
+    L.idx = st + li;
+    L.cell = c0 + 1;
+    for (int k = 2; k <= b.nz; ++k) L.cell += L.idx >= (sh.cell[c0 + k] & 0xffffu) ? 1 : 0;
+    L.slot = L.idx + sh.slot[L.cell];
+    L.valid = L.valid && L.slot - d.p_off < d.c.n;  // always, unless the scan failed
+    return L;
+}
+
+// Candidates of a wave's particles, on the matrix cores.
+//
+// v_mfma_f32_4x4x1 (16 blocks) forms, for each group of four lanes, a 4x4 outer product: lane 4g + i
+// supplies row i (a candidate), lane 4g + j column j (its own particle), and lane 4g + j receives
+// column j in four registers.  Four of them (x, y, z, 1) accumulate
+//     C + sum_k (-2 a'_k) b_k + n_b,   C = n_a + 2 sum_k a'_k o_k - cut2 - margin,
+// with a' = a - o, n_a = |a'|^2, n_b = |b - o|^2 (staged beside the record) and o the box's centre:
+// that is |a - b|^2 - cut2 - margin, rounded.  Its sign bit marks a candidate; one v_alignbit per
+// register shifts it into the lane's mask.  The four lanes of a group are consecutive particles of a
+// column of cells along z, so their candidates in a neighbouring column lie in one window of three or
+// four cells (more where cells hold fewer than four).
+//
+// Rounding: |a'_k| and |b_k - o_k| are at most 3 bins and |b_k| at most the cube's size (boxes with
+// other particles search directly), so no partial sum exceeds 20 bin size and the eight roundings err
+// by less than 8 * 2^-24 * 20 bin size < 1e-5 bin size: margin = 1.2e-5 bin size makes the marked
+// candidates a superset of the accepted ones; the drain applies the exact test.
+//
+// A lane appends its marked candidates to its list in enumeration order: cells in NEIGHBORHOOD order,
+// candidates in slot order.
+typedef float mfma_f4 __attribute__((ext_vector_type(4)));
+constexpr int kPosPad = 32 + 8;      // records read past a window's end
+
+__device__ __forceinline__ uint32_t group_first(uint32_t x) {  // of the group of four lanes
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x00, 0xf, 0xf, true);
+}
+__device__ __forceinline__ uint32_t group_last(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xff, 0xf, 0xf, true);
+}
+
+// Eight candidates from q (4 lanes' worth at q and at q + 4) into the low bits of mask, the first highest.
+__device__ __forceinline__ uint32_t mark_eight(const float4* q, float b0, float b1, float b2, const mfma_f4& cc,
+                                               uint32_t mask) {
+    const float4 p = q[0], r = q[4];
+    mfma_f4 u = __builtin_amdgcn_mfma_f32_4x4x1f32(p.w, 1.0f, cc, 0, 0, 0);
+    mfma_f4 v = __builtin_amdgcn_mfma_f32_4x4x1f32(r.w, 1.0f, cc, 0, 0, 0);
+    u = __builtin_amdgcn_mfma_f32_4x4x1f32(p.x, b0, u, 0, 0, 0);
+    v = __builtin_amdgcn_mfma_f32_4x4x1f32(r.x, b0, v, 0, 0, 0);
+    u = __builtin_amdgcn_mfma_f32_4x4x1f32(p.y, b1, u, 0, 0, 0);
+    v = __builtin_amdgcn_mfma_f32_4x4x1f32(r.y, b1, v, 0, 0, 0);
+    u = __builtin_amdgcn_mfma_f32_4x4x1f32(p.z, b2, u, 0, 0, 0);
+    v = __builtin_amdgcn_mfma_f32_4x4x1f32(r.z, b2, v, 0, 0, 0);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(u[k]), 31);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(v[k]), 31);
+    return mask;
+}
+
+// One column (dx, dy) of three cells at a time, in NEIGHBORHOOD order: append(bits, first) receives a window's
+// marked candidates 32 at a time, bit 31 - k for record first + k.
+template <typename Append>
+__device__ __forceinline__ void tile_search(const BoxShared& sh, const Box& b, const float4* s_pos, const BoxLane& L,
+                                            float b0, float b1, float b2, float c0, Append append) {
+    const uint32_t sub = lane_id() & 3u;
+    const mfma_f4 cc = {c0, c0, c0, c0};
+    const int sy = b.hz, sx = b.hy * b.hz;
+    const lds_ptr<const uint32_t> table = (lds_ptr<const uint32_t>)sh.cell + (L.cell - 1 - sy - sx);
+    uint32_t lo = table[0], hi = table[2];
+#pragma unroll 1
+    for (int dx = 0; dx < 3; ++dx) {
+#pragma unroll 1
+        for (int dy = 0; dy < 3; ++dy) {
+            const uint32_t st = lo & 0xffffu, en = hi >> 16;
+            // the next column's entries (past the last, some entries of the table)
+            const int next = dy < 2 ? dx * sx + (dy + 1) * sy : (dx < 2 ? (dx + 1) * sx : 0);
+            lo = table[next];
+            hi = table[next + 2];
+            const uint32_t w0 = group_first(st), len = group_last(en) - w0;
+            for (uint32_t w = 0; __any(w < len); w += 32u) {
+                const float4* const q = s_pos + w0 + min(w, len) + sub;
+                uint32_t mask = mark_eight(q, b0, b1, b2, cc, 0u);
+                int got = 24;
+                if (__any(len > w + 8u)) {  // wave-uniform, as below
+                    mask = mark_eight(q + 8, b0, b1, b2, cc, mask);
+                    got = 16;
+                    if (__any(len > w + 16u)) {
+                        mask = mark_eight(q + 16, b0, b1, b2, cc, mask);
+                        got = 8;
+                        if (__any(len > w + 24u)) {
+                            mask = mark_eight(q + 24, b0, b1, b2, cc, mask);
+                            got = 0;
+                        }
+                    }
+                }
+                mask <<= got;  // candidate w0 + w + k at bit 31 - k
+                // the lane's own three cells
+                const uint32_t from = max(st, w0 + w);
+                const int n = (int)(min(en, w0 + w + 32u) - from);
+                uint32_t m = n > 0 ? mask << (from - w0 - w) & (uint32_t)((int)0x80000000u >> (n - 1)) : 0u;
+                if (dx == 1 && dy == 1) {  // not the particle itself
+                    const uint32_t self = L.idx - from;
+                    m &= self < 32u ? ~(0x80000000u >> self) : ~0u;
+                }
+                append(m, from);
+            }
+        }
+    }
+}
+
+template <int BLOCK, int CAP, int WPE, bool GLOBAL>
+__global__ __launch_bounds__(BLOCK, WPE) void k_density_tile(Scenes S, const uint4* __restrict__ tiles,
+                                                        const uint32_t* __restrict__ tile_count, uint32_t tile_cap,
+                                                        const BoxTable* __restrict__ tables, uint32_t table_cap,
+                                                        const uint32_t* __restrict__ sparse,
+                                                        float4* __restrict__ posrho, float4* __restrict__ velp,
+                                                        const uint32_t* __restrict__ skey,
+                                                        const uint2* __restrict__ range, uint32_t* __restrict__ rho_max,
+                                                        uint16_t* __restrict__ llist, uint16_t* __restrict__ lcount,
+                                                        uint32_t list_cap, uint32_t list_chunks, uint32_t* __restrict__ nlist,
+                                                        uint32_t* __restrict__ ncount) {
+    constexpr uint32_t kFar = CAP + kPosPad;
+    __shared__ float4 s_pos[CAP + kPosPad + 1];
+    __shared__ uint32_t s_slot[GLOBAL ? CAP + kPosPad : 1];
+    __shared__ BoxShared sh;
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAnd(&rho_max[1], ~kDivPending);
+    const TileItems items = tile_items<BLOCK>(S, tile_count, tile_cap);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (threadIdx.x == 0) s_pos[kFar] = make_float4(1e30f, 1e30f, 1e30f, 1e30f);
+    for (uint32_t item = blockIdx.x; item < items.all; item += gridDim.x) {
+        uint32_t at_list;
+        const uint4 e = tile_item<BLOCK>(items, tiles, item, at_list);
+        const SceneDesc& d = S.desc[e.z];
+        const StepConsts c = d.c;
+        uint32_t top = 0;  // largest density of the lane's particles, as bits (NaN ranks highest)
+        auto finish = [&](uint32_t t, const float4& p, float rho) {
+            const float wall = c.wall_density ? wall_density(c, p.x, p.y, p.z) : 0.0f;
+            const float density = rho + wall;
+            const float pressure = eos(c, rho);
+            reinterpret_cast<float*>(posrho)[4 * (size_t)t + 3] = density;
+            reinterpret_cast<float*>(velp)[4 * (size_t)t + 3] = pressure;
+            const bool ok = pos_operand(p.x) && pos_operand(p.y) && pos_operand(p.z) && div_operand(pressure) &&
+                            div_operand(density) && density != 0.0f;
+            if (!ok) atomicOr(&rho_max[1], kDivUnsafe);
+            top = max(top, __float_as_uint(density) & 0x7fffffffu);
+        };
+        // a particle of a box with irregular positions: every candidate tested from HBM, added at once
+        auto direct = [&](uint32_t t) {
+            const float4 p = posrho[t];
+            float rho = c.m * poly6(c, 0.0f);
+            uint32_t written = 0;
+            auto visit = [&](uint32_t start, uint32_t end, auto own) {
+                for (uint32_t u = start; u < end; ++u) {
+                    if (decltype(own)::value && u == t) continue;
+                    const float4 q = posrho[u];
+                    const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
+                    const float d2 = (rx * rx + ry * ry) + rz * rz;
+                    if (d2 >= c.cut2) continue;
+                    rho += c.m * poly6(c, sqrtf(d2));
+                    if (GLOBAL && written < kNeighbourListMax) nlist[(size_t)written * S.total_particles + t] = u;
+                    ++written;
+                }
+            };
+            auto nothing = []() {};
+            for_each_neighbour_cell(skey[t], range + d.c_off, c, d.p_off + c.n, visit, nothing);
+            if (GLOBAL) ncount[t] = written <= kNeighbourListMax ? written : kListOverflow;
+            finish(t, p, rho);
+        };
+        if (e.y & kEntryDirect) {
+            if (threadIdx.x == 0) sh.rho = 0u;
+            __syncthreads();
+            using Entry = typename std::conditional<GLOBAL, uint32_t, float>::type;
+            constexpr int kFit = (int)(sizeof(float4) * CAP / (BLOCK * sizeof(Entry))), kDirectCap = kFit < 40 ? kFit : 40;  // the search's lists take the records' place
+            const lds_ptr<Entry> found = (lds_ptr<Entry>)reinterpret_cast<Entry*>(s_pos) + threadIdx.x;
+            for (uint32_t i = threadIdx.x; i < e.y >> 13; i += BLOCK) {
+                const uint32_t t = e.y & kEntrySparse ? sparse[min(e.w + i, S.total_particles - 1u)] : e.w + i;
+                if (t - d.p_off >= c.n) continue;  // only after a failed scan
+                const float4 p = posrho[t];
+                float rho = c.m * poly6(c, 0.0f);
+                uint32_t written = 0;
+                auto drain = [&](int cnt) {
+                    for (int k = 0; k < cnt; ++k) {
+                        if constexpr (GLOBAL) {
+                            const uint32_t u = found[k * BLOCK];
+                            const float4 q = posrho[u];
+                            const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
+                            const float d2 = (rx * rx + ry * ry) + rz * rz;
+                            rho += c.m * poly6(c, sqrtf(d2));
+                            if (written < kNeighbourListMax) nlist[(size_t)written * S.total_particles + t] = u;
+                            ++written;
+                        } else {
+                            rho += c.m * poly6(c, sqrtf(found[k * BLOCK]));
+                        }
+                    }
+                };
+                search_neighbours<BLOCK, kDirectCap, 4, false>(skey[t], t, d.p_off + c.n, p.x, p.y, p.z, posrho,
+                                                               range + d.c_off, c, found, drain);
+                if (GLOBAL) ncount[t] = written <= kNeighbourListMax ? written : kListOverflow;
+                finish(t, p, rho);
+            }
+        } else {
+            const Box b = box_of(e);
+            box_open<BLOCK>(sh, b, d, range, tables, at_list, table_cap);
+            const float ox = ((float)b.x + 0.5f * (float)b.nx) * c.bin, oy = ((float)b.y + 0.5f * (float)b.ny) * c.bin,
+                        oz = ((float)b.z + 0.5f * (float)b.nz) * c.bin;
+            const float reach = 3.001f * c.bin;
+            bool bad = false;
+            box_stage<BLOCK>(
+                sh, b, tables, at_list, table_cap, CAP, [&](uint32_t slot) { return posrho[min(slot, d.p_off + c.n - 1u)]; },
+                [&](uint32_t at, float4 q, uint32_t slot) {
+                    const float x = q.x - ox, y = q.y - oy, z = q.z - oz;
+                    bad |= !(fabsf(x) <= reach && fabsf(y) <= reach && fabsf(z) <= reach && pos_operand(q.x) &&
+                             pos_operand(q.y) && pos_operand(q.z));
+                    q.w = (x * x + y * y) + z * z;
+                    s_pos[at] = q;
+                    if (GLOBAL) s_slot[at] = slot;
+                });
+            const bool irregular = __syncthreads_or(bad ? 1 : 0) != 0;
+            if (sh.records > CAP) {  // only after a failed scan
+                __syncthreads();
+                continue;
+            }
+            const uint32_t lanes = sh.own[kMaxBox * kMaxBox];
+            const float cut = c.cut2 + 1.2e-5f * (c.bin * c.size);
+            const bool room = e.w + (lanes + 63u) / 64u <= list_chunks, listable = room && !irregular;
+            bool overflowed = false;
+            for (uint32_t ch = (uint32_t)wave; ch * 64u < lanes; ch += BLOCK / 64) {
+                const BoxLane L = box_lane(sh, b, ch * 64u + lane_id(), d);
+                const float4 p = s_pos[L.idx];
+                char* const list = reinterpret_cast<char*>(llist) + (size_t)(e.w + ch) * (list_cap * 128u) + lane_id() * 2u;
+                uint32_t cnt = list_cap + 1u;  // no list: as an overflowed one
+                if (listable) {                // workgroup-uniform
+                    const float ax = p.x - ox, ay = p.y - oy, az = p.z - oz;
+                    // lanes that repeat a particle mark nothing
+                    const float c0 = L.valid ? (p.w - cut) + 2.0f * ((ax * ox + ay * oy) + az * oz) : 1e30f;
+                    // Candidates go to the particle's list: a queue in LDS would take 4 KB a wave, and half the
+                    // waves of a CU with it.  Past the list's end they are only counted.
+                    char* const list_end = list + list_cap * 128u;
+                    char* next = list;
+                    auto append = [&](uint32_t m, uint32_t first) {
+                        if (__any(next + 32 * 128 > list_end)) {  // wave-uniform
+                            for (; m != 0u; next += 128) {
+                                const uint32_t k = (uint32_t)__builtin_clz(m);
+                                m ^= 0x80000000u >> k;
+                                if (next < list_end) *reinterpret_cast<uint16_t*>(next) = (uint16_t)((first + k) << 4);
+                            }
+                        } else {
+                            for (; m != 0u; next += 128) {
+                                const uint32_t k = (uint32_t)__builtin_clz(m);
+                                m ^= 0x80000000u >> k;
+                                *reinterpret_cast<uint16_t*>(next) = (uint16_t)((first + k) << 4);
+                            }
+                        }
+                    };
+                    tile_search(sh, b, s_pos, L, -2.0f * ax, -2.0f * ay, -2.0f * az, c0, append);
+                    cnt = (uint32_t)(next - list) / 128u;
+                }
+                if (!L.valid) continue;
+                if (room) lcount[(e.w + ch) * 64u + lane_id()] = (uint16_t)min(cnt, list_cap + 1u);
+                if (cnt > list_cap) {
+                    overflowed = true;
+                    continue;
+                }
+                // The exact test and the sum, in order, kAhead candidates a round with the next round's in
+                // flight.  Past its list a lane takes the record kFar, out of everything's reach.
+                constexpr uint32_t kAhead = 4;
+                const char* const rec = reinterpret_cast<const char*>(s_pos);
+                auto entry = [&](uint32_t k) { return (uint32_t)*reinterpret_cast<const uint16_t*>(list + k * 128u); };
+                auto dist2 = [&](uint32_t o) {
+                    const float4 q = *reinterpret_cast<const float4*>(rec + o);
+                    const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
+                    return (rx * rx + ry * ry) + rz * rz;
+                };
+                float rho = c.m * poly6(c, 0.0f);
+                uint32_t written = 0;  // accepted so far
+                uint32_t off[kAhead];
+#pragma unroll
+                for (uint32_t j = 0; j < kAhead; ++j) off[j] = entry(j);
+                for (uint32_t k = 0; __any(k < cnt); k += kAhead) {
+                    uint32_t cur[kAhead];
+#pragma unroll
+                    for (uint32_t j = 0; j < kAhead; ++j) cur[j] = k + j < cnt ? off[j] : kFar << 4;
+                    const uint32_t ahead = min(k + kAhead, list_cap - kAhead);  // wave-uniform
+#pragma unroll
+                    for (uint32_t j = 0; j < kAhead; ++j) off[j] = entry(ahead + j);
+                    const uint32_t before = written;
+#pragma unroll
+                    for (uint32_t j = 0; j < kAhead; ++j) {
+                        const float d2 = dist2(cur[j]);
+                        const float sum = rho + c.m * poly6(c, sqrt_in_range(d2));
+                        const bool in = d2 < c.cut2;
+                        rho = in ? sum : rho;
+                        if (GLOBAL && in && written < kNeighbourListMax)
+                            nlist[(size_t)written * S.total_particles + L.slot] = s_slot[cur[j] >> 4];
+                        written += in ? 1u : 0u;
+                    }
+                    // a rejected candidate (one within the margin) becomes the particle itself, which adds
+                    // nothing to the force sums
+                    if (__any(k < cnt && written - before != min(cnt - k, kAhead))) {
+#pragma unroll
+                        for (uint32_t j = 0; j < kAhead; ++j)
+                            if (k + j < cnt && !(dist2(cur[j]) < c.cut2))
+                                *reinterpret_cast<uint16_t*>(list + (k + j) * 128u) = (uint16_t)(L.idx << 4);
+                    }
+                }
+                if (GLOBAL) ncount[L.slot] = written <= kNeighbourListMax ? written : kListOverflow;
+                finish(L.slot, p, rho);
+            }
+            // Lanes without a list, after the others: the search's state next to theirs would spill.
+            if (__any(overflowed)) {
+                for (uint32_t ch = (uint32_t)wave; ch * 64u < lanes; ch += BLOCK / 64) {
+                    const BoxLane L = box_lane(sh, b, ch * 64u + lane_id(), d);
+                    if (L.valid && (!room || lcount[(e.w + ch) * 64u + lane_id()] > list_cap)) direct(L.slot);
+                }
+            }
+        }
+        for (int k = 32; k >= 1; k >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, k));
+        if (lane_id() == 0) atomicMax(&sh.rho, top);
+        __syncthreads();
+        if (threadIdx.x == 0) atomicMax(rho_max, sh.rho);
+        __syncthreads();
+    }
+}
+
+// Forces + integration of one box per workgroup.  MODE 0 and 1 as in k_update.
+template <int BLOCK, int CAP, int WPE, int MODE>
+__global__ __launch_bounds__(BLOCK, WPE) void k_update_tile(Scenes S, const uint4* __restrict__ tiles,
+                                                       const uint32_t* __restrict__ tile_count, uint32_t tile_cap,
+                                                       const BoxTable* __restrict__ tables, uint32_t table_cap,
+                                                       const uint32_t* __restrict__ sparse,
+                                                       const float4* __restrict__ posrho_in,
+                                                       const float4* __restrict__ velp_in,
+                                                       const uint32_t* __restrict__ skey,
+                                                       const uint2* __restrict__ range, float4* __restrict__ posrho_out,
+                                                       float4* __restrict__ velp_out,
+                                                       unsigned long long* __restrict__ scene_done,
+                                                       const uint32_t* __restrict__ id_sorted,
+                                                       uint32_t* __restrict__ id_out, const uint16_t* __restrict__ llist,
+                                                       const uint16_t* __restrict__ lcount, uint32_t list_cap,
+                                                       uint32_t list_chunks,
+                                                       const uint32_t* __restrict__ div_flags, float dt_arg,
+                                                       const float4* __restrict__ corr, float corr_scale,
+                                                       float4* __restrict__ acc_out, float substeps,
+                                                       RecordBackup backup) {
+    __shared__ float4 s_rec[2 * CAP];
+    float4* const s_pos = s_rec;
+    float4* const s_vel = s_rec + CAP;
+    __shared__ BoxShared sh;
+    const TileItems items = tile_items<BLOCK>(S, tile_count, tile_cap);
+    const uint32_t flags = div_flags[0];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    for (uint32_t item = blockIdx.x; item < items.all; item += gridDim.x) {
+        uint32_t at_list;
+        const uint4 e = tile_item<BLOCK>(items, tiles, item, at_list);
+        const SceneDesc& d = S.desc[e.z];
+        const StepConsts c = d.c;
+        auto finish = [&](uint32_t t, const float4& p, const float4& pv, const ForceSums& f) {
+            if (backup.posrho) {
+                backup.posrho[t] = p;
+                backup.velp[t] = pv;
+                if (backup.ids && id_sorted) backup.ids[t] = id_sorted[t];
+            }
+            V3 ext{c.g[0] * p.w, c.g[1] * p.w, c.g[2] * p.w};
+            V3 mouse{0.0f, 0.0f, 0.0f}, wall{0.0f, 0.0f, 0.0f};
+            if (c.mouse_force) mouse = mouse_force(c, p.x, p.y, p.z, pv.w);
+            if (c.wall_force) wall = wall_forces(c, p.x, p.y, p.z);
+            ext.x = ext.x + (mouse.x + wall.x);
+            ext.y = ext.y + (mouse.y + wall.y);
+            ext.z = ext.z + (mouse.z + wall.z);
+            const float denom = p.w + 1e-16f;
+            float4 po, vo;
+            if (MODE == 0) {
+                const float dt = d.dt;
+                integrate_axis(c, f.pfx, f.vfx, ext.x, denom, pv.x, p.x, dt, vo.x, po.x);
+                integrate_axis(c, f.pfy, f.vfy, ext.y, denom, pv.y, p.y, dt, vo.y, po.y);
+                integrate_axis(c, f.pfz, f.vfz, ext.z, denom, pv.z, p.z, dt, vo.z, po.z);
+            } else {
+                V3 kc{0.0f, 0.0f, 0.0f};
+                if (corr) {
+                    const float4 ct = corr[t];
+                    kc = V3{ct.x, ct.y, ct.z};
+                }
+                learned_integrate(c, f, ext, denom, p, pv, t, dt_arg, substeps, corr != nullptr, kc, corr_scale, acc_out,
+                                  po, vo);
+            }
+            po.w = p.w;
+            vo.w = pv.w;
+            posrho_out[t] = po;
+            velp_out[t] = vo;
+            if (id_out) id_out[t] = id_sorted[t];
+        };
+        // a particle without a list: every candidate tested from HBM, added at once
+        auto direct = [&](uint32_t t) {
+            const float4 p = posrho_in[t], pv = velp_in[t];
+            ForceSums f{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+            auto visit = [&](uint32_t start, uint32_t end, auto own) {
+                for (uint32_t u = start; u < end; ++u) {
+                    if (decltype(own)::value && u == t) continue;
+                    const float4 q = posrho_in[u];
+                    const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
+                    const float d2 = (rx * rx + ry * ry) + rz * rz;
+                    if (d2 >= c.cut2) continue;
+                    f.template add<false>(c, p, pv, q, velp_in[u]);
+                }
+            };
+            auto nothing = []() {};
+            for_each_neighbour_cell(skey[t], range + d.c_off, c, d.p_off + c.n, visit, nothing);
+            finish(t, p, pv, f);
+        };
+        if (e.y & kEntryDirect) {
+            constexpr int kFit = (int)(2 * sizeof(float4) * CAP / (BLOCK * sizeof(uint32_t))), kDirectCap = kFit < 40 ? kFit : 40;  // the search's lists take the records' place
+            const lds_ptr<uint32_t> found = (lds_ptr<uint32_t>)reinterpret_cast<uint32_t*>(s_rec) + threadIdx.x;
+            for (uint32_t i = threadIdx.x; i < e.y >> 13; i += BLOCK) {
+                const uint32_t t = e.y & kEntrySparse ? sparse[min(e.w + i, S.total_particles - 1u)] : e.w + i;
+                if (t - d.p_off >= c.n) continue;  // only after a failed scan
+                const float4 p = posrho_in[t], pv = velp_in[t];
+                ForceSums f{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+                auto drain = [&](int cnt) {
+                    for (int k = 0; k < cnt; ++k) {
+                        const uint32_t u = found[k * BLOCK];
+                        if (flags == 0u)
+                            f.add_in_range(c, p, pv, posrho_in[u], velp_in[u]);
+                        else
+                            f.template add<false>(c, p, pv, posrho_in[u], velp_in[u]);
+                    }
+                };
+                search_neighbours<BLOCK, kDirectCap, 4, false>(skey[t], t, d.p_off + c.n, p.x, p.y, p.z, posrho_in,
+                                                               range + d.c_off, c, found, drain);
+                finish(t, p, pv, f);
+            }
+        } else {
+            const Box b = box_of(e);
+            box_open<BLOCK>(sh, b, d, range, tables, at_list, table_cap);
+            struct Rec {
+                float4 p, v;
+            };
+            box_stage<BLOCK>(
+                sh, b, tables, at_list, table_cap, CAP,
+                [&](uint32_t slot) {
+                    const uint32_t u = min(slot, d.p_off + c.n - 1u);
+                    return Rec{posrho_in[u], velp_in[u]};
+                },
+                [&](uint32_t at, const Rec& r, uint32_t) {
+                    s_pos[at] = r.p;
+                    s_vel[at] = r.v;
+                });
+            __syncthreads();
+            if (sh.records > CAP) {  // only after a failed scan
+                __syncthreads();
+                continue;
+            }
+            const uint32_t lanes = sh.own[kMaxBox * kMaxBox];
+            const bool listed_box = !(flags & kDivPending) && e.w + (lanes + 63u) / 64u <= list_chunks;
+            for (uint32_t ch = (uint32_t)wave; ch * 64u < lanes; ch += BLOCK / 64) {
+                const BoxLane L = box_lane(sh, b, ch * 64u + lane_id(), d);
+                if (!L.valid) continue;
+                const uint32_t cnt = listed_box ? (uint32_t)lcount[(e.w + ch) * 64u + lane_id()] : list_cap + 1u;
+                if (cnt > list_cap) {
+                    direct(L.slot);
+                    continue;
+                }
+                const float4 p = s_pos[L.idx], pv = s_vel[L.idx];
+                ForceSums f{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+                const char* const list =
+                    reinterpret_cast<const char*>(llist) + (size_t)(e.w + ch) * (list_cap * 128u) + lane_id() * 2u;
+                const char* const rec_p = reinterpret_cast<const char*>(s_pos);
+                const char* const rec_v = reinterpret_cast<const char*>(s_vel);
+                auto entry = [&](uint32_t k) {
+                    return (uint32_t)*reinterpret_cast<const uint16_t*>(list + k * 128u);
+                };
+                auto pos = [&](uint32_t off) { return *reinterpret_cast<const float4*>(rec_p + off); };
+                auto vel = [&](uint32_t off) { return *reinterpret_cast<const float4*>(rec_v + off); };
+                if (flags == 0u) {
+                    // All lanes run to the longest list of the wave, kAhead entries a round, the next round's
+                    // offsets in flight.  Past its list a lane takes its own record, which adds nothing: the
+                    // differences are 0, and every sum keeps its bits (it starts at +0, see ForceSums).
+                    constexpr uint32_t kAhead = 4;
+                    const uint32_t self = L.idx << 4;
+                    uint32_t off[kAhead];
+#pragma unroll
+                    for (uint32_t j = 0; j < kAhead; ++j) off[j] = entry(j);
+                    for (uint32_t k = 0; __any(k < cnt); k += kAhead) {
+                        uint32_t cur[kAhead];
+#pragma unroll
+                        for (uint32_t j = 0; j < kAhead; ++j) cur[j] = k + j < cnt ? off[j] : self;
+                        const uint32_t ahead = min(k + kAhead, list_cap - kAhead);  // wave-uniform
+#pragma unroll
+                        for (uint32_t j = 0; j < kAhead; ++j) off[j] = entry(ahead + j);
+#pragma unroll
+                        for (uint32_t j = 0; j < kAhead; ++j) f.add_in_range(c, p, pv, pos(cur[j]), vel(cur[j]));
+                    }
+                } else {
+                    for (uint32_t k = 0; k < cnt; ++k) {
+                        const uint32_t u = min(entry(k), (sh.records - 1u) << 4);
+                        if (u == L.idx << 4) continue;  // a rejected candidate
+                        f.template add<false>(c, p, pv, pos(u), vel(u));
+                    }
+                }
+                finish(L.slot, p, pv, f);
+            }
+        }
+        __syncthreads();  // the box's last particle is done
+        if (threadIdx.x == 0) atomicMax(&scene_done[e.z], (unsigned long long)wall_clock64());
+    }
 }
 
 
@@ -1707,7 +2776,7 @@ hipError_t launch_hash(const DeviceBuffers& b, hipStream_t s) {
     if (reset > blocks) blocks = reset;
     if (blocks == 0) blocks = 1;  // still resets the step clock
     hipLaunchKernelGGL(k_hash, dim3((unsigned)blocks), dim3(kHashBlock), 0, s, S, b.posrho[0], b.key, b.rank,
-                       b.counts, b.scan_status, b.scene_done, b.step_start, b.rho_max, b.crowd_count);
+                       b.counts, b.scan_status, b.scene_done, b.step_start, b.rho_max, b.crowd_count, b.tile_count);
     return hipGetLastError();
 }
 
@@ -1718,19 +2787,34 @@ hipError_t launch_scan(const DeviceBuffers& b, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_place(const DeviceBuffers& b, hipStream_t s) {
+static unsigned tile_grid(const DeviceBuffers& b) {
+    // About one workgroup per box where boxes hold 8 particles a cell, and the chip's fill where most hold
+    // fewer; a longer list is walked with this stride.
+    const uint64_t most = (uint64_t)b.sc.total_particles / (8 * b.sc.bx * b.sc.by * b.sc.bz) + 512;
+    return (unsigned)(b.tile_cap < most ? b.tile_cap : most);
+}
+
+static TileWork tile_work(const DeviceBuffers& b, const TileShape* t) {
+    TileWork w{};
+    if (t) w = TileWork{b.tiles, b.tile_count, b.tile_cap, (uint32_t)t->cap, (uint32_t)t->block, b.tables, b.table_cap, b.sparse, kSparseRecords * (uint32_t)((t->x + 2) * (t->y + 2) * (t->z + 2))};
+    return w;
+}
+
+hipError_t launch_place(const DeviceBuffers& b, const TileShape* tiles, hipStream_t s) {
     if (b.sc.blocks256 == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_place, dim3(b.sc.blocks256), dim3(kHashBlock), 0, s, b.sc, b.key, b.rank, b.range,
-                       b.slot_tmp, b.crowd, b.crowd_count, b.crowd_cap, b.error_flag);
+    const unsigned extra = tiles ? b.sc.tblocks : 0u;
+    hipLaunchKernelGGL(k_place, dim3(b.sc.blocks256 + extra), dim3(kHashBlock), 0, s, b.sc, b.key, b.rank, b.range,
+                       b.slot_tmp, b.crowd, b.crowd_count, b.crowd_cap, b.error_flag, tile_work(b, tiles));
     return hipGetLastError();
 }
 
-hipError_t launch_gather(const DeviceBuffers& b, hipStream_t s) {
+hipError_t launch_gather(const DeviceBuffers& b, const TileShape* tiles, hipStream_t s) {
     if (b.sc.blocks256 == 0) return hipSuccess;
     static_assert(kCrowdBlocks % kNumXcd == 0, "the leading workgroups keep the XCD mapping of the others");
-    hipLaunchKernelGGL(k_gather, dim3(b.sc.blocks256 + kCrowdBlocks), dim3(kHashBlock), 0, s, b.sc, b.slot_tmp, b.key,
+    const unsigned extra = tiles ? tile_grid(b) : 0u;
+    hipLaunchKernelGGL(k_gather, dim3(b.sc.blocks256 + kCrowdBlocks + extra), dim3(kHashBlock), 0, s, b.sc, b.slot_tmp, b.key,
                        b.range, b.posrho[0], b.velp[0], b.posrho[1], b.velp[1], b.sorted, b.skey, b.ids[0],
-                       b.ids[1], b.rho_max + 1, b.crowd, b.crowd_count, b.crowd_cap);
+                       b.ids[1], b.rho_max + 1, b.crowd, b.crowd_count, b.crowd_cap, tile_work(b, tiles));
     return hipGetLastError();
 }
 
@@ -1753,9 +2837,11 @@ static const PassVariant kVariants[] = {
 #define WC_ROW(B, C, K, P) {B, C, K, P},
     WC_VARIANTS(WC_ROW)
 #undef WC_ROW
+    {384, (int)kNeighbourListMax, 4, true},  // the tile passes (their workgroup and box vary with the context)
 };
 
 int num_variants() { return (int)(sizeof(kVariants) / sizeof(kVariants[0])); }
+int tile_variant() { return num_variants() - 1; }
 PassVariant variant(int v) { return kVariants[(v >= 0 && v < num_variants()) ? v : 0]; }
 
 static unsigned pass_blocks(const Scenes& S, int block) {
@@ -1804,6 +2890,52 @@ hipError_t launch_update(const DeviceBuffers& b, int v, bool list, hipStream_t s
     WC_VARIANTS(WC_LAUNCH)
 #undef WC_LAUNCH
     return hipErrorInvalidValue;
+}
+
+// The two sizes of a tile workgroup: threads, staged records (then: waves per SIMD to compile for).
+#define WC_TILE_LARGE kTileLargeBlock, kTileLargeCap
+#define WC_TILE_SMALL kTileSmallBlock, kTileSmallCap
+
+template <int BLOCK, int CAP, int WPE>
+static void density_tile(const DeviceBuffers& b, bool list, hipStream_t s) {
+    if (list)
+        hipLaunchKernelGGL((k_density_tile<BLOCK, CAP, WPE, true>), dim3(tile_grid(b)), dim3(BLOCK), 0, s, b.sc, b.tiles,
+                           b.tile_count, b.tile_cap, reinterpret_cast<const BoxTable*>(b.tables), b.table_cap, b.sparse, b.posrho[1], b.velp[1], b.skey, b.range, b.rho_max, b.llist,
+                           b.lcount, b.list_cap, b.list_chunks, b.nlist, b.ncount);
+    else
+        hipLaunchKernelGGL((k_density_tile<BLOCK, CAP, WPE, false>), dim3(tile_grid(b)), dim3(BLOCK), 0, s, b.sc, b.tiles,
+                           b.tile_count, b.tile_cap, reinterpret_cast<const BoxTable*>(b.tables), b.table_cap, b.sparse, b.posrho[1], b.velp[1], b.skey, b.range, b.rho_max, b.llist,
+                           b.lcount, b.list_cap, b.list_chunks, nullptr, nullptr);
+}
+
+hipError_t launch_density_tile(const DeviceBuffers& b, const TileShape& t, bool list, hipStream_t s) {
+    if (list && (!b.nlist || !b.ncount)) return hipErrorInvalidValue;
+    if (t.block == kTileLargeBlock)
+        density_tile<WC_TILE_LARGE, 6>(b, list, s);
+    else
+        density_tile<WC_TILE_SMALL, 3>(b, list, s);
+    return hipGetLastError();
+}
+
+template <int BLOCK, int CAP, int WPE, int MODE>
+static void update_tile(const DeviceBuffers& b, const TileUpdate& u, hipStream_t s) {
+    hipLaunchKernelGGL((k_update_tile<BLOCK, CAP, WPE, MODE>), dim3(tile_grid(b)), dim3(BLOCK), 0, s, b.sc, b.tiles,
+                       b.tile_count, b.tile_cap, reinterpret_cast<const BoxTable*>(b.tables), b.table_cap, b.sparse, b.posrho[1], b.velp[1], b.skey, b.range, b.posrho[0], b.velp[0],
+                       b.scene_done, b.ids[1], b.ids[0], b.llist, b.lcount, b.list_cap, b.list_chunks, b.rho_max + 1, u.dt,
+                       reinterpret_cast<const float4*>(u.corr), u.corr_scale, reinterpret_cast<float4*>(u.acc_out),
+                       u.substeps, u.backup);
+}
+
+hipError_t launch_update_tile(const DeviceBuffers& b, const TileShape& t, const TileUpdate& u, hipStream_t s) {
+    if (t.block == kTileLargeBlock && u.learned)
+        update_tile<WC_TILE_LARGE, 2, 1>(b, u, s);
+    else if (t.block == kTileLargeBlock)
+        update_tile<WC_TILE_LARGE, 2, 0>(b, u, s);
+    else if (u.learned)
+        update_tile<WC_TILE_SMALL, 2, 1>(b, u, s);
+    else
+        update_tile<WC_TILE_SMALL, 2, 0>(b, u, s);
+    return hipGetLastError();
 }
 
 hipError_t launch_closure_features(const DeviceBuffers& b, const uint32_t* rows, uint32_t nrows, float dt_mult,
