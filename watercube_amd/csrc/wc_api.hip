@@ -1419,12 +1419,13 @@ WC_API int wc_mlp_create(uint32_t max_batch, uint64_t seed, wc_mlp** out) {
         alloc((void**)&m.z[l], B * wc::kMlpHidden * 4);
         alloc((void**)&m.h[l], B * wc::kMlpHidden * 2);
     }
-    alloc((void**)&m.yacc, B * wc::kMlpOutPad * 4);
     alloc((void**)&m.d4, B * wc::kMlpOutPad * 2);
-    alloc((void**)&m.gbuf, B * wc::kMlpHidden * 4);
-    alloc((void**)&m.d, B * wc::kMlpHidden * 2);
+    for (int k = 0; k < 2; ++k) alloc((void**)&m.d[k], B * wc::kMlpHidden * 2);
     alloc((void**)&m.loss, 64);
-    alloc((void**)&m.colpart, (B + wc::kColsumRows - 1) / wc::kColsumRows * wc::kMlpHidden * 4);
+    const size_t colpart = (B + wc::kColsumRows - 1) / wc::kColsumRows * wc::kMlpHidden;
+    alloc((void**)&m.colpart[0], 4 * colpart * 4);
+    for (int l = 1; l < 4; ++l) m.colpart[l] = m.colpart[0] ? m.colpart[0] + l * colpart : nullptr;
+    alloc((void**)&m.wpart, (size_t)wc::kMlpSplits * L.total * 4);
     if (!ok) {
         wc_mlp_destroy(h);
         return fail(WC_ERR_NO_MEMORY, "network buffers for a batch of %u", max_batch);
@@ -1468,8 +1469,8 @@ WC_API int wc_mlp_destroy(wc_mlp* h) {
     wc::Mlp& m = h->m;
     if (m.stream) (void)hipStreamSynchronize(m.stream);
     void* ptrs[] = {m.master, m.grad, m.adam_m, m.adam_v, m.w1, m.w1t, m.w2, m.w2t, m.w3, m.w3t, m.w4, m.w4t,
-                    m.z[0], m.z[1], m.z[2], m.h[0], m.h[1], m.h[2], m.yacc, m.d4, m.gbuf, m.d, m.loss,
-                    m.colpart};
+                    m.z[0], m.z[1], m.z[2], m.h[0], m.h[1], m.h[2], m.d4, m.d[0], m.d[1], m.loss,
+                    m.colpart[0], m.wpart};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (m.stream) (void)hipStreamDestroy(m.stream);
@@ -1514,12 +1515,12 @@ WC_API int wc_mlp_forward(wc_mlp* h, const void* x_dev, void* y_dev, uint32_t n)
     return WC_OK;
 }
 
-static int mlp_grad(wc_mlp* h, const void* x_dev, const void* t_dev, uint32_t n, double* loss) {
+static int mlp_grad(wc_mlp* h, const void* x_dev, const void* t_dev, uint32_t n, double* loss, bool adam, float lr) {
     if (!h || !x_dev || !t_dev) return fail(WC_ERR_INVALID_ARG, "NULL argument");
     if (n == 0 || n > h->m.max_batch) return fail(WC_ERR_CAPACITY, "batch %u outside [1, %u]", n, h->m.max_batch);
     wc::Mlp& m = h->m;
     WC_HIP(wc::mlp_forward_train(m, (const uint16_t*)x_dev, (const float*)t_dev, nullptr, n, m.stream));
-    WC_HIP(wc::mlp_backward(m, (const uint16_t*)x_dev, n, m.stream));
+    WC_HIP(wc::mlp_backward(m, (const uint16_t*)x_dev, n, adam, lr, m.stream));
     if (loss) {
         float sse = 0.0f;
         WC_HIP(hipMemcpyAsync(&sse, m.loss, 4, hipMemcpyDeviceToHost, m.stream));
@@ -1531,7 +1532,7 @@ static int mlp_grad(wc_mlp* h, const void* x_dev, const void* t_dev, uint32_t n,
 
 WC_API int wc_mlp_gradient(wc_mlp* h, const void* x_dev, const void* t_dev, uint32_t n, float* grad_host,
                            double* loss) {
-    int rc = mlp_grad(h, x_dev, t_dev, n, loss);
+    int rc = mlp_grad(h, x_dev, t_dev, n, loss, false, 0.0f);
     if (rc) return rc;
     if (grad_host) {
         WC_HIP(hipStreamSynchronize(h->m.stream));
@@ -1541,9 +1542,8 @@ WC_API int wc_mlp_gradient(wc_mlp* h, const void* x_dev, const void* t_dev, uint
 }
 
 WC_API int wc_mlp_train_step(wc_mlp* h, const void* x_dev, const void* t_dev, uint32_t n, float lr, double* loss) {
-    int rc = mlp_grad(h, x_dev, t_dev, n, loss);
+    int rc = mlp_grad(h, x_dev, t_dev, n, loss, true, lr);
     if (rc) return rc;
-    WC_HIP(wc::mlp_adam(h->m, lr, h->m.stream));
     if (!loss) WC_HIP(hipStreamSynchronize(h->m.stream));
     return WC_OK;
 }
@@ -1559,8 +1559,7 @@ WC_API int wc_mlp_profile_train(wc_mlp* h, const void* x_dev, const void* t_dev,
     if (err == hipSuccess) err = hipEventRecord(ev.start, h->m.stream);
     for (uint32_t r = 0; r < reps && err == hipSuccess; ++r) {
         err = wc::mlp_forward_train(h->m, (const uint16_t*)x_dev, (const float*)t_dev, nullptr, n, h->m.stream);
-        if (err == hipSuccess) err = wc::mlp_backward(h->m, (const uint16_t*)x_dev, n, h->m.stream);
-        if (err == hipSuccess) err = wc::mlp_adam(h->m, lr, h->m.stream);
+        if (err == hipSuccess) err = wc::mlp_backward(h->m, (const uint16_t*)x_dev, n, true, lr, h->m.stream);
     }
     if (err == hipSuccess) err = hipEventRecord(ev.stop, h->m.stream);
     if (err == hipSuccess) err = hipEventSynchronize(ev.stop);

@@ -22,6 +22,7 @@ struct MlpLayout {
 MlpLayout mlp_layout();
 
 constexpr int kColsumRows = 1024;  // rows per partial column sum of the bias gradients
+constexpr int kMlpSplits = 64;   // partial sums of a weight gradient at most
 
 struct Mlp {
     uint32_t max_batch = 0;
@@ -35,18 +36,15 @@ struct Mlp {
     // training workspace, max_batch rows each
     float* z[3] = {nullptr, nullptr, nullptr};     // pre-activations (fp32, 128 columns)
     uint16_t* h[3] = {nullptr, nullptr, nullptr};  // activations (bf16, 128 columns)
-    float* yacc = nullptr;                         // output layer before bias (32 columns)
     uint16_t* d4 = nullptr;                        // output delta (bf16, 32 columns)
-    float* gbuf = nullptr;                         // back-propagated gradient (fp32, 128 columns)
-    uint16_t* d = nullptr;                         // hidden delta (bf16, 128 columns)
+    uint16_t* d[2] = {nullptr, nullptr};           // hidden deltas (bf16, 128 columns), in turn
     float* loss = nullptr;                         // sum of squared errors of the last batch
-    float* colpart = nullptr;                      // column sums per chunk of kColsumRows rows
+    float* colpart[4] = {nullptr, nullptr, nullptr, nullptr};  // column sums per kColsumRows rows, of each layer
+    float* wpart = nullptr;                        // weight gradients of each split of the batch, kMlpSplits of every layer
     hipStream_t stream = nullptr;
     int device = 0;
 };
 
-hipError_t gemm(const uint16_t* A, long sam, long sak, const uint16_t* B, long sbk, long sbn, float* C, long ldc, int M,
-                int N, int K, bool accumulate, hipStream_t s);
 hipError_t mlp_refresh_bf16(Mlp& m, hipStream_t s);
 hipError_t mlp_infer(const Mlp& m, const uint16_t* X, float* Y, uint32_t n, hipStream_t s);
 // The learned closure's inputs, for inference that forms each row's layer-1 operand itself, the
@@ -65,7 +63,6 @@ struct ClosureRows {
 };
 hipError_t mlp_infer_closure(const Mlp& m, const ClosureRows& rows, float* Y, uint32_t n, hipStream_t s);
 hipError_t mlp_forward_train(Mlp& m, const uint16_t* X, const float* T, float* Y, uint32_t M, hipStream_t s);
-hipError_t mlp_backward(Mlp& m, const uint16_t* X, uint32_t M, hipStream_t s);
-hipError_t mlp_adam(Mlp& m, float lr, hipStream_t s);
+hipError_t mlp_backward(Mlp& m, const uint16_t* X, uint32_t M, bool adam, float lr, hipStream_t s);
 
 }  // namespace wc
