@@ -682,6 +682,9 @@ __device__ __forceinline__ void form_tables(const Scenes& S, const uint2* __rest
 // ------------------------------------------------------------------------------------------
 // The first particle to arrive in a cell of more than kGatherDirectMax also lists the cell for the
 // leading workgroups of k_gather, which sort its input indices instead of ranking them one by one.
+// TILES: further workgroups form the tile passes' work list (their code costs the others 1.6 us of 7.5 on a
+// million particles, so contexts without those passes run none of it).
+template <bool TILES>
 __global__ __launch_bounds__(kHashBlock) void k_place(Scenes S, const uint32_t* __restrict__ key,
                                                       const uint32_t* __restrict__ rank,
                                                       const uint2* __restrict__ range,
@@ -689,7 +692,7 @@ __global__ __launch_bounds__(kHashBlock) void k_place(Scenes S, const uint32_t* 
                                                       uint32_t* __restrict__ crowd_count, uint32_t crowd_cap,
                                                       uint32_t* __restrict__ error_flag, TileWork tiles) {
     const uint32_t b = blockIdx.x;
-    if (b >= S.blocks256) {  // the tile passes' work list
+    if (TILES && b >= S.blocks256) {
         if ((S.by + 2) * (S.bz + 2) <= 16)
             classify_boxes<16>(S, range, tiles, error_flag, b - S.blocks256);
         else
@@ -864,6 +867,7 @@ __device__ __forceinline__ void gather_crowded_cells(
     }
 }
 
+template <bool TILES>  // as for k_place: further workgroups form the cell tables
 __global__ __launch_bounds__(kHashBlock) void k_gather(Scenes S, uint32_t* __restrict__ slot_tmp,
                                                        const uint32_t* __restrict__ key,
                                                        const uint2* __restrict__ range,
@@ -884,7 +888,7 @@ __global__ __launch_bounds__(kHashBlock) void k_gather(Scenes S, uint32_t* __res
         return;
     }
     // kCrowdBlocks is a multiple of the XCD count, so block b still runs on XCD b mod 8
-    if (blockIdx.x >= kCrowdBlocks + S.blocks256) {  // the listed boxes' tables
+    if (TILES && blockIdx.x >= kCrowdBlocks + S.blocks256) {
         form_tables(S, range, tiles, blockIdx.x - kCrowdBlocks - S.blocks256, gridDim.x - kCrowdBlocks - S.blocks256);
         return;
     }
@@ -2803,7 +2807,7 @@ static TileWork tile_work(const DeviceBuffers& b, const TileShape* t) {
 hipError_t launch_place(const DeviceBuffers& b, const TileShape* tiles, hipStream_t s) {
     if (b.sc.blocks256 == 0) return hipSuccess;
     const unsigned extra = tiles ? b.sc.tblocks : 0u;
-    hipLaunchKernelGGL(k_place, dim3(b.sc.blocks256 + extra), dim3(kHashBlock), 0, s, b.sc, b.key, b.rank, b.range,
+    hipLaunchKernelGGL(tiles ? k_place<true> : k_place<false>, dim3(b.sc.blocks256 + extra), dim3(kHashBlock), 0, s, b.sc, b.key, b.rank, b.range,
                        b.slot_tmp, b.crowd, b.crowd_count, b.crowd_cap, b.error_flag, tile_work(b, tiles));
     return hipGetLastError();
 }
@@ -2812,7 +2816,7 @@ hipError_t launch_gather(const DeviceBuffers& b, const TileShape* tiles, hipStre
     if (b.sc.blocks256 == 0) return hipSuccess;
     static_assert(kCrowdBlocks % kNumXcd == 0, "the leading workgroups keep the XCD mapping of the others");
     const unsigned extra = tiles ? tile_grid(b) : 0u;
-    hipLaunchKernelGGL(k_gather, dim3(b.sc.blocks256 + kCrowdBlocks + extra), dim3(kHashBlock), 0, s, b.sc, b.slot_tmp, b.key,
+    hipLaunchKernelGGL(tiles ? k_gather<true> : k_gather<false>, dim3(b.sc.blocks256 + kCrowdBlocks + extra), dim3(kHashBlock), 0, s, b.sc, b.slot_tmp, b.key,
                        b.range, b.posrho[0], b.velp[0], b.posrho[1], b.velp[1], b.sorted, b.skey, b.ids[0],
                        b.ids[1], b.rho_max + 1, b.crowd, b.crowd_count, b.crowd_cap, tile_work(b, tiles));
     return hipGetLastError();
