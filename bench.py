@@ -357,8 +357,13 @@ def main() -> int:
     dom_s = per_launch_ms[dom] * 1e-3
     achieved = algo[dom] / dom_s / 1e9
 
+    tiles = tuning["density_variant"] == len(tuning["variants"]) - 1  # the tile passes are the last variant
+
+    def kernel_of(k):
+        return f"{k}_tile" if tiles and k in ("density", "update") else k
+
     def measured(kernels):
-        vals = [read_traffic(k) for k in kernels]
+        vals = [read_traffic(kernel_of(k)) for k in kernels]
         return None if any(v is None for v in vals) else sum(vals)
 
     pass_kernels = {"hash": ["hash"], "scan": ["scan"], "scatter": ["place", "gather"], "density": ["density"],
@@ -370,7 +375,7 @@ def main() -> int:
                 for k, v in pass_ms.items() if v > 0}
     print(f"# per-pass GB/s [algorithmic, measured]: {json.dumps(pass_gbs)}", file=sys.stderr, flush=True)
     traffic = measured([dom])
-    valu = read_valu(dom)
+    valu = read_valu(kernel_of(dom))
     valu_frac = None if valu is None else valu / dom_s / VALU_PEAK_WAVE_INSTR_PER_S
     out = {
         "metric": "particle-steps/s at 1M particles: plain vs learned large-dt, \u22641% density err",

@@ -26,7 +26,7 @@ from pathlib import Path
 SIMDS = 256 * 4
 CLOCK_HZ = 2.4e9
 VALU_WAVE_INSTR_PER_S = 256 * CLOCK_HZ
-STEP_KERNELS = ("k_hash", "k_scan", "k_place", "k_gather", "k_density", "k_update")
+STEP_KERNELS = ("k_hash", "k_scan", "k_place", "k_gather", "k_density", "k_update", "k_density_tile", "k_update_tile")
 
 
 def _one(d: Path, pattern: str) -> Path:
