@@ -530,7 +530,7 @@ int create_context(const wc_params* scenes, uint32_t num, wc_ctx** out) {
         // learned step's workspace): else the context keeps the per-particle passes.
         const size_t list_cap = wc::tile_list_cap(n), chunks = wc::tile_list_chunks(n);
         const size_t tables = n / 128 + 1024 < c->tile_entries ? n / 128 + 1024 : c->tile_entries;
-        const size_t bytes[6] = {c->tile_entries * sizeof(uint4), 256, tables * wc::kTileTableBytes, n * 4,
+        const size_t bytes[6] = {c->tile_entries * sizeof(uint4), (wc::kSceneSparse + (size_t)num) * 4, tables * wc::kTileTableBytes, n * 4,
                                  chunks * 64 * list_cap * sizeof(uint16_t), chunks * 64 * sizeof(uint16_t)};
         void** const ptr[6] = {(void**)&b.tiles,  (void**)&b.tile_count, &b.tables,
                                (void**)&b.sparse, (void**)&b.llist,      (void**)&b.lcount};
@@ -548,7 +548,8 @@ int create_context(const wc_params* scenes, uint32_t num, wc_ctx** out) {
             b.table_cap = (uint32_t)tables;
             b.list_cap = (uint32_t)list_cap;
             b.list_chunks = (uint32_t)chunks;
-            if (n >= wc::kTileMinParticles) c->density_variant = c->update_variant = wc::tile_variant();
+            if (n >= wc::kTileMinParticles && n / num >= wc::kTileMinPerScene)
+                c->density_variant = c->update_variant = wc::tile_variant();
         } else {
             c->tile_mem = nullptr;
             (void)hipGetLastError();
@@ -566,7 +567,7 @@ int create_context(const wc_params* scenes, uint32_t num, wc_ctx** out) {
     zero(b.step_start, 64);
     zero(b.rho_max, 64);
     zero(b.crowd_count, 64);
-    if (c->tile_ok) zero(b.tile_count, 256);
+    if (c->tile_ok) zero(b.tile_count, (wc::kSceneSparse + (size_t)num) * 4);
     // rho_max[1] = 2: no density pass has checked the force pass's division operands yet
     if (e == hipSuccess) e = hipMemsetAsync(reinterpret_cast<char*>(b.rho_max) + 4, 2, 1, c->stream);
     zero(b.sorted, n * 4);

@@ -181,7 +181,9 @@ int tile_variant();
 // What the sort forms for them.
 struct TileWork {
     uint4* tiles;     // work list
-    uint32_t* count;  // its entries; [1]: slots in `sparse`; [kListCount]: list chunks
+    // its entries; [1]: slots in `sparse` of a single scene; [kListCount]: list chunks; with several scenes,
+    // [kSceneSparse + s]: scene s's slots in `sparse` (from its first particle on), [kSceneSparse - 1]: entries of those
+    uint32_t* count;
     uint32_t cap;
     uint32_t rec_cap;  // records a box may stage
     uint32_t chunk;    // particles of an entry that searches directly
@@ -191,6 +193,7 @@ struct TileWork {
     uint32_t sparse_max;  // the most records of such a box and its halo
 };
 constexpr uint32_t kListCount = 32;          // in another 128-byte line: atomics on one line serialise
+constexpr uint32_t kSceneSparse = 64;
 constexpr uint32_t kTileBlock = 256;         // threads, and at most that many boxes, per classification workgroup
 // Neighbours a particle's list holds (16 bits each; particles with more search directly): dense clusters
 // have a few hundred; large contexts keep lists of half the size.
@@ -198,8 +201,9 @@ inline uint32_t tile_list_cap(uint64_t particles) { return particles <= 500000 ?
 // Contexts of this many particles start with the tile passes.  Smaller ones gain while the fluid is at rest
 // density (16,384 particles, three contexts at once: 20 us a step against 33) and lose as it spreads and boxes
 // empty (44 against 36 at step 4,000); 80,000 particles gain in both (83 against 131, 84 against 122).
-// wc_tune times both whatever the size.
-constexpr uint32_t kTileMinParticles = 50000;
+// Batches also need 20,000 particles a scene: 62 scenes of about 31,000 780 -> 693, 28 of about 14,000 207 -> 215
+// once spread.  wc_tune times both whatever the size.
+constexpr uint32_t kTileMinParticles = 50000, kTileMinPerScene = 20000;
 // Chunks of 64 lanes that lists are kept for.  Full boxes use 1.2 lanes a particle (columns are rounded to four
 // lanes, boxes to 64), a fluid that has spread up to 1.4; boxes past the memory search directly.
 inline uint64_t tile_list_chunks(uint64_t particles) { return particles / 32 + 1024; }

@@ -118,9 +118,10 @@ __global__ __launch_bounds__(kHashBlock) void k_hash(Scenes S, const float4* __r
     const uint32_t g = blockIdx.x * kHashBlock + threadIdx.x;
     if (g < S.total_tiles) scan_status[g] = 0ull;
     if (g < S.num_scenes) scene_done[g] = 0ull;
+    if (tile_count && S.num_scenes > 1 && g < S.num_scenes) tile_count[kSceneSparse + g] = 0u;
     if (g == 0) {
         *crowd_count = 0u;
-        if (tile_count) tile_count[0] = tile_count[1] = tile_count[kListCount] = 0u;
+        if (tile_count) tile_count[0] = tile_count[1] = tile_count[kListCount] = tile_count[kSceneSparse - 1] = 0u;
         *step_start = wall_clock64();
         rho_max[0] = 0u;
         rho_max[1] = kDivPending;  // the force pass's operands are unchecked until a density pass runs
@@ -463,32 +464,24 @@ __device__ __forceinline__ void classify_boxes(const Scenes& S, const uint2* __r
         sparse += s_wave[w].y;
         list_chunks += s_wave[w].z;
     }
-    // several scenes: entries of their own (one scene's sparse particles need none, tile_item)
-    const uint32_t chunks = S.num_scenes == 1 ? 0u : (sparse + T.chunk - 1) / T.chunk;
     if (threadIdx.x == 0) {
-        const unsigned long long add = (unsigned long long)sparse << 32 | (listed + chunks);
+        // the scene's sparse slots start at its first particle's place
+        const bool one = S.num_scenes == 1;
+        const unsigned long long add = (unsigned long long)(one ? sparse : 0u) << 32 | listed;
         const unsigned long long old = add ? atomicAdd(reinterpret_cast<unsigned long long*>(T.count), add) : 0ull;
         s_base.x = (uint32_t)old;
-        s_base.y = (uint32_t)(old >> 32);
+        s_base.y = one ? (uint32_t)(old >> 32) : (sparse ? d.p_off + atomicAdd(T.count + kSceneSparse + s, sparse) : 0u);
     }
     if (threadIdx.x == 64) s_base.z = list_chunks ? atomicAdd(T.count + kListCount, list_chunks) : 0u;
     if (threadIdx.x < S.tper) s_rec[threadIdx.x] = make_uint2(few ? 0x80000000u | sparse_before : rec.x, rec.y);
     __syncthreads();
-    if (fits || threadIdx.x < chunks) {
-        // chunks <= S.tper: a box adds at most sparse_max <= T.chunk particles
-        if (s_base.x + listed + chunks > T.cap) {
+    if (fits) {
+        const uint32_t at = s_base.x + before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+        origin(first + threadIdx.x, x, y, z);
+        if (at < T.cap)
+            T.tiles[at] = box_entry(x, y, z, min(bx, R - x), min(by, R - y), min(bz, R - z), s, s_base.z + chunk);
+        else
             atomicOr(error_flag, 2u);
-        } else {
-            if (fits) {
-                origin(first + threadIdx.x, x, y, z);
-                T.tiles[s_base.x + chunks + before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] =
-                    box_entry(x, y, z, min(bx, R - x), min(by, R - y), min(bz, R - z), s, s_base.z + chunk);
-            }
-            if (threadIdx.x < chunks)
-                T.tiles[s_base.x + threadIdx.x] =
-                    make_uint4(0u, kEntryDirect | kEntrySparse | min(T.chunk, sparse - threadIdx.x * T.chunk) << 13, s,
-                               s_base.y + threadIdx.x * T.chunk);
-        }
     }
     if (sparse != 0u) {
         // a few lanes a box: lane `row` lists the particles of one row
@@ -665,6 +658,17 @@ __device__ __forceinline__ void form_tables(const Scenes& S, const uint2* __rest
                                             uint32_t block, uint32_t nblocks) {
     __shared__ BoxShared sh;
     const uint32_t listed = min(min(*T.count, T.cap), T.table_cap);
+    if (block == 0 && S.num_scenes > 1) {
+        // several scenes' sparse particles: entries of a scene each, from the work list's end down
+        for (uint32_t s = threadIdx.x; s < S.num_scenes; s += kHashBlock) {
+            const SceneDesc& d = S.desc[s];
+            const uint32_t n = min(T.count[kSceneSparse + s], d.c.n), chunks = (n + T.chunk - 1) / T.chunk;
+            const uint32_t at = chunks ? atomicAdd(T.count + kSceneSparse - 1, chunks) : 0u;
+            for (uint32_t k = 0; k < chunks && at + k < T.cap; ++k)
+                T.tiles[T.cap - 1u - at - k] = make_uint4(0u, kEntryDirect | kEntrySparse | min(T.chunk, n - k * T.chunk) << 13,
+                                                          s, d.p_off + k * T.chunk);
+        }
+    }
     for (uint32_t item = block; item < listed; item += nblocks) {
         const uint4 e = T.tiles[item];
         if (e.y & kEntryDirect) continue;
@@ -1499,17 +1503,20 @@ __device__ __forceinline__ void box_open(BoxShared& sh, const Box& b, const Scen
     }
 }
 
-// The work of a pass: a single scene's sparse particles in chunks of BLOCK first, dealt round to the XCDs, then the
-// listed boxes, neighbours on one XCD.
+// The work of a pass: the sparse particles in chunks of BLOCK first (a single scene's without entries of their own),
+// dealt round to the XCDs, then the listed boxes, neighbours on one XCD.
 struct TileItems {
-    uint32_t boxes, sparse, lead, all;  // lead: items of the chunks, a multiple of kNumXcd
+    uint32_t boxes, sparse, chunks, lead, all;  // lead: items of the chunks, a multiple of kNumXcd
+    uint32_t cap;
 };
 template <int BLOCK>
 __device__ __forceinline__ TileItems tile_items(const Scenes& S, const uint32_t* __restrict__ count, uint32_t cap) {
     TileItems t;
     t.boxes = min(count[0], cap);
     t.sparse = S.num_scenes == 1 ? min(count[1], S.total_particles) : 0u;
-    t.lead = ((t.sparse + BLOCK - 1) / BLOCK + kNumXcd - 1) / kNumXcd * kNumXcd;
+    t.chunks = S.num_scenes == 1 ? (t.sparse + BLOCK - 1) / BLOCK : min(count[kSceneSparse - 1], cap - t.boxes);
+    t.cap = cap;
+    t.lead = (t.chunks + kNumXcd - 1) / kNumXcd * kNumXcd;
     t.all = t.lead + t.boxes;
     return t;
 }
@@ -1518,7 +1525,9 @@ __device__ __forceinline__ uint4 tile_item(const TileItems& t, const uint4* __re
                                            uint32_t& at_list) {
     at_list = 0u;
     if (item < t.lead) {
-        const uint32_t first = min(item * BLOCK, t.sparse);
+        if (item >= t.chunks) return make_uint4(0u, kEntryDirect, 0u, 0u);  // none
+        if (t.sparse == 0u) return tiles[t.cap - 1u - item];
+        const uint32_t first = item * BLOCK;
         return make_uint4(0u, kEntryDirect | kEntrySparse | min((uint32_t)BLOCK, t.sparse - first) << 13, 0u, first);
     }
     at_list = item - t.lead;
