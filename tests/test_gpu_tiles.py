@@ -25,13 +25,13 @@ def _clustered(oracle_params, parts, cells, seed):
 
 
 def _case(name):
-    if name == "4x2x2, 12 a cell":  # sides that no box divides
+    if name == "2x2x4, 12 a cell":  # sides that no box divides
         return scaled_block((23, 17, 19), 0.027, 1, 2.3)
     if name == "2x2x2, 51 a cell":  # more neighbours than the context's lists hold
         return scaled_block((23, 17, 19), 0.027, 1, 3.5)
-    if name == "4x4x2":
-        return scaled_block((47, 43, 47), 0.017, 2)
-    if name == "4x4x3":
+    if name == "4x2x4, 12 a cell":
+        return scaled_block((75, 73, 75), 0.01, 2, 2.3)
+    if name == "4x3x4":
         return scaled_block((53, 57, 59), 0.0151, 3)
     if name == "one cell":  # a grid that is a single box
         p, parts = scaled_block((4, 5, 4), 0.2, 4)
@@ -55,8 +55,8 @@ def _case(name):
     return p, parts
 
 
-CASES = ["4x2x2, 12 a cell", "2x2x2, 51 a cell", "4x4x2", "4x4x3", "one cell", "small, split", "small, long", "small, direct",
-         "small, split, odd positions", "4x4x3, split", "4x4x3, direct"]
+CASES = ["2x2x4, 12 a cell", "2x2x2, 51 a cell", "4x2x4, 12 a cell", "4x3x4", "one cell", "small, split", "small, long", "small, direct",
+         "small, split, odd positions", "4x3x4, split", "4x3x4, direct"]
 
 
 @pytest.mark.parametrize("case", CASES)

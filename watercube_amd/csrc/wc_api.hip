@@ -184,12 +184,12 @@ int check_params(const wc_params* p) {
 
 constexpr uint64_t kTileMaxCellsPerParticle = 64;
 
-// Base box of the tile passes.  Larger boxes stage less halo per particle; they have to fit LDS at rest
-// density (a denser one is split) and leave the chip's 256 CUs some boxes each: the largest shape of which
-// the particles fill 350.  At 8 particles a cell the whole step took, by 4x3x4 / 4x2x4 / 2x2x4 (us):
-// 16,384 particles 75 / 71 / 70, 91,125 118 / 108 / 112, 125,000 125 / 117 / 133, 262,144 152 / 164 / 187;
-// at 12 a cell 4x2x4 / 2x2x4: 125,000 155 / 149, 2,048,000 1,144 / 1,175.  Below that 2x2x4 unless a box
-// has more particles than threads: the 80,000-particle scene (20 a cell) 225 by 2x2x4, 181 by 2x2x2.
+// Base box of the tile passes.  Larger boxes stage less halo per particle; they have to fit LDS at rest density (a
+// denser one is split) and leave the chip's 256 CUs enough boxes each.  At 8 particles a cell the whole step took, by
+// 4x3x4 / 4x2x4 / 2x2x4 (us): 91,125 particles 141 / 130 / 104, 125,000 126 / 137 / 137, 262,144 141 / 158 / 176: the
+// first from 300 boxes of it.  At 12 a cell, where it does not fit, by 4x2x4 / 2x2x4: 125,000 182 / 135, 192,089 (once
+// spread, three at once) 94 / 111, 2,048,000 1,087 / 1,109: the second from 450 boxes.  Below that 2x2x4 unless a box has more particles than threads: the
+// 80,000-particle scene (20 a cell) 228 by 2x2x4, 190 by 2x2x2.
 wc::TileShape choose_tile_shape(const std::vector<wc_params>& scenes) {
     double n = 0.0, cell = 0.0;  // particles; those a cell holds at rest density
     for (const wc_params& p : scenes) {
@@ -198,10 +198,14 @@ wc::TileShape choose_tile_shape(const std::vector<wc_params>& scenes) {
         if (rest > 0.0 && rest < 1e6) cell += rest * p.num_particles;
     }
     cell = n > 0.0 ? cell / n : 0.0;
-    for (const wc::TileShape& t : {wc::TileShape{4, 3, 4, wc::kTileLargeBlock, wc::kTileLargeCap},
-                                   wc::TileShape{4, 2, 4, wc::kTileLargeBlock, wc::kTileLargeCap},
-                                   wc::TileShape{2, 2, 4, wc::kTileSmallBlock, wc::kTileSmallCap}})
-        if ((t.x + 2) * (t.y + 2) * (t.z + 2) * cell * 1.05 <= t.cap && n >= 350.0 * (t.x * t.y * t.z) * cell) return t;
+    const struct {
+        wc::TileShape t;
+        double boxes;
+    } shapes[] = {{{4, 3, 4, wc::kTileLargeBlock, wc::kTileLargeCap}, 300.0},
+                  {{4, 2, 4, wc::kTileLargeBlock, wc::kTileLargeCap}, 450.0},
+                  {{2, 2, 4, wc::kTileSmallBlock, wc::kTileSmallCap}, 350.0}};
+    for (const auto& [t, boxes] : shapes)
+        if ((t.x + 2) * (t.y + 2) * (t.z + 2) * cell * 1.05 <= t.cap && n >= boxes * (t.x * t.y * t.z) * cell) return t;
     return {2, 2, 16.0 * cell <= wc::kTileSmallBlock ? 4 : 2, wc::kTileSmallBlock, wc::kTileSmallCap};
 }
 
