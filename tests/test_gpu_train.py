@@ -50,3 +50,43 @@ def test_gradient_and_step(rows):
     net.predict(xd, yb, rows)
     a, b = ya.download()[:, :3], yb.download()[:, :3]
     assert np.linalg.norm(a - b) < 2e-2 * np.linalg.norm(b)
+
+
+def test_several_steps_follow_their_gradients():
+    """Six steps over 2,200 rows (nine partial sums a weight gradient): each step's parameters are, bit for bit,
+    Adam's float32 update (seven operations, none contracted) by the gradient of the parameters before it, and that
+    gradient is within 3e-2 of the oracle's per tensor, as in test_gradient_and_step.  Trajectories themselves are
+    not compared: adding the partial sums in another order changes gradients by float32 roundings, now and then a
+    bf16 weight rounds the other way, and parameters then part by up to about 1e-4 in a few steps."""
+    import ctypes
+
+    powf = ctypes.CDLL("libm.so.6").powf
+    powf.restype, powf.argtypes = ctypes.c_float, [ctypes.c_float, ctypes.c_float]
+    f = np.float32
+    rows, lr, b1, b2, eps = 2200, f(1e-3), f(0.9), f(0.999), f(1e-8)
+    rng = np.random.default_rng(3)
+    net = ClosureNet(max_batch=rows, seed=8)
+    p = net.params()
+    m, v = np.zeros_like(p), np.zeros_like(p)
+    Lo = MO.layout()
+    for t in range(1, 7):
+        print(f"case step {t}", flush=True)
+        x = np.zeros((rows, 208), np.float32)
+        x[:, :195] = rng.normal(0, 1, (rows, 195))
+        xb = (x.view(np.uint32) >> 16).astype(np.uint16)
+        y = np.zeros((rows, 4), np.float32)
+        y[:, :3] = rng.normal(0, 1, (rows, 3))
+        xd, yd = DeviceArray(xb.shape, np.uint16).upload(xb), DeviceArray(y.shape, np.float32).upload(y)
+        g, _ = net.gradient(xd, yd, rows)
+        _, _, ref = MO.forward_backward(p.astype(np.float64), MO.bf16_bits_to_f64(xb), y[:, :3], bf16=True)
+        for k in ("w1", "b1", "w2", "b2", "w3", "b3", "w4", "b4"):
+            a, b = (q[Lo[k][0]:Lo[k][0] + Lo[k][1]] for q in (g, ref))
+            assert np.linalg.norm(a - b) < 3e-2 * np.linalg.norm(b), (t, k)
+        net.train_step(xd.ptr, yd.ptr, rows, float(lr))
+        m = b1 * m + (f(1) - b1) * g
+        v = b2 * v + (f(1) - b2) * g * g
+        c1, c2 = f(1) - f(powf(b1, t)), f(1) - f(powf(b2, t))
+        p = p - lr * (m / c1) / (np.sqrt(v / c2) + eps)
+        got = net.params()
+        assert p.dtype == np.float32
+        assert np.array_equal(got.view(np.uint32), p.view(np.uint32)), f"step {t}: {(got != p).sum()} parameters"
