@@ -123,3 +123,29 @@ def test_tile_passes_of_several_scenes_with_thin_boxes(oracle):
             got = b.scene_particles(s)
             for k in ("density", "pressure", "velocity", "position"):
                 assert np.array_equal(got[k].view(np.uint32), st.buf1[k].view(np.uint32)), f"scene {s}: {k}"
+
+
+def test_latency_of_an_empty_scene_is_zero(oracle):
+    """The passes' leading work items are padded to a multiple of the XCD count.  Padding belongs to no scene: a scene
+    without particles, the first one here, keeps a latency of 0."""
+    import ctypes as C
+
+    from watercube_amd.batch import SceneBatch
+
+    scenes = []
+    for k, n in enumerate((0, 700, 257)):
+        p, _ = scaled_block((20, 20, 20), 0.03, 5)
+        parts = np.zeros(n, L.PARTICLE_DTYPE)
+        parts["position"] = np.random.default_rng(k).uniform(0.01, 0.99, (n, 3)).astype(np.float32)
+        p.num_particles = n
+        scenes.append((p, parts, 1e-4, "test"))
+    tile = L.lib().wc_num_variants() - 1
+    for variant in (2, tile):
+        print(f"case empty scene, variant {variant}", flush=True)
+        with SceneBatch(scenes) as b:
+            t = L.wc_tuning(variant, variant, 0)
+            L.check(L.lib().wc_set_tuning(b.ctx, C.byref(t)), "wc_set_tuning")
+            b.step(3)
+            b.synchronize()
+            lat = b.latency_ms()
+        assert lat[0] == 0.0 and (np.asarray(lat[1:]) > 0.0).all(), f"variant {variant}: {lat}"

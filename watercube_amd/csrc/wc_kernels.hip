@@ -1525,7 +1525,7 @@ __device__ __forceinline__ uint4 tile_item(const TileItems& t, const uint4* __re
                                            uint32_t& at_list) {
     at_list = 0u;
     if (item < t.lead) {
-        if (item >= t.chunks) return make_uint4(0u, kEntryDirect, 0u, 0u);  // none
+        if (item >= t.chunks) return make_uint4(0u, kEntryDirect, 0u, 0u);  // an entry of no particles
         if (t.sparse == 0u) return tiles[t.cap - 1u - item];
         const uint32_t first = item * BLOCK;
         return make_uint4(0u, kEntryDirect | kEntrySparse | min((uint32_t)BLOCK, t.sparse - first) << 13, 0u, first);
@@ -1728,6 +1728,7 @@ __global__ __launch_bounds__(BLOCK, WPE) void k_density_tile(Scenes S, const uin
     for (uint32_t item = blockIdx.x; item < items.all; item += gridDim.x) {
         uint32_t at_list;
         const uint4 e = tile_item<BLOCK>(items, tiles, item, at_list);
+        if (e.y == kEntryDirect) continue;  // no particles, and no scene's
         const SceneDesc& d = S.desc[e.z];
         const StepConsts c = d.c;
         uint32_t top = 0;  // largest density of the lane's particles, as bits (NaN ranks highest)
@@ -1950,6 +1951,7 @@ __global__ __launch_bounds__(BLOCK, WPE) void k_update_tile(Scenes S, const uint
     for (uint32_t item = blockIdx.x; item < items.all; item += gridDim.x) {
         uint32_t at_list;
         const uint4 e = tile_item<BLOCK>(items, tiles, item, at_list);
+        if (e.y == kEntryDirect) continue;  // no particles, and no scene's
         const SceneDesc& d = S.desc[e.z];
         const StepConsts c = d.c;
         auto finish = [&](uint32_t t, const float4& p, const float4& pv, const ForceSums& f) {
