@@ -149,3 +149,35 @@ def test_latency_of_an_empty_scene_is_zero(oracle):
             b.synchronize()
             lat = b.latency_ms()
         assert lat[0] == 0.0 and (np.asarray(lat[1:]) > 0.0).all(), f"variant {variant}: {lat}"
+
+
+def test_cube_size_unrelated_to_the_grid(oracle):
+    """wc_create takes `size` and `bin_size` as they are.  On a grid a thousand times wider than `size` every neighbour is
+    kept: candidates are marked with a margin that has to cover the rounding of coordinates up to the grid's width.
+    A neighbour lost at the cutoff hardly shows in the sums, so the lists' lengths are compared too, with those of the
+    per-particle pass."""
+    n = 40_000
+    p, _ = scaled_block((40, 40, 40), 0.02, 6)
+    h = 1.0 / 16
+    p.num_particles, p.grid_res, p.size, p.bin_size, p.kernel_radius, p.particle_mass = n, 16, 1e-3, h, h, 1000.0 / n
+    p.poly6_const, p.spiky_const, p.visc_const = 315 / (64 * np.pi * h ** 9), -45 / (np.pi * h ** 6), 45 / (np.pi * h ** 6)
+    parts = np.zeros(n, L.PARTICLE_DTYPE)
+    parts["position"] = np.random.default_rng(11).uniform(0.01, 0.99, (n, 3)).astype(np.float32)
+    tile = L.lib().wc_num_variants() - 1
+    st = oracle.OracleState(p, parts)
+    st.step(2e-6, 1)
+    counts = []
+    for v in (tile, 2):
+        print(f"case wide grid, variant {v}", flush=True)
+        with Fluid(p, parts) as f:
+            f.set_tuning(v, v, 1)
+            f.sort_.run()
+            f.runDensityProg()
+            counts.append(f.neighbour_counts())
+            f.runUpdateProg(2e-6)
+            f.synchronize()
+            got = f.particles(1)
+        for k in ("density", "pressure", "velocity", "position"):
+            bad = got[k].view(np.uint32) != st.buf1[k].view(np.uint32)
+            assert not bad.any(), f"variant {v}: {k} differs at {int(bad.sum())} places"
+    assert np.array_equal(counts[0], counts[1]), f"{int((counts[0] != counts[1]).sum())} lists differ"

@@ -1619,10 +1619,12 @@ __device__ __forceinline__ BoxLane box_lane(const BoxShared& sh, const Box& b, u
 // column of cells along z, so their candidates in a neighbouring column lie in one window of three or
 // four cells (more where cells hold fewer than four).
 //
-// Rounding: |a'_k| and |b_k - o_k| are at most 3 bins and |b_k| at most the cube's size (boxes with
-// other particles search directly), so no partial sum exceeds 20 bin size and the eight roundings err
-// by less than 8 * 2^-24 * 20 bin size < 1e-5 bin size: margin = 1.2e-5 bin size makes the marked
-// candidates a superset of the accepted ones; the drain applies the exact test.
+// Rounding, in units of bin^2: |a'_k| and |b_k - o_k| are at most 3 (boxes with a particle further out search directly), o
+// lies in the grid of R cells a side, so |b_k| <= R + 3, whatever the cube's `size` is.  n_a and n_b are at most 27,
+// 2 sum a'_k o_k and the three products 18 R and 18 (R + 3), and a cutoff over 108 accepts every pair.  So no partial sum
+// exceeds 18 R + 220, and with the inputs' own rounding the sum errs by less than 2^-24 (144 R + 2,010) < 1.2e-5 (R + 10):
+// with that margin the marked candidates are a superset of the accepted ones (measured: 0.2 of it at most), and the drain
+// applies the exact test.
 //
 // A lane appends its marked candidates to its list in enumeration order: cells in NEIGHBORHOOD order,
 // candidates in slot order.
@@ -1820,7 +1822,7 @@ __global__ __launch_bounds__(BLOCK, WPE) void k_density_tile(Scenes S, const uin
                 continue;
             }
             const uint32_t lanes = sh.own[kMaxBox * kMaxBox];
-            const float cut = c.cut2 + 1.2e-5f * (c.bin * c.size);
+            const float cut = c.cut2 + 1.2e-5f * c.bin * (c.bin * (float)(c.R + 10));
             const bool room = e.w + (lanes + 63u) / 64u <= list_chunks, listable = room && !irregular;
             bool overflowed = false;
             for (uint32_t ch = (uint32_t)wave; ch * 64u < lanes; ch += BLOCK / 64) {
