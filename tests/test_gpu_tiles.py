@@ -181,3 +181,32 @@ def test_cube_size_unrelated_to_the_grid(oracle):
             bad = got[k].view(np.uint32) != st.buf1[k].view(np.uint32)
             assert not bad.any(), f"variant {v}: {k} differs at {int(bad.sum())} places"
     assert np.array_equal(counts[0], counts[1]), f"{int((counts[0] != counts[1]).sum())} lists differ"
+
+
+def test_mass_whose_half_is_not_exact(oracle):
+    """The force pass by tiles moves a half from the pair pressure into the mass, which is exact for normal floats
+    only.  A mass of three units of the smallest float, with kernel constants that bring densities into the shared
+    arithmetic's range: the oracle's bits."""
+    p, parts = scaled_block((20, 20, 20), 0.015, 5)
+    parts["position"] *= np.float32(100.0)
+    parts["velocity"] = np.random.default_rng(4).normal(0, 0.1, parts["velocity"].shape).astype(np.float32)
+    p.size, p.kernel_radius = 100.0, 3.0
+    L.derive(p)
+    p.particle_mass = 3 * 2.0 ** -149
+    p.poly6_const, p.spiky_const, p.visc_const = 1e34, -1e37, 1e36
+    p.rest_density, p.stiffness = 1e-8, 1.0
+    tile = L.lib().wc_num_variants() - 1
+    st = oracle.OracleState(p, parts)
+    st.step(2e-6, 1)
+    assert 2.0 ** -40 < st.buf1["density"].min() and st.buf1["density"].max() < 1.0  # in the range
+    print("case subnormal mass", flush=True)
+    with Fluid(p, parts) as f:
+        for v in (2, tile):
+            f.upload(parts)
+            f.set_tuning(v, v, 0)
+            f.step(2e-6, 1)
+            f.synchronize()
+            got = f.particles(1)
+            for k in ("density", "pressure", "velocity", "position"):
+                bad = got[k].view(np.uint32) != st.buf1[k].view(np.uint32)
+                assert not bad.any(), f"variant {v}: {k} differs at {int(bad.sum())} places"

@@ -184,6 +184,16 @@ int check_params(const wc_params* p) {
 
 constexpr uint64_t kTileMaxCellsPerParticle = 64;
 
+// Constants for which the tile passes' short force arithmetic has the reference's bits.  It halves the mass instead of
+// the pair pressure: exact for normal floats.  And a lane past its list adds its own record, every term of which has to
+// be 0 and not 0 times infinity: m p / rho stays finite up to m = 2^40 (p and rho lie in [2^-40, 2^40]), the kernel
+// terms while these are finite.
+bool short_arithmetic(const wc_params& p) {
+    const float m = fabsf(p.particle_mass);
+    return (m == 0.0f || (m >= 0x1p-100f && m <= 0x1p40f)) && p.kernel_radius <= 0x1p60f &&
+           isfinite(p.spiky_const) && isfinite(p.visc_const * p.kernel_radius);
+}
+
 // Base box of the tile passes.  Larger boxes stage less halo per particle; they have to fit LDS at rest density (a
 // denser one is split) and leave the chip's 256 CUs enough boxes each.  At 8 particles a cell the whole step took, by
 // 4x3x4 / 4x2x4 / 2x2x4 (us): 91,125 particles 141 / 130 / 104, 125,000 126 / 137 / 137, 262,144 141 / 158 / 176: the
@@ -234,6 +244,7 @@ int layout_scenes(wc_ctx* c, uint64_t max_entries) {
     uint32_t* tiles = blk256 + (S + 1);
     uint32_t* tblk = tiles + (S + 1);
     uint64_t p_off = 0, c_off = 0, boxes = 0, cells = 0;
+    bool exact = true;
     c->tile_shape = choose_tile_shape(c->params);
     const wc::TileShape shape = c->tile_shape;
     c->tile_per = tiles_per_block(c->params, shape);
@@ -255,6 +266,7 @@ int layout_scenes(wc_ctx* c, uint64_t max_entries) {
         tblk[s + 1] = tblk[s] + ceil_div(d.ntiles, c->tile_per);
         boxes += d.ntiles;
         cells += d.c.ncells;
+        exact = exact && (d.c.n == 0 || short_arithmetic(p));
         p_off += d.c.n;
         c_off += (uint64_t)nt * wc::kScanTile;
         if (p_off > 0xFFFFFF00ull || c_off > 0xFFFFFF00ull)
@@ -265,7 +277,7 @@ int layout_scenes(wc_ctx* c, uint64_t max_entries) {
     // The tile passes look at every base box: on a grid with far more cells than particles that costs
     // more than they gain.
     const uint64_t entries = wc::tile_capacity(boxes, p_off);
-    c->tile_ok = p_off > 0 && cells <= kTileMaxCellsPerParticle * p_off && entries <= max_entries;
+    c->tile_ok = exact && p_off > 0 && cells <= kTileMaxCellsPerParticle * p_off && entries <= max_entries;
     c->tile_entries = c->tile_ok ? (uint32_t)entries : 0u;
     c->scene_tab.clear();
     if (S > 1) {
