@@ -210,3 +210,40 @@ def test_mass_whose_half_is_not_exact(oracle):
             for k in ("density", "pressure", "velocity", "position"):
                 bad = got[k].view(np.uint32) != st.buf1[k].view(np.uint32)
                 assert not bad.any(), f"variant {v}: {k} differs at {int(bad.sum())} places"
+
+
+@pytest.mark.parametrize("sequence", ["step", "step, lists off, step", "step, sort", "step, other passes",
+                                      "profiled", "learned run"])
+def test_neighbour_counts_are_those_of_the_last_listing_pass(sequence):
+    """wc_get_neighbour_counts answers for the last density pass that ran in list mode, whatever ran after it: by tiles,
+    whose steps leave the lists out until they are asked for, as by the per-particle passes."""
+    import ctypes as C
+
+    from watercube_amd.scenes import workload
+
+    p, parts, dt, _ = workload("dam_break_16k")
+    tile = L.lib().wc_num_variants() - 1
+    steps = 20 + len(sequence)  # freed memory holds no other sequence's counts
+    out = []
+    for v in (tile, 2):
+        print(f"case {sequence}, variant {v}", flush=True)
+        with Fluid(p, parts) as f:
+            f.set_tuning(v, v, 1)
+            if sequence == "profiled":
+                f.profile(dt, steps)
+            elif sequence == "learned run":
+                st = L.wc_closure_stats()
+                L.check(L.lib().wc_closure_run(f.ctx, None, C.c_float(dt), 4, steps, C.c_float(1e30), C.byref(st)), "run")
+            else:
+                f.step(dt, steps)
+            if sequence == "step, lists off, step":
+                f.set_tuning(v, v, 0)
+                f.step(dt, steps)
+            elif sequence == "step, sort":
+                f.sort_.run()
+            elif sequence == "step, other passes":
+                f.set_tuning(2, 2, 0)
+                f.sort_.run()
+                f.runDensityProg()
+            out.append(f.neighbour_counts())
+    assert np.array_equal(out[0], out[1])

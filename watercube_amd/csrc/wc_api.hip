@@ -152,6 +152,9 @@ struct wc_ctx {
     bool tiles_ok = false;   // ... and the work list is that sort's
     bool llist_ok = false;   // the tiles' lists and counts are those of a density pass on that sort
     bool nlist_ok = false;   // nlist and ncount likewise
+    // The last density pass in list mode ran by tiles and left nlist and ncount out; refresh_lists() forms them before
+    // anything reads them or takes away what they are formed from (the sort, the work list, list mode itself).
+    bool lists_owed = false;
     double clock_khz = 100000.0;  // wall_clock64 rate
     // learned-closure workspace (allocated on first use)
     uint16_t* cl_x = nullptr;       // features, n x 208 bf16
@@ -401,12 +404,13 @@ int particle_variant(int v) { return v == wc::tile_variant() ? 2 : v; }
 void note_sort(wc_ctx* c, bool tiles) {
     c->sorted_ok = true;
     c->tiles_ok = tiles;
-    c->llist_ok = c->nlist_ok = false;
+    c->llist_ok = c->nlist_ok = c->lists_owed = false;
 }
 void note_step(wc_ctx* c) {
     note_sort(c, density_by_tiles(c));
     c->llist_ok = density_by_tiles(c);
     c->nlist_ok = c->neighbour_list && !update_by_tiles(c);
+    c->lists_owed = c->neighbour_list && update_by_tiles(c);
 }
 
 // The kernels of a sort, in order, each followed by after(k) (k-th of the passes wc_pass_name names).
@@ -437,10 +441,12 @@ hipError_t launch_density_pass(wc_ctx* c, bool lists) {
         const hipError_t e = wc::launch_density_tile(c->b, c->tile_shape, write, c->stream);
         c->llist_ok = true;
         c->nlist_ok = write;
+        c->lists_owed = c->neighbour_list && !write;
         return e;
     }
     c->llist_ok = false;
     c->nlist_ok = c->neighbour_list;
+    c->lists_owed = false;
     return wc::launch_density(c->b, particle_variant(c->density_variant), c->neighbour_list, c->stream);
 }
 
@@ -449,11 +455,12 @@ hipError_t launch_update_pass(wc_ctx* c) {
     return wc::launch_update(c->b, particle_variant(c->update_variant), c->neighbour_list && c->nlist_ok, c->stream);
 }
 
-// nlist and ncount of the last density pass, for readers in list mode: a density pass by tiles that
-// left them out runs again and writes them (and the same densities).  After an upload the counts are
-// marked overflowed and every reader searches.
-hipError_t refresh_lists(wc_ctx* c) {
-    if (!c->llist_ok || c->nlist_ok || !c->b.nlist || !c->b.ncount) return hipSuccess;
+// nlist and ncount of the last density pass in list mode, if it left them out: the pass runs again on the same sort and
+// writes them (and the same densities).  `current`: for a reader in list mode that takes them for the current sort's, also
+// when that pass ran before list mode was switched on.
+hipError_t refresh_lists(wc_ctx* c, bool current) {
+    if (!c->lists_owed && !(current && c->neighbour_list && c->llist_ok && !c->nlist_ok)) return hipSuccess;
+    c->lists_owed = false;
     c->nlist_ok = true;
     return wc::launch_density_tile(c->b, c->tile_shape, true, c->stream);
 }
@@ -686,7 +693,7 @@ int copy_records_in(wc_ctx* c, uint32_t first, const wc_particle* host, uint32_t
         WC_HIP(wc::launch_split_records(c->staging + first, c->b.posrho[b] + first, c->b.velp[b] + first, n,
                                         c->stream));
     // buffer 2 changed under the last sort: its cell keys, neighbour lists and division check
-    c->sorted_ok = c->tiles_ok = c->llist_ok = c->nlist_ok = false;
+    c->sorted_ok = c->tiles_ok = c->llist_ok = c->nlist_ok = c->lists_owed = false;
     WC_HIP(wc::launch_invalidate(c->b, c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
     return WC_OK;
@@ -917,7 +924,7 @@ WC_API int wc_set_params(wc_ctx* c, const wc_params* p) {
     rc = upload_tables(c);
     if (rc) return rc;
     // keys, lists and the division check of buffer 2 were formed with the old constants
-    c->sorted_ok = c->tiles_ok = c->llist_ok = c->nlist_ok = false;
+    c->sorted_ok = c->tiles_ok = c->llist_ok = c->nlist_ok = c->lists_owed = false;
     WC_HIP(wc::launch_invalidate(c->b, c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
     return WC_OK;
@@ -962,6 +969,7 @@ WC_API int wc_sort_run(wc_ctx* c) {
     if (!c) return fail(WC_ERR_INVALID_ARG, "ctx is NULL");
     int rc = set_device(c);
     if (rc) return rc;
+    WC_HIP(refresh_lists(c, false));
     return enqueue_sort(c);
 }
 
@@ -1203,12 +1211,13 @@ WC_API int wc_set_tuning(wc_ctx* c, const wc_tuning* t) {
     const int nv = wc::num_variants();
     if (t->density_variant < 0 || t->density_variant >= nv || t->update_variant < 0 || t->update_variant >= nv)
         return fail(WC_ERR_INVALID_ARG, "variant outside [0, %d)", nv);
+    const int rc = set_device(c);
+    if (rc) return rc;
     if (t->neighbour_list) {
-        const int rc = set_device(c);
-        if (rc) return rc;
         const int ra = ensure_neighbour_lists(c);
         if (ra) return ra;
     }
+    if (!t->neighbour_list) WC_HIP(refresh_lists(c, false));
     c->density_variant = t->density_variant;
     c->update_variant = t->update_variant;
     c->neighbour_list = t->neighbour_list != 0;
@@ -1222,7 +1231,7 @@ WC_API int wc_get_neighbour_counts(wc_ctx* c, uint32_t* host, uint32_t n) {
     if (n != c->total_particles) return fail(WC_ERR_INVALID_ARG, "n = %u, the context holds %u", n, c->total_particles);
     int rc = set_device(c);
     if (rc) return rc;
-    WC_HIP(refresh_lists(c));
+    WC_HIP(refresh_lists(c, false));
     WC_HIP(hipMemcpyAsync(host, c->b.ncount, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
     return WC_OK;
@@ -1294,6 +1303,7 @@ WC_API int wc_tune(wc_ctx* c, float dt, uint32_t reps, wc_tuning* chosen, double
         if (err != hipSuccess) return fail(WC_ERR_HIP, "tuning failed: %s", hipGetErrorString(err));
         c->llist_ok = c->tile_ok;
         c->nlist_ok = true;
+        c->lists_owed = false;
         // The per-particle variants of the two passes combine freely; the tile variant's passes only with
         // each other (its force pass reads its density pass's lists).  Those lists are the same in both
         // modes, so a pick of the tile variant keeps neighbour lists available.
@@ -1652,7 +1662,7 @@ WC_API int wc_closure_features(wc_ctx* c, float dt_mult, const uint32_t* rows_ho
     } else {
         nrows = n;
     }
-    if (c->neighbour_list) WC_HIP(refresh_lists(c));
+    WC_HIP(refresh_lists(c, true));
     WC_HIP(wc::launch_closure_features(c->b, rows, nrows, dt_mult, (uint16_t*)x_dev, c->neighbour_list,
                                        c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
@@ -1684,7 +1694,7 @@ WC_API int wc_closure_infer(wc_ctx* c, wc_mlp* net, float dt_mult, void* y_dev) 
     rc = set_device(c);
     if (rc) return rc;
     WC_HIP(hipStreamSynchronize(net->m.stream));
-    WC_HIP(refresh_lists(c));
+    WC_HIP(refresh_lists(c, true));
     WC_HIP(closure_infer_from_lists(c, net, dt_mult, (float*)y_dev));
     WC_HIP(hipStreamSynchronize(c->stream));
     return WC_OK;
