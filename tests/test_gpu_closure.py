@@ -452,3 +452,26 @@ def test_frozen_force_integrator_matches_its_formula():
     assert free.sum() > 0.9 * n
     assert np.array_equal(out["position"][free].view(np.uint32), want_x[free].view(np.uint32))
     assert np.array_equal(out["velocity"][free].view(np.uint32), want_v[free].view(np.uint32))
+
+
+@pytest.mark.parametrize("variant", [2, -1], ids=["per particle", "tiles"])
+def test_lists_switched_on_after_the_density_pass(variant):
+    """List mode switched on between the density pass and inference: no lists are written yet, so none are read.  The
+    counts say overflowed, and inference gives the bits of the searching features followed by the network."""
+    p, parts = scenes.scaled_block((23, 21, 19), 0.01, seed=7, h_over_s=2.0)
+    n = p.num_particles
+    v = variant % L.lib().wc_num_variants()
+    net = ClosureNet(max_batch=64)
+    net.set_params((np.random.default_rng(12).normal(0, 0.05, ClosureNet.num_params())).astype(np.float32))
+    x, y1, y2 = DeviceArray((n, 208), np.uint16), DeviceArray((n, 4), np.float32), DeviceArray((n, 4), np.float32)
+    print(f"case lists switched on late, variant {v}", flush=True)
+    with Fluid(p, parts) as f:
+        f.set_tuning(v, v, 0)
+        f.sort_.run()
+        f.runDensityProg()
+        L.check(L.lib().wc_closure_features(f.ctx, C.c_float(4.0), None, 0, x.ptr), "wc_closure_features")
+        f.set_tuning(v, v, 1)
+        assert (f.neighbour_counts() == 0xFFFFFFFF).all()
+        L.check(L.lib().wc_closure_infer(f.ctx, net.h, C.c_float(4.0), y1.ptr), "wc_closure_infer")
+        L.check(L.lib().wc_mlp_predict(net.h, x.ptr, y2.ptr, n), "wc_mlp_predict")
+    assert np.array_equal(y1.download().view(np.uint32), y2.download().view(np.uint32))

@@ -388,10 +388,12 @@ int ensure_neighbour_lists(wc_ctx* c) {
         c->b.nlist = nullptr;
         return fail(WC_ERR_NO_MEMORY, "neighbour lists for %zu particles", n);
     }
-    if (!c->b.ncount && hipMalloc(&c->b.ncount, n * 4) != hipSuccess) {
+    if (hipMalloc(&c->b.ncount, n * 4) != hipSuccess) {
         c->b.ncount = nullptr;
         return fail(WC_ERR_NO_MEMORY, "neighbour counts for %zu particles", n);
     }
+    // Until a density pass writes the lists every one counts as overflowed: a reader then searches.
+    WC_HIP(hipMemsetAsync(c->b.ncount, 0xff, n * 4, c->stream));
     return WC_OK;
 }
 
