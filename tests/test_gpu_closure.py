@@ -474,4 +474,8 @@ def test_lists_switched_on_after_the_density_pass(variant):
         assert (f.neighbour_counts() == 0xFFFFFFFF).all()
         L.check(L.lib().wc_closure_infer(f.ctx, net.h, C.c_float(4.0), y1.ptr), "wc_closure_infer")
         L.check(L.lib().wc_mlp_predict(net.h, x.ptr, y2.ptr, n), "wc_mlp_predict")
-    assert np.array_equal(y1.download().view(np.uint32), y2.download().view(np.uint32))
+        assert np.array_equal(y1.download().view(np.uint32), y2.download().view(np.uint32))
+        before = x.download()
+        x.upload(np.zeros_like(before))
+        L.check(L.lib().wc_closure_features(f.ctx, C.c_float(4.0), None, 0, x.ptr), "wc_closure_features")
+        assert np.array_equal(x.download(), before)

@@ -1697,7 +1697,14 @@ WC_API int wc_closure_infer(wc_ctx* c, wc_mlp* net, float dt_mult, void* y_dev) 
     if (rc) return rc;
     WC_HIP(hipStreamSynchronize(net->m.stream));
     WC_HIP(refresh_lists(c, true));
-    WC_HIP(closure_infer_from_lists(c, net, dt_mult, (float*)y_dev));
+    if (c->nlist_ok) {
+        WC_HIP(closure_infer_from_lists(c, net, dt_mult, (float*)y_dev));
+    } else {
+        // No density pass in list mode since the last sort, upload or parameter change.  Rows may be marked overflowed
+        // and yet have few neighbours, which the selection does not expect; the feature kernel searches for those.
+        WC_HIP(wc::launch_closure_features(c->b, nullptr, c->total_particles, dt_mult, c->cl_x, true, c->stream));
+        WC_HIP(wc::mlp_infer(net->m, c->cl_x, (float*)y_dev, c->total_particles, c->stream));
+    }
     WC_HIP(hipStreamSynchronize(c->stream));
     return WC_OK;
 }
