@@ -276,7 +276,9 @@ WC_API const char* wc_pass_name(int k);
  * stages boxes of cells in LDS instead (both passes of it run together; without the memory for it,
  * or on a grid of more than 64 cells a particle, it stands for variant 2).  Every variant computes
  * bit-identical results, only speed differs.  Contexts of 50,000 particles and more, and of 20,000 a
- * scene, start with the last variant, others with variant 2.  No reference counterpart: the reference dispatches
+ * scene, start with the last variant if at rest density boxes fit LDS and lists hold the neighbours,
+ * others with variant 2: the parameters alone decide, so a state far from rest (a thin gas, say) may
+ * be faster by what wc_tune finds for it.  No reference counterpart: the reference dispatches
  * fixed 128-invocation work groups (src/core/util.h:18). */
 typedef struct wc_tuning {
     int32_t density_variant;

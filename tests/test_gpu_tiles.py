@@ -247,3 +247,16 @@ def test_neighbour_counts_are_those_of_the_last_listing_pass(sequence):
                 f.runDensityProg()
             out.append(f.neighbour_counts())
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("n_side,spacing,ratio,tiles", [((40, 40, 40), 0.0175, 2.0, True), ((40, 40, 40), 0.0175, 3.5, False),
+                                                       ((40, 40, 40), 0.0175, 4.7, False), ((36, 36, 36), 0.0175, 2.0, False),
+                                                       ((100, 100, 100), 0.008, 3.3, False)])
+def test_contexts_start_with_the_faster_passes(n_side, spacing, ratio, tiles):
+    """The start follows size and density (test_choose.py has the rule's edges): with 46 and 104 particles a cell, or 151
+    neighbours at a million, the per-particle passes are up to seven times faster."""
+    p, parts = scaled_block(n_side, spacing, 1, ratio)
+    with Fluid(p, parts) as f:
+        start = f.get_tuning()
+    v = L.lib().wc_num_variants() - 1 if tiles else 2
+    assert start == (v, v, 0)

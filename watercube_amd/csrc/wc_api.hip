@@ -197,29 +197,11 @@ bool short_arithmetic(const wc_params& p) {
            isfinite(p.spiky_const) && isfinite(p.visc_const * p.kernel_radius);
 }
 
-// Base box of the tile passes.  Larger boxes stage less halo per particle; they have to fit LDS at rest density (a
-// denser one is split) and leave the chip's 256 CUs enough boxes each.  At 8 particles a cell the whole step took, by
-// 4x3x4 / 4x2x4 / 2x2x4 (us): 91,125 particles 141 / 130 / 104, 125,000 126 / 137 / 137, 262,144 141 / 158 / 176: the
-// first from 300 boxes of it.  At 12 a cell, where it does not fit, by 4x2x4 / 2x2x4: 125,000 182 / 135, 192,089 (once
-// spread, three at once) 94 / 111, 2,048,000 1,087 / 1,109: the second from 450 boxes.  Below that 2x2x4 unless a box has more particles than threads: the
-// 80,000-particle scene (20 a cell) 228 by 2x2x4, 190 by 2x2x2.
-wc::TileShape choose_tile_shape(const std::vector<wc_params>& scenes) {
-    double n = 0.0, cell = 0.0;  // particles; those a cell holds at rest density
-    for (const wc_params& p : scenes) {
-        n += p.num_particles;
-        const double rest = (double)p.rest_density / (double)p.particle_mass * pow((double)p.bin_size, 3.0);
-        if (rest > 0.0 && rest < 1e6) cell += rest * p.num_particles;
-    }
-    cell = n > 0.0 ? cell / n : 0.0;
-    const struct {
-        wc::TileShape t;
-        double boxes;
-    } shapes[] = {{{4, 3, 4, wc::kTileLargeBlock, wc::kTileLargeCap}, 300.0},
-                  {{4, 2, 4, wc::kTileLargeBlock, wc::kTileLargeCap}, 450.0},
-                  {{2, 2, 4, wc::kTileSmallBlock, wc::kTileSmallCap}, 350.0}};
-    for (const auto& [t, boxes] : shapes)
-        if ((t.x + 2) * (t.y + 2) * (t.z + 2) * cell * 1.05 <= t.cap && n >= boxes * (t.x * t.y * t.z) * cell) return t;
-    return {2, 2, 16.0 * cell <= wc::kTileSmallBlock ? 4 : 2, wc::kTileSmallBlock, wc::kTileSmallCap};
+std::vector<wc::SceneFill> scene_fills(const std::vector<wc_params>& scenes) {
+    std::vector<wc::SceneFill> out;
+    for (const wc_params& p : scenes)
+        out.push_back(wc::scene_fill(p.num_particles, p.grid_res, p.bin_size, p.kernel_radius, p.rest_density, p.particle_mass));
+    return out;
 }
 
 // Base boxes classified per workgroup: about 2,000 workgroups, at least 8 boxes each (fewer workgroups
@@ -248,7 +230,7 @@ int layout_scenes(wc_ctx* c, uint64_t max_entries) {
     uint32_t* tblk = tiles + (S + 1);
     uint64_t p_off = 0, c_off = 0, boxes = 0, cells = 0;
     bool exact = true;
-    c->tile_shape = choose_tile_shape(c->params);
+    c->tile_shape = wc::choose_tile_shape(scene_fills(c->params));
     const wc::TileShape shape = c->tile_shape;
     c->tile_per = tiles_per_block(c->params, shape);
     for (uint32_t s = 0; s < S; ++s) {
@@ -573,7 +555,7 @@ int create_context(const wc_params* scenes, uint32_t num, wc_ctx** out) {
             b.table_cap = (uint32_t)tables;
             b.list_cap = (uint32_t)list_cap;
             b.list_chunks = (uint32_t)chunks;
-            if (n >= wc::kTileMinParticles && n / num >= wc::kTileMinPerScene)
+            if (wc::start_on_tiles(scene_fills(c->params), c->tile_shape))
                 c->density_variant = c->update_variant = wc::tile_variant();
         } else {
             c->tile_mem = nullptr;

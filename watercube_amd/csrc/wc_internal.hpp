@@ -11,6 +11,7 @@
 #include <stdint.h>
 
 #include "../../include/watercube.h"
+#include "wc_choose.hpp"
 
 namespace wc {
 
@@ -169,14 +170,6 @@ struct PassVariant {
 int num_variants();
 PassVariant variant(int v);
 
-// Tile passes (the last variant): a workgroup stages one box of cells and its halo in LDS.
-struct TileShape {
-    int x, y, z;  // cells of a base box
-    int block;    // threads per workgroup: kTileLargeBlock or kTileSmallBlock
-    int cap;      // records (box and halo) its LDS holds
-};
-constexpr int kTileLargeBlock = 512, kTileLargeCap = 1920;
-constexpr int kTileSmallBlock = 256, kTileSmallCap = 2304;
 int tile_variant();
 // What the sort forms for them.
 struct TileWork {
@@ -195,15 +188,6 @@ struct TileWork {
 constexpr uint32_t kListCount = 32;          // in another 128-byte line: atomics on one line serialise
 constexpr uint32_t kSceneSparse = 64;
 constexpr uint32_t kTileBlock = 256;         // threads, and at most that many boxes, per classification workgroup
-// Neighbours a particle's list holds (16 bits each; particles with more search directly): dense clusters
-// have a few hundred; large contexts keep lists of half the size.
-inline uint32_t tile_list_cap(uint64_t particles) { return particles <= 500000 ? 512u : particles <= 4000000 ? 256u : 128u; }
-// Contexts of this many particles start with the tile passes.  Smaller ones gain while the fluid is at rest
-// density (16,384 particles, three contexts at once: 20 us a step against 33) and lose as it spreads and boxes
-// empty (44 against 36 at step 4,000); 80,000 particles gain in both (83 against 131, 84 against 122).
-// Batches also need 20,000 particles a scene: 62 scenes of about 31,000 780 -> 693, 28 of about 14,000 207 -> 215
-// once spread.  wc_tune times both whatever the size.
-constexpr uint32_t kTileMinParticles = 50000, kTileMinPerScene = 20000;
 // Chunks of 64 lanes that lists are kept for.  Full boxes use 1.2 lanes a particle (columns are rounded to four
 // lanes, boxes to 64), a fluid that has spread up to 1.4; boxes past the memory search directly.
 inline uint64_t tile_list_chunks(uint64_t particles) { return particles / 32 + 1024; }
