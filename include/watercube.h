@@ -300,7 +300,8 @@ WC_API int wc_get_neighbour_counts(wc_ctx* ctx, uint32_t* host, uint32_t n);
 
 /* Autotuner: sorts the current state once, then times every variant of the density pass and of
  * the force pass (reps launches each, HIP events on the context's stream), both without and with
- * neighbour lists, and keeps the fastest variant pair of the faster mode for later steps.  dt > 0
+ * neighbour lists, then whole steps (reps each) of the fastest pair without lists, with them and of
+ * the last variant, and keeps the fastest of these for later steps.  dt > 0
  * sets every scene's step size first; dt <= 0 keeps them.  Particle buffer 1 is restored
  * afterwards; buffer 2 (the sorted copy the next step rebuilds anyway) is left sorted.  Each
  * non-NULL array receives wc_num_variants() average launch times in milliseconds: the two passes

@@ -3,7 +3,25 @@
 
 #include "wc_choose.hpp"
 
-int main() {
+// variants, whether the tile passes can run, then the times per mode and pass
+static int tune() {
+    int nv, tiles;
+    while (scanf("%d %d", &nv, &tiles) == 2) {
+        std::vector<double> t[2][2];
+        for (auto& m : t)
+            for (auto& v : m) {
+                v.resize(nv);
+                for (double& x : v)
+                    if (scanf("%lf", &x) != 1) return 1;
+            }
+        for (const wc::TuningPick& p : wc::tuning_candidates(t, tiles != 0))
+            printf("%d %d %d\n", p.density, p.update, p.lists ? 1 : 0);
+    }
+    return 0;
+}
+
+int main(int argc, char**) {
+    if (argc > 1) return tune();
     int scenes;
     while (scanf("%d", &scenes) == 1) {
         std::vector<wc::SceneFill> fills;

@@ -1,5 +1,5 @@
 """The library's choices by size and density (csrc/wc_choose.hpp), on the CPU: box shapes of the tile passes, and which
-contexts start with them.  Expected values are the faster of both sides as measured (the header names the times)."""
+contexts start with them, and the tuner's candidates.  Expected values are the faster of both sides as measured (the header names the times)."""
 import subprocess
 from pathlib import Path
 
@@ -11,11 +11,15 @@ CSRC = HERE.parent / "watercube_amd" / "csrc"
 
 
 @pytest.fixture(scope="module")
-def choose(tmp_path_factory):
+def exe(tmp_path_factory):
     exe = tmp_path_factory.mktemp("choose") / "choose"
     subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-I", str(CSRC), str(HERE / "choose_main.cpp"), "-o",
                     str(exe)], check=True)
+    return exe
 
+
+@pytest.fixture(scope="module")
+def choose(exe):
     def run(*contexts):
         """Each context a list of scenes (n, R, bin, h, rest density, mass); (starts, shape) of each."""
         text = "".join(f"{len(c)} " + " ".join(str(v) for s in c for v in s) + "\n" for c in contexts)
@@ -98,3 +102,24 @@ def test_box_shapes(choose):
                 assert halo * cell <= cap[t], (n, cell, t)
             else:
                 assert t == (2, 2, 2)
+
+
+def test_tuner_candidates(exe):
+    """The fastest pair of each mode, and the tile passes (the last variant) together: neither of them in another pair."""
+    def candidates(tiles, t):
+        text = f"{len(t[0][0])} {int(tiles)} " + " ".join(str(x) for m in t for p in m for x in p)
+        r = subprocess.run([str(exe), "tune"], input=text, capture_output=True, text=True, check=True)
+        return [tuple(map(int, ln.split())) for ln in r.stdout.splitlines()]
+
+    # [lists][pass][variant], three per-particle variants and the tiles
+    t = [[[0.050, 0.048, 0.052, 0.040], [0.060, 0.066, 0.063, 0.070]], [[0.055, 0.057, 0.054, 0.041], [0.041, 0.044, 0.040, 0.029]]]
+    assert candidates(True, t) == [(1, 0, 0), (2, 2, 1), (3, 3, 1)]
+    assert candidates(False, t) == [(1, 0, 0), (2, 2, 1)]
+    # too far behind the least sum (0.070): more than 1.3 of it and 0.05 ms
+    t = [[[0.09, 0.04, 0.05, 0.04], [0.06, 0.06, 0.07, 0.03]], [[0.1, 0.1, 0.1, 0.05], [0.042, 0.07, 0.041, 0.03]]]
+    t[1][0] = [0.09, 0.1, 0.1, 0.05]
+    assert candidates(True, t) == [(1, 0, 0), (0, 2, 1), (3, 3, 1)]
+    t[1][0] = [0.12, 0.13, 0.14, 0.05]
+    assert candidates(True, t) == [(1, 0, 0), (3, 3, 1)]
+    t[0][1] = [0.3] * 3 + [0.03]
+    assert candidates(True, t) == [(3, 3, 1)] and candidates(False, t) == [(0, 2, 1)]

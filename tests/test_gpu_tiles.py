@@ -260,3 +260,31 @@ def test_contexts_start_with_the_faster_passes(n_side, spacing, ratio, tiles):
         start = f.get_tuning()
     v = L.lib().wc_num_variants() - 1 if tiles else 2
     assert start == (v, v, 0)
+
+
+@pytest.mark.parametrize("per", [2, 8])
+def test_tuner_leaves_the_state_and_its_lists(per, oracle):
+    """wc_tune times steps, and restores buffer 1; buffer 2, the cells and the neighbour lists are those of that state
+    whichever passes it picks, and the next steps give the oracle's bits."""
+    p, parts = scaled_block((30, 30, 30), 0.025, 4)
+    n = len(parts)
+    p.grid_res = round((n / per) ** (1 / 3))
+    p.kernel_radius = 0.999 / p.grid_res
+    L.derive(p)
+    parts["position"] = np.random.default_rng(2).uniform(0.01, 0.99, (n, 3)).astype(np.float32)
+    print(f"case tuner, {per} a cell", flush=True)
+    st = oracle.OracleState(p, parts)
+    with Fluid(p, parts) as f:
+        f.set_tuning(2, 2, 1)
+        f.sort_.run()
+        f.runDensityProg()
+        want = f.particles(2).tobytes(), f.neighbour_counts().tobytes(), f.sort_.getOffsetBuffer().tobytes()
+        f.tune(1e-4, reps=2)
+        assert f.particles(1).tobytes() == parts.tobytes()
+        assert (f.particles(2).tobytes(), f.neighbour_counts().tobytes(), f.sort_.getOffsetBuffer().tobytes()) == want
+        f.runUpdateProg(1e-4)
+        st.step(1e-4, 1)
+        assert np.array_equal(f.particles(1).view(np.uint32), st.buf1.view(np.uint32))
+        f.step(1e-4, 3)
+        st.step(1e-4, 3)
+        assert np.array_equal(f.particles(1).view(np.uint32), st.buf1.view(np.uint32))

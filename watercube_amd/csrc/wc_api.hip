@@ -1251,6 +1251,17 @@ WC_API int wc_tune(wc_ctx* c, float dt, uint32_t reps, wc_tuning* chosen, double
             err = hipMemcpyAsync(save_pos, c->b.posrho[0], n * sizeof(float4), hipMemcpyDeviceToDevice, c->stream);
         if (err == hipSuccess)
             err = hipMemcpyAsync(save_vel, c->b.velp[0], n * sizeof(float4), hipMemcpyDeviceToDevice, c->stream);
+        // average time of `launch`, after one to warm up
+        auto timed = [&](auto launch, double& ms_out) {
+            err = launch();
+            if (err == hipSuccess) err = hipEventRecord(ev.start, c->stream);
+            for (uint32_t r = 0; r < reps && err == hipSuccess; ++r) err = launch();
+            if (err == hipSuccess) err = hipEventRecord(ev.stop, c->stream);
+            if (err == hipSuccess) err = hipEventSynchronize(ev.stop);
+            float ms = 0.0f;
+            if (err == hipSuccess) err = hipEventElapsedTime(&ms, ev.start, ev.stop);
+            ms_out = (double)ms / reps;
+        };
         if (err == hipSuccess) err = launch_sort(c, c->tile_ok, [](int) { return hipSuccess; });
         // Both passes are idempotent on the sorted buffer: density rewrites the same densities
         // (and, with lists, the same lists), the force pass rewrites buffer 1 from buffer 2 alone.
@@ -1266,49 +1277,50 @@ WC_API int wc_tune(wc_ctx* c, float dt, uint32_t reps, wc_tuning* chosen, double
                         return pass == 0 ? wc::launch_density(c->b, particle_variant(v), mode == 1, c->stream)
                                          : wc::launch_update(c->b, particle_variant(v), mode == 1, c->stream);
                     };
-                    err = launch();  // warm-up
-                    if (err == hipSuccess) err = hipEventRecord(ev.start, c->stream);
-                    for (uint32_t r = 0; r < reps && err == hipSuccess; ++r) err = launch();
-                    if (err == hipSuccess) err = hipEventRecord(ev.stop, c->stream);
-                    if (err == hipSuccess) err = hipEventSynchronize(ev.stop);
-                    float ms = 0.0f;
-                    if (err == hipSuccess) err = hipEventElapsedTime(&ms, ev.start, ev.stop);
-                    t[mode][pass][v] = (double)ms / reps;
+                    timed(launch, t[mode][pass][v]);
                 }
             }
         }
+        auto restore = [&]() {
+            if (err == hipSuccess)
+                err = hipMemcpyAsync(c->b.posrho[0], save_pos, n * sizeof(float4), hipMemcpyDeviceToDevice, c->stream);
+            if (err == hipSuccess)
+                err = hipMemcpyAsync(c->b.velp[0], save_vel, n * sizeof(float4), hipMemcpyDeviceToDevice, c->stream);
+        };
+        const wc::TuningPick before{c->density_variant, c->update_variant, c->neighbour_list};
+        auto use = [&](const wc::TuningPick& p) {
+            c->density_variant = p.density;
+            c->update_variant = p.update;
+            c->neighbour_list = p.lists;
+        };
+        wc::TuningPick pick = before;
+        double fastest = 0.0;
+        const std::vector<wc::TuningPick> candidates = wc::tuning_candidates(t, c->tile_ok);
+        for (const wc::TuningPick& p : candidates) {
+            restore();
+            if (err != hipSuccess) break;
+            use(p);
+            double ms = 0.0;
+            if (candidates.size() > 1)
+                timed([&]() { return enqueue_step(c) == WC_OK ? hipSuccess : hipErrorUnknown; }, ms);
+            if (candidates.size() == 1 || fastest == 0.0 || ms < fastest) {
+                fastest = ms;
+                pick = p;
+            }
+        }
+        // buffer 2 as the passes leave it for the state that the caller sees, with the lists whatever the pick
+        restore();
+        use(err == hipSuccess ? pick : before);
+        drop_graph(c);
+        if (err == hipSuccess) err = launch_sort(c, density_by_tiles(c), [](int) { return hipSuccess; });
         if (err == hipSuccess)
-            err = hipMemcpyAsync(c->b.posrho[0], save_pos, n * sizeof(float4), hipMemcpyDeviceToDevice, c->stream);
-        if (err == hipSuccess)
-            err = hipMemcpyAsync(c->b.velp[0], save_vel, n * sizeof(float4), hipMemcpyDeviceToDevice, c->stream);
+            err = density_by_tiles(c) ? launch_density_pass(c, true)
+                                      : wc::launch_density(c->b, particle_variant(c->density_variant), true, c->stream);
+        c->nlist_ok = err == hipSuccess;
         if (err == hipSuccess) err = hipStreamSynchronize(c->stream);
         (void)hipFree(save_pos);
         (void)hipFree(save_vel);
         if (err != hipSuccess) return fail(WC_ERR_HIP, "tuning failed: %s", hipGetErrorString(err));
-        c->llist_ok = c->tile_ok;
-        c->nlist_ok = true;
-        c->lists_owed = false;
-        // The per-particle variants of the two passes combine freely; the tile variant's passes only with
-        // each other (its force pass reads its density pass's lists).  Those lists are the same in both
-        // modes, so a pick of the tile variant keeps neighbour lists available.
-        const int tile = wc::tile_variant();
-        int best[2][2] = {{0, 0}, {0, 0}};
-        for (int mode = 0; mode < 2; ++mode)
-            for (int pass = 0; pass < 2; ++pass)
-                for (int v = 1; v < nv; ++v)
-                    if (v != tile && t[mode][pass][v] < t[mode][pass][best[mode][pass]]) best[mode][pass] = v;
-        const double step0 = t[0][0][best[0][0]] + t[0][1][best[0][1]];
-        const double step1 = t[1][0][best[1][0]] + t[1][1][best[1][1]];
-        const double step_tile = fmin(t[0][0][tile], t[1][0][tile]) + fmin(t[0][1][tile], t[1][1][tile]);
-        const int mode = step1 < step0 ? 1 : 0;
-        c->density_variant = best[mode][0];
-        c->update_variant = best[mode][1];
-        c->neighbour_list = mode == 1;
-        if (c->tile_ok && step_tile < fmin(step0, step1)) {
-            c->density_variant = c->update_variant = tile;
-            c->neighbour_list = true;
-        }
-        drop_graph(c);
     }
     if (chosen) {
         chosen->density_variant = c->density_variant;

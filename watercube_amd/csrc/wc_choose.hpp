@@ -115,4 +115,36 @@ inline bool start_on_tiles(const std::vector<SceneFill>& scenes, const TileShape
     return n <= most;
 }
 
+// The tuner's candidates from the times t[lists][pass][variant] of the density and force pass: the fastest pair without
+// neighbour lists, with them, and the last variant's (by tiles), whose passes run only with each other and form the same
+// lists in both modes.  Which of them it is, whole steps decide: the tile passes' sort also forms their work list and
+// tables (a million particles 20 us, 17.8 million 0.28 ms), and a pass timed alone finds its data in the caches.  Left out
+// are candidates too far behind for either (times in ms).
+struct TuningPick {
+    int density, update;
+    bool lists;
+};
+inline std::vector<TuningPick> tuning_candidates(const std::vector<double> (&t)[2][2], bool tiles) {
+    const int tile = (int)t[0][0].size() - 1;
+    std::vector<TuningPick> all, out;
+    std::vector<double> sum;
+    for (int mode = 0; mode < 2; ++mode) {
+        int best[2] = {0, 0};
+        for (int pass = 0; pass < 2; ++pass)
+            for (int v = 1; v < tile; ++v)
+                if (t[mode][pass][v] < t[mode][pass][best[pass]]) best[pass] = v;
+        all.push_back({best[0], best[1], mode == 1});
+        sum.push_back(t[mode][0][best[0]] + t[mode][1][best[1]]);
+    }
+    if (tiles) {
+        all.push_back({tile, tile, true});
+        sum.push_back(fmin(t[0][0][tile], t[1][0][tile]) + fmin(t[0][1][tile], t[1][1][tile]));
+    }
+    double least = sum[0];
+    for (double v : sum) least = fmin(least, v);
+    for (size_t k = 0; k < all.size(); ++k)
+        if (sum[k] <= 1.3 * least + 0.05) out.push_back(all[k]);
+    return out;
+}
+
 }  // namespace wc
