@@ -479,3 +479,19 @@ def test_lists_switched_on_after_the_density_pass(variant):
         x.upload(np.zeros_like(before))
         L.check(L.lib().wc_closure_features(f.ctx, C.c_float(4.0), None, 0, x.ptr), "wc_closure_features")
         assert np.array_equal(x.download(), before)
+
+
+def test_tuner_restores_identities():
+    """wc_tune restores buffer 1; tracked identities stay with its records, now and after the next steps."""
+    p, parts, dt, _ = scenes.workload("dam_break_16k")
+    print("case identities through the tuner", flush=True)
+    with Fluid(p, parts) as a, Fluid(p, parts) as b:
+        for f in (a, b):
+            f.track_ids(True)  # and no step yet: the next sort moves most particles
+        before = a.ids(1)
+        a.tune(dt, reps=1)
+        assert np.array_equal(a.ids(1), before)
+        for f in (a, b):
+            f.step(dt, 3)
+        assert a.particles(1).tobytes() == b.particles(1).tobytes()
+        assert np.array_equal(a.ids(1), b.ids(1))

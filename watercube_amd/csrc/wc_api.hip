@@ -1245,12 +1245,20 @@ WC_API int wc_tune(wc_ctx* c, float dt, uint32_t reps, wc_tuning* chosen, double
             (void)hipFree(save_pos);
             return fail(WC_ERR_NO_MEMORY, "tuning copy of %zu particles", n);
         }
+        uint32_t* save_ids = nullptr;  // identities move with the records
+        if (c->b.ids[0] && hipMalloc(&save_ids, n * sizeof(uint32_t)) != hipSuccess) {
+            (void)hipFree(save_pos);
+            (void)hipFree(save_vel);
+            return fail(WC_ERR_NO_MEMORY, "tuning copy of %zu identities", n);
+        }
         EventPair ev;
         hipError_t err = ev.create();
         if (err == hipSuccess)
             err = hipMemcpyAsync(save_pos, c->b.posrho[0], n * sizeof(float4), hipMemcpyDeviceToDevice, c->stream);
         if (err == hipSuccess)
             err = hipMemcpyAsync(save_vel, c->b.velp[0], n * sizeof(float4), hipMemcpyDeviceToDevice, c->stream);
+        if (err == hipSuccess && save_ids)
+            err = hipMemcpyAsync(save_ids, c->b.ids[0], n * sizeof(uint32_t), hipMemcpyDeviceToDevice, c->stream);
         // average time of `launch`, after one to warm up
         auto timed = [&](auto launch, double& ms_out) {
             err = launch();
@@ -1286,6 +1294,8 @@ WC_API int wc_tune(wc_ctx* c, float dt, uint32_t reps, wc_tuning* chosen, double
                 err = hipMemcpyAsync(c->b.posrho[0], save_pos, n * sizeof(float4), hipMemcpyDeviceToDevice, c->stream);
             if (err == hipSuccess)
                 err = hipMemcpyAsync(c->b.velp[0], save_vel, n * sizeof(float4), hipMemcpyDeviceToDevice, c->stream);
+            if (err == hipSuccess && save_ids)
+                err = hipMemcpyAsync(c->b.ids[0], save_ids, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, c->stream);
         };
         const wc::TuningPick before{c->density_variant, c->update_variant, c->neighbour_list};
         auto use = [&](const wc::TuningPick& p) {
@@ -1320,6 +1330,7 @@ WC_API int wc_tune(wc_ctx* c, float dt, uint32_t reps, wc_tuning* chosen, double
         if (err == hipSuccess) err = hipStreamSynchronize(c->stream);
         (void)hipFree(save_pos);
         (void)hipFree(save_vel);
+        if (save_ids) (void)hipFree(save_ids);
         if (err != hipSuccess) return fail(WC_ERR_HIP, "tuning failed: %s", hipGetErrorString(err));
     }
     if (chosen) {
