@@ -288,3 +288,94 @@ def test_tuner_leaves_the_state_and_its_lists(per, oracle):
         f.step(1e-4, 3)
         st.step(1e-4, 3)
         assert np.array_equal(f.particles(1).view(np.uint32), st.buf1.view(np.uint32))
+
+
+def _held(make, count):
+    """Bytes of GPU memory that `count` contexts made by make() hold, per context."""
+    import ctypes as C
+
+    def free():  # the HIP runtime the library itself is linked with
+        a, b = C.c_size_t(), C.c_size_t()
+        assert L.lib().hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    before = free()
+    made = [make() for _ in range(count)]
+    held = before - free()
+    for f in made:
+        f.close()
+    return held / count
+
+
+@pytest.mark.parametrize("case", ["2,048", "one particle", "16,384", "64,000 per particle", "64,000 tuned off", "2,048 by tiles"])
+def test_memory_of_contexts_without_the_tile_passes(case):
+    """A context holds the tile passes' buffers (2 KB a particle and more) only if it runs them; few boxes and particles
+    need few list chunks."""
+    tile = L.lib().wc_num_variants() - 1
+    n_side = {"2,048": (16, 16, 8), "one particle": (1, 1, 1), "16,384": (32, 32, 16), "2,048 by tiles": (16, 16, 8)}.get(case, (40, 40, 40))
+    p, parts = scaled_block(n_side, 0.015, 1)
+    if case == "64,000 tuned off":  # a thin gas, which the tuner finds faster per particle
+        p.grid_res, p.kernel_radius = 28, 0.999 / 28
+        L.derive(p)
+        parts["position"] = np.random.default_rng(1).uniform(0.01, 0.99, (len(parts), 3)).astype(np.float32)
+
+    def make():
+        f = Fluid(p, parts).setup()
+        if case == "64,000 per particle":
+            f.set_tuning(2, 2, 0)
+        elif case == "64,000 tuned off":
+            f.tune(1e-6, reps=2)
+            assert f.get_tuning()[0] != tile
+        elif case == "2,048 by tiles":
+            f.set_tuning(tile, tile, 0)
+        f.step(1e-6, 2)
+        f.synchronize()
+        return f
+
+    make().close()  # what the library and the runtime load once
+    cells = int(p.grid_res) ** 3
+    base = 200 * len(parts) + 16 * cells + (260 * len(parts) if case == "64,000 tuned off" else 0)
+    # some 24 buffers, a stream and two graphs take 8 MB however small; 2,048 particles 357 list chunks of 64 KB
+    limit = base + (12 << 20) + (28 << 20 if case == "2,048 by tiles" else 0)
+    held = _held(make, 8)
+    print(f"case {case}: {held / 1e6:.1f} MB a context, limit {limit / 1e6:.1f}", flush=True)
+    assert held < limit
+
+
+def test_buffers_follow_the_tuning(oracle):
+    """The tile passes' buffers come with the first sort that needs them, also after steps of other passes, a larger grid or
+    a tuner's run: the oracle's bits throughout."""
+    import ctypes as C
+
+    tile = L.lib().wc_num_variants() - 1
+    p, parts = scaled_block((30, 31, 29), 0.02, 3)
+    small, _ = scaled_block((30, 31, 29), 0.02, 3, 3.3)  # fewer cells, other boxes
+    st = oracle.OracleState(p, parts)
+    with Fluid(p, parts) as f:
+        def check(what, q=p):
+            nonlocal st
+            print(f"case {what}", flush=True)
+            st = oracle.OracleState(q, st.buf1)
+            f.step(2e-5, 2)
+            st.step(2e-5, 2)
+            f.synchronize()
+            assert np.array_equal(f.particles(1).view(np.uint32), st.buf1.view(np.uint32)), what
+
+        check("per particle")
+        L.check(L.lib().wc_set_params(f.ctx, C.byref(small)), "wc_set_params")
+        f.set_tuning(tile, tile, 1)
+        check("tiles, few cells", small)
+        L.check(L.lib().wc_set_params(f.ctx, C.byref(p)), "wc_set_params")
+        check("tiles, more cells")
+        f.set_tuning(2, 2, 1)
+        check("per particle again")
+        f.tune(1e-7, reps=1)
+        check("tuned")
+        f.set_tuning(tile, tile, 1)
+        f.sort_.run()
+        f.runDensityProg()
+        f.runUpdateProg(2e-5)
+        st.step(2e-5, 1)
+        f.synchronize()
+        assert np.array_equal(f.particles(1).view(np.uint32), st.buf1.view(np.uint32))
+        check("after passes one by one")

@@ -144,9 +144,11 @@ struct wc_ctx {
     // tile passes: their base box (choose_tile_shape()), and whether the context may use them
     wc::TileShape tile_shape{};
     uint32_t tile_per = 1;  // base boxes per classification workgroup
+    bool tile_fit = false;      // the scenes allow them; with their buffers in place (ensure_tiles()), tile_ok
     bool tile_ok = false;
-    uint32_t tile_entries = 0;  // entries the work list needs at most
+    uint64_t tile_boxes = 0;    // base boxes of all scenes
     void* tile_mem = nullptr;   // the tile passes' buffers, one allocation
+    bool tile_refused = false;  // there was no room for them; asked again after wc_set_tuning, wc_tune, wc_set_params
     // What the last queued passes left in the buffers; a host upload or a parameter change clears all.
     bool sorted_ok = false;  // buffer 2 holds the last sort's output, every slot in its cell's range
     bool tiles_ok = false;   // ... and the work list is that sort's
@@ -217,9 +219,8 @@ uint32_t tiles_per_block(const std::vector<wc_params>& scenes, const wc::TileSha
     return per;
 }
 
-// Lays the scenes out (particle and cell offsets, block and tile tables) from c->params.  max_entries: what
-// the tile passes' work list may hold.
-int layout_scenes(wc_ctx* c, uint64_t max_entries) {
+// Lays the scenes out (particle and cell offsets, block and tile tables) from c->params.
+int layout_scenes(wc_ctx* c) {
     const uint32_t S = c->num_scenes;
     c->desc.assign(S, SceneDesc{});
     c->tables.assign(5 * (size_t)(S + 1), 0u);
@@ -261,9 +262,10 @@ int layout_scenes(wc_ctx* c, uint64_t max_entries) {
     c->total_cells = (uint32_t)c_off;
     // The tile passes look at every base box: on a grid with far more cells than particles that costs
     // more than they gain.
-    const uint64_t entries = wc::tile_capacity(boxes, p_off);
-    c->tile_ok = exact && p_off > 0 && cells <= kTileMaxCellsPerParticle * p_off && entries <= max_entries;
-    c->tile_entries = c->tile_ok ? (uint32_t)entries : 0u;
+    c->tile_boxes = boxes;
+    c->tile_fit = exact && p_off > 0 && cells <= kTileMaxCellsPerParticle * p_off &&
+                  wc::tile_capacity(boxes, p_off) <= 0xFFFFFFFFull;
+    c->tile_ok = c->tile_refused = false;
     c->scene_tab.clear();
     if (S > 1) {
         for (const uint32_t* first : {blk64, blk128, blk256, tiles, tblk})
@@ -379,6 +381,62 @@ int ensure_neighbour_lists(wc_ctx* c) {
     return WC_OK;
 }
 
+void release_tiles(wc_ctx* c) {
+    if (c->tile_mem) (void)hipFree(c->tile_mem);
+    c->tile_mem = nullptr;
+    c->b.tiles = nullptr;
+    c->b.tile_count = nullptr;
+    c->tile_ok = c->tiles_ok = c->llist_ok = c->lists_owed = false;
+}
+
+// The tile passes' buffers, allocated before the first sort that feeds those passes (a context that never runs them
+// holds none), and again if a change of parameters asks for more.  Not under capture.  tile_ok says whether they are there.
+hipError_t ensure_tiles(wc_ctx* c) {
+    c->tile_ok = false;
+    if (!c->tile_fit || c->tile_refused) return hipSuccess;
+    DeviceBuffers& b = c->b;
+    const size_t n = c->particle_cap ? c->particle_cap : 1;
+    const size_t entries = (size_t)wc::tile_capacity(c->tile_boxes, n);
+    const size_t chunks = (size_t)wc::tile_list_chunks(n);
+    c->tile_ok = c->tile_mem && entries <= b.tile_cap;
+    if (c->tile_ok) return hipSuccess;
+    hipError_t e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) return e;
+    drop_graph(c);
+    release_tiles(c);
+    // Only with room left for what a caller may ask for later, about 1 KB a particle (neighbour lists, a learned step's
+    // workspace): else the context keeps the per-particle passes.
+    const size_t list_cap = wc::tile_list_cap(n);
+    const size_t tables = n / 128 + 1024 < entries ? n / 128 + 1024 : entries;
+    const size_t count_bytes = (wc::kSceneSparse + (size_t)c->num_scenes) * 4;
+    const size_t bytes[6] = {entries * sizeof(uint4), count_bytes, tables * wc::kTileTableBytes, n * 4,
+                             chunks * 64 * list_cap * sizeof(uint16_t), chunks * 64 * sizeof(uint16_t)};
+    void** const ptr[6] = {(void**)&b.tiles,  (void**)&b.tile_count, &b.tables,
+                           (void**)&b.sparse, (void**)&b.llist,      (void**)&b.lcount};
+    size_t free_bytes = 0, total_bytes = 0, all = 0;
+    for (size_t v : bytes) all += (v + 255) / 256 * 256;
+    if (entries > 0xFFFFFFFFull || hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess || all + n * 1024 > free_bytes ||
+        hipMalloc(&c->tile_mem, all) != hipSuccess) {
+        c->tile_mem = nullptr;
+        c->tile_refused = true;
+        (void)hipGetLastError();
+        return hipSuccess;
+    }
+    char* at = static_cast<char*>(c->tile_mem);
+    for (int k = 0; k < 6; ++k) {
+        *ptr[k] = at;
+        at += (bytes[k] + 255) / 256 * 256;
+    }
+    b.tile_cap = (uint32_t)entries;
+    b.table_cap = (uint32_t)tables;
+    b.list_cap = (uint32_t)list_cap;
+    b.list_chunks = (uint32_t)chunks;
+    c->tile_ok = true;
+    return hipMemsetAsync(b.tile_count, 0, count_bytes, c->stream);
+}
+// ... if the current tuning runs those passes.  Before a sort is queued.
+hipError_t prepare_tiles(wc_ctx* c) { return c->density_variant == wc::tile_variant() ? ensure_tiles(c) : hipSuccess; }
+
 bool density_by_tiles(const wc_ctx* c) { return c->tile_ok && c->density_variant == wc::tile_variant(); }
 bool update_by_tiles(const wc_ctx* c) { return density_by_tiles(c) && c->update_variant == wc::tile_variant(); }
 // the per-particle variant of a pass whose tile form cannot run
@@ -476,7 +534,7 @@ int create_context(const wc_params* scenes, uint32_t num, wc_ctx** out) {
     if (!c) return fail(WC_ERR_NO_MEMORY, "host allocation failed");
     c->num_scenes = num;
     c->params.assign(scenes, scenes + num);
-    int rc = layout_scenes(c, 0xFFFFFFFFu);
+    int rc = layout_scenes(c);
     if (rc) {
         delete c;
         return rc;
@@ -532,36 +590,8 @@ int create_context(const wc_params* scenes, uint32_t num, wc_ctx** out) {
         return fail(WC_ERR_NO_MEMORY, "device allocation failed (%u particles, %u cells)", c->total_particles,
                     c->total_cells);
     }
-    if (c->tile_ok) {
-        // Only with room left for what a caller may ask for later, about 1 KB a particle (neighbour lists, a
-        // learned step's workspace): else the context keeps the per-particle passes.
-        const size_t list_cap = wc::tile_list_cap(n), chunks = wc::tile_list_chunks(n);
-        const size_t tables = n / 128 + 1024 < c->tile_entries ? n / 128 + 1024 : c->tile_entries;
-        const size_t bytes[6] = {c->tile_entries * sizeof(uint4), (wc::kSceneSparse + (size_t)num) * 4, tables * wc::kTileTableBytes, n * 4,
-                                 chunks * 64 * list_cap * sizeof(uint16_t), chunks * 64 * sizeof(uint16_t)};
-        void** const ptr[6] = {(void**)&b.tiles,  (void**)&b.tile_count, &b.tables,
-                               (void**)&b.sparse, (void**)&b.llist,      (void**)&b.lcount};
-        size_t free_bytes = 0, total_bytes = 0, all = 0;
-        for (size_t v : bytes) all += (v + 255) / 256 * 256;
-        c->tile_ok = hipMemGetInfo(&free_bytes, &total_bytes) == hipSuccess && all + n * 1024 <= free_bytes &&
-                     hipMalloc(&c->tile_mem, all) == hipSuccess;
-        if (c->tile_ok) {
-            char* at = static_cast<char*>(c->tile_mem);
-            for (int k = 0; k < 6; ++k) {
-                *ptr[k] = at;
-                at += (bytes[k] + 255) / 256 * 256;
-            }
-            b.tile_cap = c->tile_entries;
-            b.table_cap = (uint32_t)tables;
-            b.list_cap = (uint32_t)list_cap;
-            b.list_chunks = (uint32_t)chunks;
-            if (wc::start_on_tiles(scene_fills(c->params), c->tile_shape))
-                c->density_variant = c->update_variant = wc::tile_variant();
-        } else {
-            c->tile_mem = nullptr;
-            (void)hipGetLastError();
-        }
-    }
+    if (c->tile_fit && wc::start_on_tiles(scene_fills(c->params), c->tile_shape))
+        c->density_variant = c->update_variant = wc::tile_variant();
     hipError_t e = hipSuccess;
     auto zero = [&](void* p, size_t bytes) {
         if (e == hipSuccess) e = hipMemsetAsync(p, 0, bytes, c->stream);
@@ -574,7 +604,6 @@ int create_context(const wc_params* scenes, uint32_t num, wc_ctx** out) {
     zero(b.step_start, 64);
     zero(b.rho_max, 64);
     zero(b.crowd_count, 64);
-    if (c->tile_ok) zero(b.tile_count, (wc::kSceneSparse + (size_t)num) * 4);
     // rho_max[1] = 2: no density pass has checked the force pass's division operands yet
     if (e == hipSuccess) e = hipMemsetAsync(reinterpret_cast<char*>(b.rho_max) + 4, 2, 1, c->stream);
     zero(b.sorted, n * 4);
@@ -636,6 +665,7 @@ int run_steps(wc_ctx* c, uint32_t nsteps) {
     if (nsteps == 0) return WC_OK;
     int rc = set_device(c);
     if (rc) return rc;
+    WC_HIP(prepare_tiles(c));
     if (!c->graph_valid) {
         rc = capture_step(c);
         if (rc) return rc;
@@ -901,7 +931,7 @@ WC_API int wc_set_params(wc_ctx* c, const wc_params* p) {
     WC_HIP(hipStreamSynchronize(c->stream));
     const float dt = c->desc[0].dt;
     c->params[0] = *p;
-    rc = layout_scenes(c, c->b.tile_cap);
+    rc = layout_scenes(c);
     if (rc) return rc;
     c->desc[0].dt = dt;
     drop_graph(c);
@@ -954,6 +984,7 @@ WC_API int wc_sort_run(wc_ctx* c) {
     int rc = set_device(c);
     if (rc) return rc;
     WC_HIP(refresh_lists(c, false));
+    WC_HIP(prepare_tiles(c));
     return enqueue_sort(c);
 }
 
@@ -1135,6 +1166,7 @@ WC_API int wc_profile_steps(wc_ctx* c, float dt, uint32_t nsteps, double ms_tota
     if (rc) return rc;
     rc = set_device(c);
     if (rc) return rc;
+    WC_HIP(prepare_tiles(c));
     const size_t nev = (size_t)nsteps * (WC_NUM_PASSES + 1);
     std::vector<hipEvent_t> ev(nev, nullptr);
     for (auto& e : ev)
@@ -1205,6 +1237,7 @@ WC_API int wc_set_tuning(wc_ctx* c, const wc_tuning* t) {
     c->density_variant = t->density_variant;
     c->update_variant = t->update_variant;
     c->neighbour_list = t->neighbour_list != 0;
+    c->tile_refused = false;
     drop_graph(c);
     return WC_OK;
 }
@@ -1238,6 +1271,8 @@ WC_API int wc_tune(wc_ctx* c, float dt, uint32_t reps, wc_tuning* chosen, double
     if (n > 0) {
         rc = ensure_neighbour_lists(c);
         if (rc) return rc;
+        c->tile_refused = false;
+        WC_HIP(ensure_tiles(c));
         // Keep buffer 1 (the state the caller sees); the passes below rewrite it.
         float4 *save_pos = nullptr, *save_vel = nullptr;
         WC_HIP(hipMalloc(&save_pos, n * sizeof(float4)));
@@ -1322,6 +1357,10 @@ WC_API int wc_tune(wc_ctx* c, float dt, uint32_t reps, wc_tuning* chosen, double
         restore();
         use(err == hipSuccess ? pick : before);
         drop_graph(c);
+        if (err == hipSuccess && c->tile_mem && c->density_variant != wc::tile_variant()) {
+            err = hipStreamSynchronize(c->stream);
+            release_tiles(c);
+        }
         if (err == hipSuccess) err = launch_sort(c, density_by_tiles(c), [](int) { return hipSuccess; });
         if (err == hipSuccess)
             err = density_by_tiles(c) ? launch_density_pass(c, true)
@@ -1833,6 +1872,7 @@ WC_API int wc_closure_run(wc_ctx* c, wc_mlp* net, float dt, uint32_t K, uint32_t
     // the network's own stream may still be writing its bf16 weights
     if (net) WC_HIP(hipStreamSynchronize(net->m.stream));
     float prev_max = 0.0f;
+    WC_HIP(prepare_tiles(c));
     rc = sort_density();
     if (!rc) rc = read_rho_max(c, &prev_max);
     stats->peak_density = prev_max / rho0;

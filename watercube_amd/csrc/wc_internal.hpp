@@ -189,8 +189,13 @@ constexpr uint32_t kListCount = 32;          // in another 128-byte line: atomic
 constexpr uint32_t kSceneSparse = 64;
 constexpr uint32_t kTileBlock = 256;         // threads, and at most that many boxes, per classification workgroup
 // Chunks of 64 lanes that lists are kept for.  Full boxes use 1.2 lanes a particle (columns are rounded to four
-// lanes, boxes to 64), a fluid that has spread up to 1.4; boxes past the memory search directly.
-inline uint64_t tile_list_chunks(uint64_t particles) { return particles / 32 + 1024; }
+// lanes, boxes to 64), a fluid that has spread up to 1.4; boxes past the memory search directly.  A staged box and its
+// halo hold over two particles a cell, at least 129, and a particle lies in the halos of at most 8: n / 16 boxes at most,
+// with at most n / 64 chunks and 1.75 for each.
+inline uint64_t tile_list_chunks(uint64_t particles) {
+    const uint64_t many = particles / 32 + 1024, few = particles / 6 + 16;
+    return many < few ? many : few;
+}
 constexpr size_t kTileTableBytes = 1824;     // cell table of a box
 // Entries a sort can list.  One per base tile; a box whose halo holds more than `cap` >= 1024 records
 // becomes boxes of 2x2x2 cells, then single cells, then chunks of at least 256 particles: every
