@@ -379,3 +379,24 @@ def test_buffers_follow_the_tuning(oracle):
         f.synchronize()
         assert np.array_equal(f.particles(1).view(np.uint32), st.buf1.view(np.uint32))
         check("after passes one by one")
+
+
+def test_kernel_terms_that_overflow(oracle):
+    """A pair without positive pressure adds nothing, also when the kernel's term overflows: the force pass by tiles adds 0
+    times that term, so contexts with such constants keep the other passes.  The oracle's bits."""
+    p, parts = scaled_block((20, 20, 20), 0.015, 5)
+    parts["position"] *= np.float32(100.0)
+    p.size, p.kernel_radius = 100.0, 3.0
+    L.derive(p)
+    p.particle_mass, p.rest_density, p.stiffness = 1.0, 1e6, 1.0  # every pressure negative
+    p.spiky_const = -3e38  # the nearest neighbours, 1.2 to 1.8 away: (3 - d)^2 times this is infinite
+    tile = L.lib().wc_num_variants() - 1
+    st = oracle.OracleState(p, parts)
+    st.step(1e-3, 2)
+    assert np.isfinite(st.buf1["velocity"]).all() and (st.buf1["pressure"] < 0).all()
+    print("case kernel term overflows", flush=True)
+    with Fluid(p, parts) as f:
+        f.set_tuning(tile, tile, 0)
+        f.step(1e-3, 2)
+        f.synchronize()
+        assert np.array_equal(f.particles(1).view(np.uint32), st.buf1.view(np.uint32))

@@ -190,13 +190,13 @@ int check_params(const wc_params* p) {
 constexpr uint64_t kTileMaxCellsPerParticle = 64;
 
 // Constants for which the tile passes' short force arithmetic has the reference's bits.  It halves the mass instead of
-// the pair pressure: exact for normal floats.  And a lane past its list adds its own record, every term of which has to
-// be 0 and not 0 times infinity: m p / rho stays finite up to m = 2^40 (p and rho lie in [2^-40, 2^40]), the kernel
-// terms while these are finite.
+// the pair pressure: exact for normal floats.  And it adds 0 times a kernel term where the reference skips a pair whose
+// pressure is not positive, and a lane past its list its own record: every term has to be finite.  m p / rho is up to
+// m = 2^40 (p and rho lie in [2^-40, 2^40]), the kernel terms while those of distance 0 are.
 bool short_arithmetic(const wc_params& p) {
     const float m = fabsf(p.particle_mass);
     return (m == 0.0f || (m >= 0x1p-100f && m <= 0x1p40f)) && p.kernel_radius <= 0x1p60f &&
-           isfinite(p.spiky_const) && isfinite(p.visc_const * p.kernel_radius);
+           isfinite(p.spiky_const * (p.kernel_radius * p.kernel_radius)) && isfinite(p.visc_const * p.kernel_radius);
 }
 
 std::vector<wc::SceneFill> scene_fills(const std::vector<wc_params>& scenes) {
