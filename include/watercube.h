@@ -171,11 +171,11 @@ WC_API int wc_density(wc_ctx* ctx);
 /* Fluid::runUpdateProg(buffer2, buffer1, dt) (src/core/Fluid.cpp:294-321): update.comp:134-232.
  * `dt` is the integration step itself (the reference passes frame time * time_scale_).  Reads
  * the densities and pressures of the preceding wc_density on the same sort, as the reference's
- * pass order does.  The sort and the density pass also check that every position is 0 or within
- * [2^-20, 2^20] in magnitude, and every velocity, density and pressure 0 or within [2^-40, 2^40];
- * when they are, the pass forms
- * each neighbour's quotients from shared reciprocals (same bits as IEEE division), otherwise,
- * and when no density pass followed the last sort, it divides as IEEE does. */
+ * pass order does.  The sort and the density pass also check that every position, velocity,
+ * density and pressure is 0 or within [2^-40, 2^40] in magnitude (positions by boxes of cells:
+ * [2^-20, 2^20]); when they are, the pass forms each neighbour's quotients from shared reciprocals
+ * (same bits as IEEE division), otherwise, and when no density pass followed the last sort, it
+ * divides as IEEE does. */
 WC_API int wc_update(wc_ctx* ctx, float dt);
 
 /* Fluid::runAdvectProg(buffer, time) (src/core/Fluid.cpp:326-336, advect.comp:20-59), whose call

@@ -1025,7 +1025,7 @@ __global__ __launch_bounds__(BLOCK) void k_density(Scenes S, float4* __restrict_
         reinterpret_cast<float*>(posrho)[4 * (size_t)t + 3] = density;
         reinterpret_cast<float*>(velp)[4 * (size_t)t + 3] = pressure;
         // the other operands of the force pass's quotients (the sort checks the velocities)
-        const bool ok = pos_operand(p.x) && pos_operand(p.y) && pos_operand(p.z) && div_operand(pressure) &&
+        const bool ok = div_operand(p.x) && div_operand(p.y) && div_operand(p.z) && div_operand(pressure) &&
                         div_operand(density) && density != 0.0f;
         if (!ok) atomicOr(&rho_max[1], kDivUnsafe);
     }
