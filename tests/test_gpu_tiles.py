@@ -1,10 +1,13 @@
 """The tile passes (the last tuning variant) against the oracle, bit for bit, at the edges of their boxes."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from watercube_amd import Fluid
 from watercube_amd import _lib as L
 from watercube_amd.scenes import scaled_block
+from watercube_amd.scenes import workload
 
 pytestmark = pytest.mark.gpu
 
@@ -128,8 +131,6 @@ def test_tile_passes_of_several_scenes_with_thin_boxes(oracle):
 def test_latency_of_an_empty_scene_is_zero(oracle):
     """The passes' leading work items are padded to a multiple of the XCD count.  Padding belongs to no scene: a scene
     without particles, the first one here, keeps a latency of 0."""
-    import ctypes as C
-
     from watercube_amd.batch import SceneBatch
 
     scenes = []
@@ -217,10 +218,6 @@ def test_mass_whose_half_is_not_exact(oracle):
 def test_neighbour_counts_are_those_of_the_last_listing_pass(sequence):
     """wc_get_neighbour_counts answers for the last density pass that ran in list mode, whatever ran after it: by tiles,
     whose steps leave the lists out until they are asked for, as by the per-particle passes."""
-    import ctypes as C
-
-    from watercube_amd.scenes import workload
-
     p, parts, dt, _ = workload("dam_break_16k")
     tile = L.lib().wc_num_variants() - 1
     steps = 20 + len(sequence)  # freed memory holds no other sequence's counts
@@ -292,8 +289,6 @@ def test_tuner_leaves_the_state_and_its_lists(per, oracle):
 
 def _held(make, count):
     """Bytes of GPU memory that `count` contexts made by make() hold, per context."""
-    import ctypes as C
-
     def free():  # the HIP runtime the library itself is linked with
         a, b = C.c_size_t(), C.c_size_t()
         assert L.lib().hipMemGetInfo(C.byref(a), C.byref(b)) == 0
@@ -345,8 +340,6 @@ def test_memory_of_contexts_without_the_tile_passes(case):
 def test_buffers_follow_the_tuning(oracle):
     """The tile passes' buffers come with the first sort that needs them, also after steps of other passes, a larger grid or
     a tuner's run: the oracle's bits throughout."""
-    import ctypes as C
-
     tile = L.lib().wc_num_variants() - 1
     p, parts = scaled_block((30, 31, 29), 0.02, 3)
     small, _ = scaled_block((30, 31, 29), 0.02, 3, 3.3)  # fewer cells, other boxes
@@ -400,3 +393,44 @@ def test_kernel_terms_that_overflow(oracle):
         f.step(1e-3, 2)
         f.synchronize()
         assert np.array_equal(f.particles(1).view(np.uint32), st.buf1.view(np.uint32))
+
+
+@pytest.mark.parametrize("scene,marks", [("block_1m", (100, 300, 500)), ("block_sphere_17m", (3, 20))])
+def test_tile_trajectory_of_the_large_scenes(scene, marks):
+    """The benchmark's scenes by the passes that they start on, whose lists hold 256 and 128 entries there, against the
+    per-particle passes with lists (which the 500-step comparison with the oracle pins): the same bits all the way."""
+    p, parts, dt, _ = workload(scene)
+    tile = L.lib().wc_num_variants() - 1
+    with Fluid(p, parts) as a, Fluid(p, parts) as b:
+        assert a.get_tuning()[:2] == (tile, tile)
+        a.set_tuning(tile, tile, 1)
+        b.set_tuning(4, 0, 1)
+        done = 0
+        for upto in marks:
+            print(f"case {scene}: steps {done}..{upto}", flush=True)
+            a.step(dt, upto - done)
+            b.step(dt, upto - done)
+            a.synchronize()
+            b.synchronize()
+            done = upto
+            x, y = a.particles(1).view(np.uint32), b.particles(1).view(np.uint32)
+            assert np.array_equal(x, y), f"{scene} after {done} steps: {int((x != y).sum())} words differ"
+
+
+def test_parameters_that_change_the_box_shape(oracle):
+    """wc_set_params between steps, with kernel radii whose rest density asks for other boxes each time (and back)."""
+    p, parts = scaled_block((40, 37, 41), 0.02, 8)
+    tile = L.lib().wc_num_variants() - 1
+    st = oracle.OracleState(p, parts)
+    with Fluid(p, parts) as f:
+        f.set_tuning(tile, tile, 0)
+        for ratio in (2.0, 2.7, 2.3, 3.5, 2.0):
+            print(f"case kernel radius {ratio}", flush=True)
+            q, _ = scaled_block((40, 37, 41), 0.02, 8, ratio)
+            L.check(L.lib().wc_set_params(f.ctx, C.byref(q)), "wc_set_params")
+            st = oracle.OracleState(q, st.buf1)
+            f.step(2e-5, 2)
+            st.step(2e-5, 2)
+            f.synchronize()
+            got = f.particles(1)
+            assert np.array_equal(got.view(np.uint32), st.buf1.view(np.uint32)), f"ratio {ratio}"
