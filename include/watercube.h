@@ -289,6 +289,7 @@ typedef struct wc_tuning {
     int32_t neighbour_list;
 } wc_tuning;
 WC_API int wc_num_variants(void);
+/* The choice that variant v stands for; all 0 for the last one, which is no particle per lane. */
 WC_API int wc_variant_info(int v, int32_t* block, int32_t* list_cap, int32_t* chunk, int32_t* plane_drain);
 WC_API int wc_get_tuning(const wc_ctx* ctx, wc_tuning* out);
 WC_API int wc_set_tuning(wc_ctx* ctx, const wc_tuning* tuning);

@@ -123,3 +123,11 @@ def test_tuner_candidates(exe):
     assert candidates(True, t) == [(1, 0, 0), (3, 3, 1)]
     t[0][1] = [0.3] * 3 + [0.03]
     assert candidates(True, t) == [(3, 3, 1)] and candidates(False, t) == [(0, 2, 1)]
+
+
+def test_descriptor_of_the_tile_variant():
+    """The last variant has no workgroup, list length and slots in flight of its own: none are reported."""
+    from watercube_amd import _lib as L
+
+    v = L.variants()
+    assert v[-1] == (0, 0, 0, 0) and all(b in (64, 128, 256) and c > 0 and k > 0 for b, c, k, _ in v[:-1])

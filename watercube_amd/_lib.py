@@ -228,7 +228,7 @@ def u32ptr(a: np.ndarray):
 
 def variants() -> list[tuple[int, int, int, int]]:
     """(threads per workgroup, LDS list entries per lane, slots in flight, per-plane drain) of
-    each variant of the neighbour passes."""
+    each variant of the neighbour passes ((0, 0, 0, 0): the last one, by boxes of cells)."""
     out = []
     for v in range(lib().wc_num_variants()):
         b, c, k, d = C.c_int32(), C.c_int32(), C.c_int32(), C.c_int32()

@@ -150,8 +150,7 @@ struct wc_ctx {
     void* tile_mem = nullptr;   // the tile passes' buffers, one allocation
     bool tile_refused = false;  // there was no room for them; asked again after wc_set_tuning, wc_tune, wc_set_params
     // What the last queued passes left in the buffers; a host upload or a parameter change clears all.
-    bool sorted_ok = false;  // buffer 2 holds the last sort's output, every slot in its cell's range
-    bool tiles_ok = false;   // ... and the work list is that sort's
+    bool tiles_ok = false;   // the work list is the last sort's, and buffer 2 still that sort's output
     bool llist_ok = false;   // the tiles' lists and counts are those of a density pass on that sort
     bool nlist_ok = false;   // nlist and ncount likewise
     // The last density pass in list mode ran by tiles and left nlist and ncount out; refresh_lists() forms them before
@@ -444,7 +443,6 @@ int particle_variant(int v) { return v == wc::tile_variant() ? 2 : v; }
 
 // What the buffers hold after a sort, and after the whole step of the current tuning.
 void note_sort(wc_ctx* c, bool tiles) {
-    c->sorted_ok = true;
     c->tiles_ok = tiles;
     c->llist_ok = c->nlist_ok = c->lists_owed = false;
 }
@@ -707,7 +705,7 @@ int copy_records_in(wc_ctx* c, uint32_t first, const wc_particle* host, uint32_t
         WC_HIP(wc::launch_split_records(c->staging + first, c->b.posrho[b] + first, c->b.velp[b] + first, n,
                                         c->stream));
     // buffer 2 changed under the last sort: its cell keys, neighbour lists and division check
-    c->sorted_ok = c->tiles_ok = c->llist_ok = c->nlist_ok = c->lists_owed = false;
+    c->tiles_ok = c->llist_ok = c->nlist_ok = c->lists_owed = false;
     WC_HIP(wc::launch_invalidate(c->b, c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
     return WC_OK;
@@ -938,7 +936,7 @@ WC_API int wc_set_params(wc_ctx* c, const wc_params* p) {
     rc = upload_tables(c);
     if (rc) return rc;
     // keys, lists and the division check of buffer 2 were formed with the old constants
-    c->sorted_ok = c->tiles_ok = c->llist_ok = c->nlist_ok = c->lists_owed = false;
+    c->tiles_ok = c->llist_ok = c->nlist_ok = c->lists_owed = false;
     WC_HIP(wc::launch_invalidate(c->b, c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
     return WC_OK;

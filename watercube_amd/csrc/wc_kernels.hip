@@ -2816,7 +2816,7 @@ static const PassVariant kVariants[] = {
 #define WC_ROW(B, C, K, P) {B, C, K, P},
     WC_VARIANTS(WC_ROW)
 #undef WC_ROW
-    {384, (int)kNeighbourListMax, 4, true},  // the tile passes (their workgroup and box vary with the context)
+    {0, 0, 0, false},  // the tile passes: no particle a lane, workgroup and lists by the context's box and size
 };
 
 int num_variants() { return (int)(sizeof(kVariants) / sizeof(kVariants[0])); }
