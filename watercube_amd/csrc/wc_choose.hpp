@@ -115,6 +115,16 @@ inline bool start_on_tiles(const std::vector<SceneFill>& scenes, const TileShape
     return n <= most;
 }
 
+// Boxes with at most this many records per cell of the box and its halo are not staged: their particles' slots go to
+// the list of sparse ones, which is searched directly.  A fluid that has spread over the cube, us a step of three contexts
+// at once, with no such line / 1.33 / 2 / 3 / 4 records: 192,089 particles at step 4,000 140 / 98 / 97 / 98 / 103 (105 by
+// the per-particle passes), a million at step 2,000 405 / 370 / 363 / 364 / 369 (467).  A block at its start has few thin
+// boxes, in its skin, and a context that does not fill the chip waits for their particles: by 2 / 3 (one context) 64,000
+// particles 73 / 100, 250,047 108 / 134, but 493,000 186 / 187, 704,969 270 / 272, a million 328 / 328.  A gas that fills
+// the cube, 2 / 3 / by variant 2: a million, two a cell 706 / 587 / 640, three a cell 705 / 667 / 689; 195,112, two a cell,
+// 189 / 162 / 175; 64,000 121 / 111 / 100.
+inline uint32_t sparse_records(uint64_t particles) { return particles >= 600000 ? 3u : 2u; }
+
 // The tuner's candidates from the times t[lists][pass][variant] of the density and force pass: the fastest pair without
 // neighbour lists, with them, and the last variant's (by tiles), whose passes run only with each other and form the same
 // lists in both modes.  Which of them it is, whole steps decide: the tile passes' sort also forms their work list and

@@ -306,13 +306,6 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(Scenes S, uint32_t* __res
 // Listed are the base boxes that hold particles.  One whose records with its halo exceed LDS is listed
 // as boxes of 2x2x2 cells, then as single cells, then as chunks of particles that search in HBM.
 // ------------------------------------------------------------------------------------------
-// Boxes with at most this many records per cell of the box and its halo are not staged: their particles' slots go
-// to T.sparse, which is searched directly.  A fluid that has spread over the cube, us a step of three contexts at
-// once, with no such line / 1.33 / 2 / 3 / 4 records: 192,089 particles at step 4,000 140 / 98 / 97 / 98 / 103 (105
-// by the per-particle passes), a million at step 2,000 405 / 370 / 363 / 364 / 369 (467), a gas of one particle a
-// cell 278 / 75 / 74 / 74 / 75 (77), of two 161 / 147 / 134 / 109 / 108 (98).  At its start, when only the block's
-// skin is that thin, its few particles lengthen the force pass (55 us to 78 at 2, 100 at 3).
-constexpr uint32_t kSparseRecords = 2;
 constexpr uint32_t kEntryDirect = 1u << 12;                 // particles searched for directly: e.w + i
 constexpr uint32_t kEntrySparse = 1u;                       // ... their slots at sparse[e.w + i]
 constexpr int kMaxBox = 4;                                  // cells per side of a box
@@ -2775,7 +2768,16 @@ static unsigned tile_grid(const DeviceBuffers& b) {
 
 static TileWork tile_work(const DeviceBuffers& b, const TileShape* t) {
     TileWork w{};
-    if (t) w = TileWork{b.tiles, b.tile_count, b.tile_cap, (uint32_t)t->cap, (uint32_t)t->block, b.tables, b.table_cap, b.sparse, kSparseRecords * (uint32_t)((t->x + 2) * (t->y + 2) * (t->z + 2))};
+    if (!t) return w;
+    w.tiles = b.tiles;
+    w.count = b.tile_count;
+    w.cap = b.tile_cap;
+    w.rec_cap = (uint32_t)t->cap;
+    w.chunk = (uint32_t)t->block;
+    w.tables = b.tables;
+    w.table_cap = b.table_cap;
+    w.sparse = b.sparse;
+    w.sparse_max = sparse_records(b.sc.total_particles) * (uint32_t)((t->x + 2) * (t->y + 2) * (t->z + 2));
     return w;
 }
 
