@@ -201,7 +201,8 @@ bool short_arithmetic(const wc_params& p) {
 std::vector<wc::SceneFill> scene_fills(const std::vector<wc_params>& scenes) {
     std::vector<wc::SceneFill> out;
     for (const wc_params& p : scenes)
-        out.push_back(wc::scene_fill(p.num_particles, p.grid_res, p.bin_size, p.kernel_radius, p.rest_density, p.particle_mass));
+        out.push_back(wc::scene_fill(p.num_particles, p.grid_res, p.bin_size, p.kernel_radius, p.rest_density,
+                                     p.particle_mass));
     return out;
 }
 
@@ -389,7 +390,8 @@ void release_tiles(wc_ctx* c) {
 }
 
 // The tile passes' buffers, allocated before the first sort that feeds those passes (a context that never runs them
-// holds none), and again if a change of parameters asks for more.  Not under capture.  tile_ok says whether they are there.
+// holds none), and again if a change of parameters asks for more.  Not under capture.  tile_ok says whether they are
+// there.
 hipError_t ensure_tiles(wc_ctx* c) {
     c->tile_ok = false;
     if (!c->tile_fit || c->tile_refused) return hipSuccess;
@@ -414,8 +416,8 @@ hipError_t ensure_tiles(wc_ctx* c) {
                            (void**)&b.sparse, (void**)&b.llist,      (void**)&b.lcount};
     size_t free_bytes = 0, total_bytes = 0, all = 0;
     for (size_t v : bytes) all += (v + 255) / 256 * 256;
-    if (entries > 0xFFFFFFFFull || hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess || all + n * 1024 > free_bytes ||
-        hipMalloc(&c->tile_mem, all) != hipSuccess) {
+    if (entries > 0xFFFFFFFFull || hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess ||
+        all + n * 1024 > free_bytes || hipMalloc(&c->tile_mem, all) != hipSuccess) {
         c->tile_mem = nullptr;
         c->tile_refused = true;
         (void)hipGetLastError();
@@ -491,13 +493,14 @@ hipError_t launch_density_pass(wc_ctx* c, bool lists) {
 }
 
 hipError_t launch_update_pass(wc_ctx* c) {
-    if (update_by_tiles(c) && c->llist_ok) return wc::launch_update_tile(c->b, c->tile_shape, wc::TileUpdate{}, c->stream);
+    if (update_by_tiles(c) && c->llist_ok)
+        return wc::launch_update_tile(c->b, c->tile_shape, wc::TileUpdate{}, c->stream);
     return wc::launch_update(c->b, particle_variant(c->update_variant), c->neighbour_list && c->nlist_ok, c->stream);
 }
 
 // nlist and ncount of the last density pass in list mode, if it left them out: the pass runs again on the same sort and
-// writes them (and the same densities).  `current`: for a reader in list mode that takes them for the current sort's, also
-// when that pass ran before list mode was switched on.
+// writes them (and the same densities).  `current`: for a reader in list mode that takes them for the current sort's,
+// also when that pass ran before list mode was switched on.
 hipError_t refresh_lists(wc_ctx* c, bool current) {
     if (!c->lists_owed && !(current && c->neighbour_list && c->llist_ok && !c->nlist_ok)) return hipSuccess;
     c->lists_owed = false;
@@ -1127,8 +1130,12 @@ WC_API int wc_scene_latency(wc_ctx* c, double* ms, uint32_t num_scenes) {
     return WC_OK;
 }
 
-WC_API int wc_get_counts(wc_ctx* c, uint32_t* host, uint32_t ncells) { return scene_cells(c, 0, host, nullptr, ncells); }
-WC_API int wc_get_offsets(wc_ctx* c, uint32_t* host, uint32_t ncells) { return scene_cells(c, 0, nullptr, host, ncells); }
+WC_API int wc_get_counts(wc_ctx* c, uint32_t* host, uint32_t ncells) {
+    return scene_cells(c, 0, host, nullptr, ncells);
+}
+WC_API int wc_get_offsets(wc_ctx* c, uint32_t* host, uint32_t ncells) {
+    return scene_cells(c, 0, nullptr, host, ncells);
+}
 WC_API int wc_scene_get_cells(wc_ctx* c, uint32_t scene, uint32_t* counts, uint32_t* offsets, uint32_t ncells) {
     return scene_cells(c, scene, counts, offsets, ncells);
 }
@@ -1390,7 +1397,8 @@ WC_API int wc_tune(wc_ctx* c, float dt, uint32_t reps, wc_tuning* chosen, double
 WC_API int wc_device_alloc(size_t bytes, void** out) {
     if (!out) return fail(WC_ERR_INVALID_ARG, "out is NULL");
     *out = nullptr;
-    if (hipMalloc(out, bytes ? bytes : 16) != hipSuccess) return fail(WC_ERR_NO_MEMORY, "hipMalloc of %zu bytes", bytes);
+    if (hipMalloc(out, bytes ? bytes : 16) != hipSuccess)
+        return fail(WC_ERR_NO_MEMORY, "hipMalloc of %zu bytes", bytes);
     return WC_OK;
 }
 WC_API int wc_device_free(void* p) {
@@ -1754,7 +1762,8 @@ WC_API int wc_closure_infer(wc_ctx* c, wc_mlp* net, float dt_mult, void* y_dev) 
 // The learned step's force pass: by tiles when their lists are there and no correction is averaged over
 // neighbours, else per particle.
 static hipError_t launch_learned_update(wc_ctx* c, const wc::TileUpdate& u, bool smooth) {
-    if (update_by_tiles(c) && c->llist_ok && !(smooth && u.corr)) return wc::launch_update_tile(c->b, c->tile_shape, u, c->stream);
+    if (update_by_tiles(c) && c->llist_ok && !(smooth && u.corr))
+        return wc::launch_update_tile(c->b, c->tile_shape, u, c->stream);
     return wc::launch_closure_update(c->b, u.dt, u.corr, u.corr_scale, u.acc_out, smooth, u.substeps,
                                      c->neighbour_list && c->nlist_ok, c->stream, u.backup);
 }

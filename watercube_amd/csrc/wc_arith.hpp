@@ -39,8 +39,8 @@ __device__ __forceinline__ float rcp_in_range(float x) {
     return fmaf(fmaf(-x, y, 1.0f), y, y);
 }
 
-// The tile passes' positions: those of 0 or of [2^-20, 2^20] in magnitude differ by 0 or at least 2^-43, so their squared
-// distances are 0 or in sqrt_in_range's range.
+// The tile passes' positions: those of 0 or of [2^-20, 2^20] in magnitude differ by 0 or at least 2^-43, so their
+// squared distances are 0 or in sqrt_in_range's range.
 __device__ __forceinline__ bool pos_operand(float x) {
     const uint32_t u = __float_as_uint(x) & 0x7fffffffu;
     return u == 0u || u - 0x35800000u <= 0x49800000u - 0x35800000u;

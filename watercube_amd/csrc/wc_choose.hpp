@@ -22,7 +22,9 @@ constexpr int kTileSmallBlock = 256, kTileSmallCap = 2304;
 
 // Neighbours a particle's list holds (16 bits each; particles with more search directly): dense clusters
 // have a few hundred; large contexts keep lists of half the size.
-inline uint32_t tile_list_cap(uint64_t particles) { return particles <= 500000 ? 512u : particles <= 4000000 ? 256u : 128u; }
+inline uint32_t tile_list_cap(uint64_t particles) {
+    return particles <= 500000 ? 512u : particles <= 4000000 ? 256u : 128u;
+}
 
 // What a scene's parameters say of its density.
 struct SceneFill {
@@ -46,10 +48,10 @@ inline SceneFill scene_fill(uint32_t n, int grid_res, double bin, double h, doub
 // denser one is split) and leave the chip's 256 CUs enough boxes each.  At 8 particles a cell the whole step took, by
 // 4x3x4 / 4x2x4 / 2x2x4 (us): 91,125 particles 141 / 130 / 104, 125,000 126 / 137 / 137, 262,144 141 / 158 / 176: the
 // first from 300 boxes of it.  At 12 a cell, where it does not fit, by 4x2x4 / 2x2x4: 125,000 182 / 135, 192,089 (once
-// spread, three at once) 94 / 111, 2,048,000 1,087 / 1,109: the second from 450 boxes.  Up to 16 a cell 2x2x4 otherwise.
-// Above, where a box of it has more particles than threads, by 2x2x4 / 2x2x2: 59,319 (20 a cell) 192 / 143, 125,000
-// (20) 249 / 234, 343,000 (19) 553 / 542, 704,969 (17) 969 / 1,071, 1,000,000 (19) 1,321 / 1,388, 4,492,125 (19)
-// 5,762 / 6,093: 2x2x2 below 2,000 boxes of 2x2x4.
+// spread, three at once) 94 / 111, 2,048,000 1,087 / 1,109: the second from 450 boxes.  Up to 16 a cell 2x2x4
+// otherwise. Above, where a box of it has more particles than threads, by 2x2x4 / 2x2x2: 59,319 (20 a cell) 192 / 143,
+// 125,000 (20) 249 / 234, 343,000 (19) 553 / 542, 704,969 (17) 969 / 1,071, 1,000,000 (19) 1,321 / 1,388, 4,492,125
+// (19) 5,762 / 6,093: 2x2x2 below 2,000 boxes of 2x2x4.
 inline TileShape choose_tile_shape(const std::vector<SceneFill>& scenes) {
     double n = 0.0, cell = 0.0;
     for (const SceneFill& f : scenes) {
@@ -65,7 +67,8 @@ inline TileShape choose_tile_shape(const std::vector<SceneFill>& scenes) {
                   {{2, 2, 4, kTileSmallBlock, kTileSmallCap}, 2000.0}};
     for (const auto& s : shapes) {
         const TileShape& t = s.t;
-        if ((t.x + 2) * (t.y + 2) * (t.z + 2) * cell * 1.05 <= t.cap && n >= s.boxes * (t.x * t.y * t.z) * cell) return t;
+        if ((t.x + 2) * (t.y + 2) * (t.z + 2) * cell * 1.05 <= t.cap && n >= s.boxes * (t.x * t.y * t.z) * cell)
+            return t;
     }
     return {2, 2, 16.0 * cell <= kTileSmallBlock ? 4 : 2, kTileSmallBlock, kTileSmallCap};
 }
@@ -78,14 +81,14 @@ inline TileShape choose_tile_shape(const std::vector<SceneFill>& scenes) {
 constexpr uint32_t kTileMinParticles = 50000, kTileMinPerScene = 20000;
 
 // Whether a context starts with the tile passes.  Beside the sizes above they need, for nine tenths of the particles,
-// boxes that fit LDS, and lists that hold the neighbours: what does not fit is searched for one particle at a time, from
-// HBM.  A step by tiles / by variant 2 (us): boxes that do not fit, 64,000 particles (46 a cell) 625 / 512, 250,047 (46)
-// 1,833 / 919, (104) 5,111 / 2,246; lists that do not, 1,000,000 (268 neighbours, 256 entries) 30,502 / 4,372, 4,492,125
-// (151, 128 entries) 141,144 / 10,523.
+// boxes that fit LDS, and lists that hold the neighbours: what does not fit is searched for one particle at a time,
+// from HBM.  A step by tiles / by variant 2 (us): boxes that do not fit, 64,000 particles (46 a cell) 625 / 512,
+// 250,047 (46) 1,833 / 919, (104) 5,111 / 2,246; lists that do not, 1,000,000 (268 neighbours, 256 entries) 30,502 /
+// 4,372, 4,492,125 (151, 128 entries) 141,144 / 10,523.
 //
 // Where both fit, by occupancy.  Up to 16 a cell they gain at any size (343,000 particles, 15.6 a cell, 423 / 552;
-// 1,000,000, 14.7, 1,014 / 1,069; 4,492,125, 14.8, 4,097 / 4,343).  Above, lanes of a workgroup idle; with a kernel radius
-// of the cell's side, or (r) of 0.84 of it, where less of that work finds neighbours:
+// 1,000,000, 14.7, 1,014 / 1,069; 4,492,125, 14.8, 4,097 / 4,343).  Above, lanes of a workgroup idle; with a kernel
+// radius of the cell's side, or (r) of 0.84 of it, where less of that work finds neighbours:
 //   16 to 20:    343,000 (17) 537 / 586, but 704,969 (17) 972 / 954, 2,000,376 (17) 2,694 / 2,324
 //                r: 1,481,544 (17) 1,136 / 1,270, but 2,985,984 (19) 2,653 / 2,579
 //   20 to 22.5:  1,000,000 (21) 1,278 / 1,396, but 2,000,376 (21) 2,645 / 2,546
@@ -116,20 +119,20 @@ inline bool start_on_tiles(const std::vector<SceneFill>& scenes, const TileShape
 }
 
 // Boxes with at most this many records per cell of the box and its halo are not staged: their particles' slots go to
-// the list of sparse ones, which is searched directly.  A fluid that has spread over the cube, us a step of three contexts
-// at once, with no such line / 1.33 / 2 / 3 / 4 records: 192,089 particles at step 4,000 140 / 98 / 97 / 98 / 103 (105 by
-// the per-particle passes), a million at step 2,000 405 / 370 / 363 / 364 / 369 (467).  A block at its start has few thin
-// boxes, in its skin, and a context that does not fill the chip waits for their particles: by 2 / 3 (one context) 64,000
-// particles 73 / 100, 250,047 108 / 134, but 493,000 186 / 187, 704,969 270 / 272, a million 328 / 328.  A gas that fills
-// the cube, 2 / 3 / by variant 2: a million, two a cell 706 / 587 / 640, three a cell 705 / 667 / 689; 195,112, two a cell,
-// 189 / 162 / 175; 64,000 121 / 111 / 100.
+// the list of sparse ones, which is searched directly.  A fluid that has spread over the cube, us a step of three
+// contexts at once, with no such line / 1.33 / 2 / 3 / 4 records: 192,089 particles at step 4,000 140 / 98 / 97 / 98 /
+// 103 (105 by the per-particle passes), a million at step 2,000 405 / 370 / 363 / 364 / 369 (467).  A block at its
+// start has few thin boxes, in its skin, and a context that does not fill the chip waits for their particles: by 2 / 3
+// (one context) 64,000 particles 73 / 100, 250,047 108 / 134, but 493,000 186 / 187, 704,969 270 / 272, a million 328 /
+// 328.  A gas that fills the cube, 2 / 3 / by variant 2: a million, two a cell 706 / 587 / 640, three a cell 705 / 667
+// / 689; 195,112, two a cell, 189 / 162 / 175; 64,000 121 / 111 / 100.
 inline uint32_t sparse_records(uint64_t particles) { return particles >= 600000 ? 3u : 2u; }
 
 // The tuner's candidates from the times t[lists][pass][variant] of the density and force pass: the fastest pair without
-// neighbour lists, with them, and the last variant's (by tiles), whose passes run only with each other and form the same
-// lists in both modes.  Which of them it is, whole steps decide: the tile passes' sort also forms their work list and
-// tables (a million particles 20 us, 17.8 million 0.28 ms), and a pass timed alone finds its data in the caches.  Left out
-// are candidates too far behind for either (times in ms).
+// neighbour lists, with them, and the last variant's (by tiles), whose passes run only with each other and form the
+// same lists in both modes.  Which of them it is, whole steps decide: the tile passes' sort also forms their work list
+// and tables (a million particles 20 us, 17.8 million 0.28 ms), and a pass timed alone finds its data in the caches.
+// Left out are candidates too far behind for either (times in ms).
 struct TuningPick {
     int density, update;
     bool lists;

@@ -175,7 +175,8 @@ int tile_variant();
 struct TileWork {
     uint4* tiles;     // work list
     // its entries; [1]: slots in `sparse` of a single scene; [kListCount]: list chunks; with several scenes,
-    // [kSceneSparse + s]: scene s's slots in `sparse` (from its first particle on), [kSceneSparse - 1]: entries of those
+    // [kSceneSparse + s]: scene s's slots in `sparse` (from its first particle on), [kSceneSparse - 1]: entries of
+    // those
     uint32_t* count;
     uint32_t cap;
     uint32_t rec_cap;  // records a box may stage
@@ -188,9 +189,9 @@ struct TileWork {
 constexpr uint32_t kListCount = 32;          // in another 128-byte line: atomics on one line serialise
 constexpr uint32_t kSceneSparse = 64;
 constexpr uint32_t kTileBlock = 256;         // threads, and at most that many boxes, per classification workgroup
-// Chunks of 64 lanes that lists are kept for.  Full boxes use 1.2 lanes a particle (columns are rounded to four
-// lanes, boxes to 64), a fluid that has spread up to 1.4; boxes past the memory search directly.  A staged box and its
-// halo hold over two particles a cell, at least 129, and a particle lies in the halos of at most 8: n / 16 boxes at most,
+// Chunks of 64 lanes that lists are kept for.  Full boxes use 1.2 lanes a particle (columns are rounded to four lanes,
+// boxes to 64), a fluid that has spread up to 1.4; boxes past the memory search directly.  A staged box and its halo
+// hold over two particles a cell, at least 129, and a particle lies in the halos of at most 8: n / 16 boxes at most,
 // with at most n / 64 chunks and 1.75 for each.
 inline uint64_t tile_list_chunks(uint64_t particles) {
     const uint64_t many = particles / 32 + 1024, few = particles / 6 + 16;

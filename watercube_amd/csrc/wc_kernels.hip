@@ -326,7 +326,8 @@ __device__ __forceinline__ uint2 row_slots(const SceneDesc& d, const uint2* __re
                                            int z) {
     const int R = d.c.R;
     const uint2* row = range + d.c_off + ((size_t)z * R + y) * R;
-    const uint2 a = cell_range_in(row, (uint32_t)x0, d.p_off, d.c.n), b = cell_range_in(row, (uint32_t)x1, d.p_off, d.c.n);
+    const uint2 a = cell_range_in(row, (uint32_t)x0, d.p_off, d.c.n);
+    const uint2 b = cell_range_in(row, (uint32_t)x1, d.p_off, d.c.n);
     const uint32_t end = b.x + b.y;
     return make_uint2(a.x, end > a.x ? end - a.x : 0u);
 }
@@ -345,14 +346,15 @@ __device__ __forceinline__ uint32_t box_chunks(uint32_t particles, int nx, int n
 }
 
 __device__ __forceinline__ uint4 box_entry(int x, int y, int z, int nx, int ny, int nz, uint32_t s, uint32_t chunk) {
-    return make_uint4((uint32_t)x | (uint32_t)y << 10 | (uint32_t)z << 20, (uint32_t)nx | (uint32_t)ny << 4 | (uint32_t)nz << 8,
+    return make_uint4((uint32_t)x | (uint32_t)y << 10 | (uint32_t)z << 20,
+                      (uint32_t)nx | (uint32_t)ny << 4 | (uint32_t)nz << 8,
                       s, chunk);
 }
 
 // A box of at most 2x2x2 cells that does not fit LDS: its cells one by one, or a cell's particles in
 // chunks (one thread's work; dense clusters only).
-__device__ __forceinline__ void list_cells(const SceneDesc& d, const uint2* __restrict__ range, int x, int y, int z, int nx,
-                                           int ny, int nz, uint32_t s, const TileWork& T,
+__device__ __forceinline__ void list_cells(const SceneDesc& d, const uint2* __restrict__ range, int x, int y, int z,
+                                           int nx, int ny, int nz, uint32_t s, const TileWork& T,
                                            uint32_t* __restrict__ error_flag) {
     const int R = d.c.R;
 #pragma unroll 1
@@ -370,7 +372,8 @@ __device__ __forceinline__ void list_cells(const SceneDesc& d, const uint2* __re
                         all += row_slots(d, range, max(i - 1, 0), min(i + 2, R) - 1, cy, cz).y;
                 }
                 if (all <= T.rec_cap) {
-                    list_tile(T, error_flag, box_entry(i, j, k, 1, 1, 1, s, atomicAdd(T.count + kListCount, box_chunks(slots.y, 1, 1))));
+                    const uint32_t chunk = atomicAdd(T.count + kListCount, box_chunks(slots.y, 1, 1));
+                    list_tile(T, error_flag, box_entry(i, j, k, 1, 1, 1, s, chunk));
                 } else {
                     for (uint32_t a = 0; a < slots.y; a += T.chunk)
                         list_tile(T, error_flag,
@@ -422,8 +425,8 @@ __device__ __forceinline__ void classify_boxes(const Scenes& S, const uint2* __r
         for (uint32_t u = 0; u < 4; ++u) {
             const uint32_t k = k0 + u * (kTileBlock / LANES);
             origin(first + k, x, y, z);
-            rec[u] = box_records_by<LANES>(d, range, (int)(threadIdx.x % LANES), k < S.tper && first + k < d.ntiles, x, y, z,
-                                           bx, by, bz);
+            rec[u] = box_records_by<LANES>(d, range, (int)(threadIdx.x % LANES), k < S.tper && first + k < d.ntiles,
+                                           x, y, z, bx, by, bz);
         }
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u) {
@@ -449,7 +452,8 @@ __device__ __forceinline__ void classify_boxes(const Scenes& S, const uint2* __r
     }
     if (lane == 63) s_wave[wave] = make_uint3((uint32_t)__popcll(m), incl, lists_incl);
     __syncthreads();
-    uint32_t before = 0, listed = 0, sparse = 0, sparse_before = incl - take, chunk = lists_incl - lists, list_chunks = 0;
+    uint32_t before = 0, listed = 0, sparse = 0, list_chunks = 0;
+    uint32_t sparse_before = incl - take, chunk = lists_incl - lists;
     for (unsigned w = 0; w < kTileBlock / 64; ++w) {
         before += w < wave ? s_wave[w].x : 0u;
         sparse_before += w < wave ? s_wave[w].y : 0u;
@@ -464,7 +468,8 @@ __device__ __forceinline__ void classify_boxes(const Scenes& S, const uint2* __r
         const unsigned long long add = (unsigned long long)(one ? sparse : 0u) << 32 | listed;
         const unsigned long long old = add ? atomicAdd(reinterpret_cast<unsigned long long*>(T.count), add) : 0ull;
         s_base.x = (uint32_t)old;
-        s_base.y = one ? (uint32_t)(old >> 32) : (sparse ? d.p_off + atomicAdd(T.count + kSceneSparse + s, sparse) : 0u);
+        s_base.y = one ? (uint32_t)(old >> 32)
+                       : (sparse ? d.p_off + atomicAdd(T.count + kSceneSparse + s, sparse) : 0u);
     }
     if (threadIdx.x == 64) s_base.z = list_chunks ? atomicAdd(T.count + kListCount, list_chunks) : 0u;
     if (threadIdx.x < S.tper) s_rec[threadIdx.x] = make_uint2(few ? 0x80000000u | sparse_before : rec.x, rec.y);
@@ -512,14 +517,17 @@ __device__ __forceinline__ void classify_boxes(const Scenes& S, const uint2* __r
             const int q = q0 + (int)(lane / 16u);
             const int i = x + q % px * 2, j = y + q / px % py * 2, l = z + q / (px * py) * 2;
             // a part ends with its box
-            const int ex = min(min(2, x + bx - i), R - i), ey = min(min(2, y + by - j), R - j), ez = min(min(2, z + bz - l), R - l);
+            const int ex = min(min(2, x + bx - i), R - i), ey = min(min(2, y + by - j), R - j);
+            const int ez = min(min(2, z + bz - l), R - l);
             const bool any = q < parts && ex > 0 && ey > 0 && ez > 0;
             const uint2 part = box_records_by<16>(d, range, (int)(lane % 16u), any, i, j, l, ex, ey, ez);
             if (lane % 16u == 0 && part.x != 0) {
-                if (part.y <= T.rec_cap)
-                    list_tile(T, error_flag, box_entry(i, j, l, ex, ey, ez, s, atomicAdd(T.count + kListCount, box_chunks(part.x, ex, ey))));
-                else
+                if (part.y <= T.rec_cap) {
+                    const uint32_t chunk = atomicAdd(T.count + kListCount, box_chunks(part.x, ex, ey));
+                    list_tile(T, error_flag, box_entry(i, j, l, ex, ey, ez, s, chunk));
+                } else {
                     list_cells(d, range, i, j, l, ex, ey, ez, s, T, error_flag);
+                }
             }
         }
     }
@@ -561,7 +569,9 @@ __device__ __forceinline__ Box box_of(const uint4& e) {
 }
 
 // i / d for i < 256, d <= 36
-__device__ __forceinline__ int small_div(int i, int d) { return (int)((uint32_t)i * (uint32_t)((65536 + d - 1) / d) >> 16); }
+__device__ __forceinline__ int small_div(int i, int d) {
+    return (int)((uint32_t)i * (uint32_t)((65536 + d - 1) / d) >> 16);
+}
 
 // Halo cell (x fastest) i of a box, as its index in the table (z fastest).
 __device__ __forceinline__ int table_cell(const Box& b, int i) {
@@ -596,7 +606,8 @@ __device__ __forceinline__ void box_lanes(BoxShared& sh, const Box& b) {
 // Cell table of a box: every thread takes a halo cell (out-of-grid cells are empty), a prefix sum over the
 // counts gives each its records in LDS.  BLOCK threads take ceil(216 / BLOCK) cells each, in order.
 template <int BLOCK>
-__device__ __forceinline__ void box_cells(BoxShared& sh, const Box& b, const SceneDesc& d, const uint2* __restrict__ range) {
+__device__ __forceinline__ void box_cells(BoxShared& sh, const Box& b, const SceneDesc& d,
+                                          const uint2* __restrict__ range) {
     constexpr int kPer = (kMaxCells + BLOCK - 1) / BLOCK;
     const int tid = threadIdx.x, ncell = b.hx * b.hy * b.hz, R = d.c.R;
     const unsigned lane = lane_id(), wave = threadIdx.x >> 6;
@@ -659,8 +670,9 @@ __device__ __forceinline__ void form_tables(const Scenes& S, const uint2* __rest
             const uint32_t n = min(T.count[kSceneSparse + s], d.c.n), chunks = (n + T.chunk - 1) / T.chunk;
             const uint32_t at = chunks ? atomicAdd(T.count + kSceneSparse - 1, chunks) : 0u;
             for (uint32_t k = 0; k < chunks && at + k < T.cap; ++k)
-                T.tiles[T.cap - 1u - at - k] = make_uint4(0u, kEntryDirect | kEntrySparse | min(T.chunk, n - k * T.chunk) << 13,
-                                                          s, d.p_off + k * T.chunk);
+                T.tiles[T.cap - 1u - at - k] =
+                    make_uint4(0u, kEntryDirect | kEntrySparse | min(T.chunk, n - k * T.chunk) << 13, s,
+                               d.p_off + k * T.chunk);
         }
     }
     for (uint32_t item = block; item < listed; item += nblocks) {
@@ -834,7 +846,8 @@ __global__ __launch_bounds__(kHashBlock) void k_gather(Scenes S, uint32_t* __res
                                                        const float4* __restrict__ velp_in,
                                                        float4* __restrict__ posrho_out, float4* __restrict__ velp_out,
                                                        uint32_t* __restrict__ sorted, uint32_t* __restrict__ skey,
-                                                       const uint32_t* __restrict__ id_in, uint32_t* __restrict__ id_out,
+                                                       const uint32_t* __restrict__ id_in,
+                                                       uint32_t* __restrict__ id_out,
                                                        uint32_t* __restrict__ div_flags,
                                                        const uint2* __restrict__ crowd,
                                                        const uint32_t* __restrict__ crowd_count, uint32_t crowd_cap,
@@ -1159,8 +1172,8 @@ struct ForceSums {
     // The same sums with the square root and the reciprocals in their short forms: every operand
     // passes div_operand (positions pos_operand), so each step rounds as in add.  The pair pressure is
     // half the quotient by rho_j, exactly, and the half goes into the mass (a power of two).
-    __device__ __forceinline__ void add_in_range(const StepConsts& c, const float4& p, const float4& pv, const float4& q,
-                                                 const float4& qv) {
+    __device__ __forceinline__ void add_in_range(const StepConsts& c, const float4& p, const float4& pv,
+                                                 const float4& q, const float4& qv) {
         const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
         const float dist = sqrt_in_range((rx * rx + ry * ry) + rz * rz);
         const float iw = rcp_in_range(q.w);
@@ -1447,8 +1460,9 @@ __global__ __launch_bounds__(BLOCK) void k_update(Scenes S, const float4* __rest
 // ------------------------------------------------------------------------------------------
 // The box's table into sh: as k_gather formed it, or formed here for entries past its memory.
 template <int BLOCK>
-__device__ __forceinline__ void box_open(BoxShared& sh, const Box& b, const SceneDesc& d, const uint2* __restrict__ range,
-                                         const BoxTable* __restrict__ tables, uint32_t item, uint32_t table_cap) {
+__device__ __forceinline__ void box_open(BoxShared& sh, const Box& b, const SceneDesc& d,
+                                         const uint2* __restrict__ range, const BoxTable* __restrict__ tables,
+                                         uint32_t item, uint32_t table_cap) {
     if (threadIdx.x == 0) sh.rho = 0u;
     if (item < table_cap) {  // workgroup-uniform
         for (uint32_t k = threadIdx.x; k < sizeof(BoxTable) / 16; k += BLOCK)
@@ -1494,7 +1508,8 @@ __device__ __forceinline__ uint4 tile_item(const TileItems& t, const uint4* __re
 // x side by side, with up to 16 records of kFlight cells in flight.  The table is read where box_open reads it,
 // without waiting for sh.
 template <int BLOCK, typename Load, typename Store>
-__device__ __forceinline__ void box_stage_from(const Box& b, const BoxTable* table, uint32_t cap, Load load, Store store) {
+__device__ __forceinline__ void box_stage_from(const Box& b, const BoxTable* table, uint32_t cap, Load load,
+                                               Store store) {
     constexpr int kFlight = 3, kGroups = BLOCK / 8;
     const uint32_t sub = threadIdx.x & 7u;
     const int ncell = b.hx * b.hy * b.hz;
@@ -1574,12 +1589,12 @@ __device__ __forceinline__ BoxLane box_lane(const BoxShared& sh, const Box& b, u
 // column of cells along z, so their candidates in a neighbouring column lie in one window of three or
 // four cells (more where cells hold fewer than four).
 //
-// Rounding, in units of bin^2: |a'_k| and |b_k - o_k| are at most 3 (boxes with a particle further out search directly), o
-// lies in the grid of R cells a side, so |b_k| <= R + 3, whatever the cube's `size` is.  n_a and n_b are at most 27,
-// 2 sum a'_k o_k and the three products 18 R and 18 (R + 3), and a cutoff over 108 accepts every pair.  So no partial sum
-// exceeds 18 R + 220, and with the inputs' own rounding the sum errs by less than 2^-24 (144 R + 2,010) < 1.2e-5 (R + 10):
-// with that margin the marked candidates are a superset of the accepted ones (measured: 0.2 of it at most), and the drain
-// applies the exact test.
+// Rounding, in units of bin^2: |a'_k| and |b_k - o_k| are at most 3 (boxes with a particle further out search
+// directly), o lies in the grid of R cells a side, so |b_k| <= R + 3, whatever the cube's `size` is.  n_a and n_b are
+// at most 27, 2 sum a'_k o_k and the three products 18 R and 18 (R + 3), and a cutoff over 108 accepts every pair.  So
+// no partial sum exceeds 18 R + 220, and with the inputs' own rounding the sum errs by less than 2^-24 (144 R + 2,010)
+// < 1.2e-5 (R + 10): with that margin the marked candidates are a superset of the accepted ones (measured: 0.2 of it at
+// most), and the drain applies the exact test.
 //
 // A lane appends its marked candidates to its list in enumeration order: cells in NEIGHBORHOOD order,
 // candidates in slot order.
@@ -1672,7 +1687,8 @@ __global__ __launch_bounds__(BLOCK, WPE) void k_density_tile(Scenes S, const uin
                                                         const uint32_t* __restrict__ skey,
                                                         const uint2* __restrict__ range, uint32_t* __restrict__ rho_max,
                                                         uint16_t* __restrict__ llist, uint16_t* __restrict__ lcount,
-                                                        uint32_t list_cap, uint32_t list_chunks, uint32_t* __restrict__ nlist,
+                                                        uint32_t list_cap, uint32_t list_chunks,
+                                                        uint32_t* __restrict__ nlist,
                                                         uint32_t* __restrict__ ncount) {
     constexpr uint32_t kFar = CAP + kPosPad;
     __shared__ float4 s_pos[CAP + kPosPad + 1];
@@ -1726,7 +1742,9 @@ __global__ __launch_bounds__(BLOCK, WPE) void k_density_tile(Scenes S, const uin
             if (threadIdx.x == 0) sh.rho = 0u;
             __syncthreads();
             using Entry = typename std::conditional<GLOBAL, uint32_t, float>::type;
-            constexpr int kFit = (int)(sizeof(float4) * CAP / (BLOCK * sizeof(Entry))), kDirectCap = kFit < 40 ? kFit : 40;  // the search's lists take the records' place
+            // the search's lists take the records' place
+            constexpr int kFit = (int)(sizeof(float4) * CAP / (BLOCK * sizeof(Entry)));
+            constexpr int kDirectCap = kFit < 40 ? kFit : 40;
             const lds_ptr<Entry> found = (lds_ptr<Entry>)reinterpret_cast<Entry*>(s_pos) + threadIdx.x;
             for (uint32_t i = threadIdx.x; i < e.y >> 13; i += BLOCK) {
                 const uint32_t t = e.y & kEntrySparse ? sparse[min(e.w + i, S.total_particles - 1u)] : e.w + i;
@@ -1762,7 +1780,8 @@ __global__ __launch_bounds__(BLOCK, WPE) void k_density_tile(Scenes S, const uin
             const float reach = 3.001f * c.bin;
             bool bad = false;
             box_stage<BLOCK>(
-                sh, b, tables, at_list, table_cap, CAP, [&](uint32_t slot) { return posrho[min(slot, d.p_off + c.n - 1u)]; },
+                sh, b, tables, at_list, table_cap, CAP,
+                [&](uint32_t slot) { return posrho[min(slot, d.p_off + c.n - 1u)]; },
                 [&](uint32_t at, float4 q, uint32_t slot) {
                     const float x = q.x - ox, y = q.y - oy, z = q.z - oz;
                     bad |= !(fabsf(x) <= reach && fabsf(y) <= reach && fabsf(z) <= reach && pos_operand(q.x) &&
@@ -1783,7 +1802,8 @@ __global__ __launch_bounds__(BLOCK, WPE) void k_density_tile(Scenes S, const uin
             for (uint32_t ch = (uint32_t)wave; ch * 64u < lanes; ch += BLOCK / 64) {
                 const BoxLane L = box_lane(sh, b, ch * 64u + lane_id(), d);
                 const float4 p = s_pos[L.idx];
-                char* const list = reinterpret_cast<char*>(llist) + (size_t)(e.w + ch) * (list_cap * 128u) + lane_id() * 2u;
+                char* const list =
+                    reinterpret_cast<char*>(llist) + (size_t)(e.w + ch) * (list_cap * 128u) + lane_id() * 2u;
                 uint32_t cnt = list_cap + 1u;  // no list: as an overflowed one
                 if (listable) {                // workgroup-uniform
                     const float ax = p.x - ox, ay = p.y - oy, az = p.z - oz;
@@ -1891,7 +1911,8 @@ __global__ __launch_bounds__(BLOCK, WPE) void k_update_tile(Scenes S, const uint
                                                        float4* __restrict__ velp_out,
                                                        unsigned long long* __restrict__ scene_done,
                                                        const uint32_t* __restrict__ id_sorted,
-                                                       uint32_t* __restrict__ id_out, const uint16_t* __restrict__ llist,
+                                                       uint32_t* __restrict__ id_out,
+                                                       const uint16_t* __restrict__ llist,
                                                        const uint16_t* __restrict__ lcount, uint32_t list_cap,
                                                        uint32_t list_chunks,
                                                        const uint32_t* __restrict__ div_flags, float dt_arg,
@@ -1937,8 +1958,8 @@ __global__ __launch_bounds__(BLOCK, WPE) void k_update_tile(Scenes S, const uint
                     const float4 ct = corr[t];
                     kc = V3{ct.x, ct.y, ct.z};
                 }
-                learned_integrate(c, f, ext, denom, p, pv, t, dt_arg, substeps, corr != nullptr, kc, corr_scale, acc_out,
-                                  po, vo);
+                learned_integrate(c, f, ext, denom, p, pv, t, dt_arg, substeps, corr != nullptr, kc, corr_scale,
+                                  acc_out, po, vo);
             }
             po.w = p.w;
             vo.w = pv.w;
@@ -1965,7 +1986,9 @@ __global__ __launch_bounds__(BLOCK, WPE) void k_update_tile(Scenes S, const uint
             finish(t, p, pv, f);
         };
         if (e.y & kEntryDirect) {
-            constexpr int kFit = (int)(2 * sizeof(float4) * CAP / (BLOCK * sizeof(uint32_t))), kDirectCap = kFit < 40 ? kFit : 40;  // the search's lists take the records' place
+            // the search's lists take the records' place
+            constexpr int kFit = (int)(2 * sizeof(float4) * CAP / (BLOCK * sizeof(uint32_t)));
+            constexpr int kDirectCap = kFit < 40 ? kFit : 40;
             const lds_ptr<uint32_t> found = (lds_ptr<uint32_t>)reinterpret_cast<uint32_t*>(s_rec) + threadIdx.x;
             for (uint32_t i = threadIdx.x; i < e.y >> 13; i += BLOCK) {
                 const uint32_t t = e.y & kEntrySparse ? sparse[min(e.w + i, S.total_particles - 1u)] : e.w + i;
@@ -2343,7 +2366,8 @@ __device__ __forceinline__ void select_by_threshold(uint32_t t, uint32_t m, uint
     }
     uint4* row = reinterpret_cast<uint4*>(sel_out + (size_t)t * kClosureNeighbours);
 #pragma unroll
-    for (int j = 0; j < kClosureNeighbours / 4; ++j) row[j] = make_uint4(u[4 * j], u[4 * j + 1], u[4 * j + 2], u[4 * j + 3]);
+    for (int j = 0; j < kClosureNeighbours / 4; ++j)
+        row[j] = make_uint4(u[4 * j], u[4 * j + 1], u[4 * j + 2], u[4 * j + 3]);
 }
 
 // The kClosureNeighbours nearest of the m listed neighbours of slot t, kSelRegCap < m <=
@@ -2361,7 +2385,8 @@ __device__ __forceinline__ void select_by_threshold(uint32_t t, uint32_t m, uint
 //   in the row's spare last word); the row's kClosureNeighbours words then go out as 16-byte
 //   stores, one 128-byte line.
 constexpr int kSelStageWords = kClosureNeighbours + 1;  // per lane: odd, so lanes' rows fall in different banks
-__device__ __forceinline__ void select_by_bisection(uint32_t t, uint32_t m, uint32_t n, const float4* __restrict__ posrho,
+__device__ __forceinline__ void select_by_bisection(uint32_t t, uint32_t m, uint32_t n,
+                                                    const float4* __restrict__ posrho,
                                                     const uint32_t* __restrict__ nlist, size_t stride,
                                                     uint32_t* __restrict__ sel_out, lds_ptr<uint32_t> stage) {
     constexpr int CAP = (int)kNeighbourListMax, kGroup = 4, kGroups = CAP / kGroup;  // 64 keys held: smaller groups
@@ -2784,8 +2809,9 @@ static TileWork tile_work(const DeviceBuffers& b, const TileShape* t) {
 hipError_t launch_place(const DeviceBuffers& b, const TileShape* tiles, hipStream_t s) {
     if (b.sc.blocks256 == 0) return hipSuccess;
     const unsigned extra = tiles ? b.sc.tblocks : 0u;
-    hipLaunchKernelGGL(tiles ? k_place<true> : k_place<false>, dim3(b.sc.blocks256 + extra), dim3(kHashBlock), 0, s, b.sc, b.key, b.rank, b.range,
-                       b.slot_tmp, b.crowd, b.crowd_count, b.crowd_cap, b.error_flag, tile_work(b, tiles));
+    hipLaunchKernelGGL(tiles ? k_place<true> : k_place<false>, dim3(b.sc.blocks256 + extra), dim3(kHashBlock), 0, s,
+                       b.sc, b.key, b.rank, b.range, b.slot_tmp, b.crowd, b.crowd_count, b.crowd_cap, b.error_flag,
+                       tile_work(b, tiles));
     return hipGetLastError();
 }
 
@@ -2793,9 +2819,10 @@ hipError_t launch_gather(const DeviceBuffers& b, const TileShape* tiles, hipStre
     if (b.sc.blocks256 == 0) return hipSuccess;
     static_assert(kCrowdBlocks % kNumXcd == 0, "the leading workgroups keep the XCD mapping of the others");
     const unsigned extra = tiles ? tile_grid(b) : 0u;
-    hipLaunchKernelGGL(tiles ? k_gather<true> : k_gather<false>, dim3(b.sc.blocks256 + kCrowdBlocks + extra), dim3(kHashBlock), 0, s, b.sc, b.slot_tmp, b.key,
-                       b.range, b.posrho[0], b.velp[0], b.posrho[1], b.velp[1], b.sorted, b.skey, b.ids[0],
-                       b.ids[1], b.rho_max + 1, b.crowd, b.crowd_count, b.crowd_cap, tile_work(b, tiles));
+    hipLaunchKernelGGL(tiles ? k_gather<true> : k_gather<false>, dim3(b.sc.blocks256 + kCrowdBlocks + extra),
+                       dim3(kHashBlock), 0, s, b.sc, b.slot_tmp, b.key, b.range, b.posrho[0], b.velp[0], b.posrho[1],
+                       b.velp[1], b.sorted, b.skey, b.ids[0], b.ids[1], b.rho_max + 1, b.crowd, b.crowd_count,
+                       b.crowd_cap, tile_work(b, tiles));
     return hipGetLastError();
 }
 
@@ -2880,13 +2907,15 @@ hipError_t launch_update(const DeviceBuffers& b, int v, bool list, hipStream_t s
 template <int BLOCK, int CAP, int WPE>
 static void density_tile(const DeviceBuffers& b, bool list, hipStream_t s) {
     if (list)
-        hipLaunchKernelGGL((k_density_tile<BLOCK, CAP, WPE, true>), dim3(tile_grid(b)), dim3(BLOCK), 0, s, b.sc, b.tiles,
-                           b.tile_count, b.tile_cap, reinterpret_cast<const BoxTable*>(b.tables), b.table_cap, b.sparse, b.posrho[1], b.velp[1], b.skey, b.range, b.rho_max, b.llist,
-                           b.lcount, b.list_cap, b.list_chunks, b.nlist, b.ncount);
+        hipLaunchKernelGGL((k_density_tile<BLOCK, CAP, WPE, true>), dim3(tile_grid(b)), dim3(BLOCK), 0, s, b.sc,
+                           b.tiles, b.tile_count, b.tile_cap, reinterpret_cast<const BoxTable*>(b.tables), b.table_cap,
+                           b.sparse, b.posrho[1], b.velp[1], b.skey, b.range, b.rho_max, b.llist, b.lcount, b.list_cap,
+                           b.list_chunks, b.nlist, b.ncount);
     else
-        hipLaunchKernelGGL((k_density_tile<BLOCK, CAP, WPE, false>), dim3(tile_grid(b)), dim3(BLOCK), 0, s, b.sc, b.tiles,
-                           b.tile_count, b.tile_cap, reinterpret_cast<const BoxTable*>(b.tables), b.table_cap, b.sparse, b.posrho[1], b.velp[1], b.skey, b.range, b.rho_max, b.llist,
-                           b.lcount, b.list_cap, b.list_chunks, nullptr, nullptr);
+        hipLaunchKernelGGL((k_density_tile<BLOCK, CAP, WPE, false>), dim3(tile_grid(b)), dim3(BLOCK), 0, s, b.sc,
+                           b.tiles, b.tile_count, b.tile_cap, reinterpret_cast<const BoxTable*>(b.tables), b.table_cap,
+                           b.sparse, b.posrho[1], b.velp[1], b.skey, b.range, b.rho_max, b.llist, b.lcount, b.list_cap,
+                           b.list_chunks, nullptr, nullptr);
 }
 
 hipError_t launch_density_tile(const DeviceBuffers& b, const TileShape& t, bool list, hipStream_t s) {
@@ -2901,8 +2930,9 @@ hipError_t launch_density_tile(const DeviceBuffers& b, const TileShape& t, bool 
 template <int BLOCK, int CAP, int WPE, int MODE>
 static void update_tile(const DeviceBuffers& b, const TileUpdate& u, hipStream_t s) {
     hipLaunchKernelGGL((k_update_tile<BLOCK, CAP, WPE, MODE>), dim3(tile_grid(b)), dim3(BLOCK), 0, s, b.sc, b.tiles,
-                       b.tile_count, b.tile_cap, reinterpret_cast<const BoxTable*>(b.tables), b.table_cap, b.sparse, b.posrho[1], b.velp[1], b.skey, b.range, b.posrho[0], b.velp[0],
-                       b.scene_done, b.ids[1], b.ids[0], b.llist, b.lcount, b.list_cap, b.list_chunks, b.rho_max + 1, u.dt,
+                       b.tile_count, b.tile_cap, reinterpret_cast<const BoxTable*>(b.tables), b.table_cap, b.sparse,
+                       b.posrho[1], b.velp[1], b.skey, b.range, b.posrho[0], b.velp[0], b.scene_done, b.ids[1],
+                       b.ids[0], b.llist, b.lcount, b.list_cap, b.list_chunks, b.rho_max + 1, u.dt,
                        reinterpret_cast<const float4*>(u.corr), u.corr_scale, reinterpret_cast<float4*>(u.acc_out),
                        u.substeps, u.backup);
 }

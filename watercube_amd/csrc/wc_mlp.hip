@@ -217,8 +217,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int block, uint16_t
 
 // Bias gradients, first part: sums of D's columns (M x N, bf16) over chunks of kColsumRows rows, 64 columns
 // and 4 row groups a workgroup, in a fixed order.
-__device__ __forceinline__ void column_sums(const uint16_t* __restrict__ D, float* __restrict__ part, int M, int N, int block,
-                                            float* red) {
+__device__ __forceinline__ void column_sums(const uint16_t* __restrict__ D, float* __restrict__ part, int M, int N,
+                                            int block, float* red) {
     const int l = threadIdx.x & 63, g = threadIdx.x >> 6, nx = (N + 63) / 64;
     const int c = block % nx * 64 + l, chunk = block / nx, r0 = chunk * kColsumRows;
     const int r1 = min(M, r0 + kColsumRows);
@@ -241,8 +241,8 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
 
 // A layer's weight gradient H^T D, split over the rows of the batch, its bias gradient's partial sums and the
 // layer below's delta, all from D.
-__global__ __launch_bounds__(256) void k_gemm_backward(GemmArgs weights, int weight_blocks, GemmArgs delta, int delta_blocks,
-                                                       float* colpart) {
+__global__ __launch_bounds__(256) void k_gemm_backward(GemmArgs weights, int weight_blocks, GemmArgs delta,
+                                                       int delta_blocks, float* colpart) {
     __shared__ __attribute__((aligned(16))) uint16_t As[kGemmTile * kGemmLdk];
     __shared__ __attribute__((aligned(16))) uint16_t Bs[kGemmTile * kGemmLdk];
     const int block = (int)blockIdx.x;
@@ -587,7 +587,8 @@ __device__ __forceinline__ void fetch_entries(RowFetch& f, const ClosureRows& cr
     // (step stride), one selected address advanced per entry rather than a branch per source
     const bool sel = f.listed > 32u;
     const size_t step = sel ? (size_t)1 : cr.stride;
-    const uint32_t* src = (sel ? cr.sel + (size_t)f.row * kSelRow : cr.nlist + f.row) + (size_t)(kLaneNeighbours * q4) * step;
+    const uint32_t* src =
+        (sel ? cr.sel + (size_t)f.row * kSelRow : cr.nlist + f.row) + (size_t)(kLaneNeighbours * q4) * step;
 #pragma unroll
     for (int i = 0; i < kLaneNeighbours; ++i) {
         f.e[i] = *src;
@@ -703,8 +704,8 @@ inline unsigned nblk(long n, int per) { return (unsigned)((n + per - 1) / per); 
 // Host side
 // ------------------------------------------------------------------------------------------
 // M x N product with K in `splits`; the caller fills in the epilogue's operands.
-static GemmArgs gemm_args(const uint16_t* A, long sam, long sak, const uint16_t* B, long sbk, long sbn, int M, int N, int K,
-                          int splits) {
+static GemmArgs gemm_args(const uint16_t* A, long sam, long sak, const uint16_t* B, long sbk, long sbn, int M, int N,
+                          int K, int splits) {
     GemmArgs g{};
     g.A = A, g.B = B;
     g.sam = sam, g.sak = sak, g.sbk = sbk, g.sbn = sbn;

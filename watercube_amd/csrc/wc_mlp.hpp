@@ -40,7 +40,8 @@ struct Mlp {
     uint16_t* d[2] = {nullptr, nullptr};           // hidden deltas (bf16, 128 columns), in turn
     float* loss = nullptr;                         // sum of squared errors of the last batch
     float* colpart[4] = {nullptr, nullptr, nullptr, nullptr};  // column sums per kColsumRows rows, of each layer
-    float* wpart = nullptr;                        // weight gradients of each split of the batch, kMlpSplits of every layer
+    // weight gradients of each split of the batch, kMlpSplits of every layer
+    float* wpart = nullptr;                      
     hipStream_t stream = nullptr;
     int device = 0;
 };
