@@ -389,9 +389,9 @@ void release_tiles(wc_ctx* c) {
     c->tile_ok = c->tiles_ok = c->llist_ok = c->lists_owed = false;
 }
 
-// The tile passes' buffers, allocated before the first sort that feeds those passes (a context that never runs them
-// holds none), and again if a change of parameters asks for more.  Not under capture.  tile_ok says whether they are
-// there.
+// The tile passes' buffers: allocated when a context starts with those passes or is tuned to them, not under capture and
+// not by its first step (0.1 to 0.4 ms); again if a change of parameters asks for more; given back when it is tuned to
+// other passes.  tile_ok says whether they are there.
 hipError_t ensure_tiles(wc_ctx* c) {
     c->tile_ok = false;
     if (!c->tile_fit || c->tile_refused) return hipSuccess;
@@ -435,7 +435,7 @@ hipError_t ensure_tiles(wc_ctx* c) {
     c->tile_ok = true;
     return hipMemsetAsync(b.tile_count, 0, count_bytes, c->stream);
 }
-// ... if the current tuning runs those passes.  Before a sort is queued.
+// ... if the current tuning runs those passes.  Before a sort is queued: parameters may have changed.
 hipError_t prepare_tiles(wc_ctx* c) { return c->density_variant == wc::tile_variant() ? ensure_tiles(c) : hipSuccess; }
 
 bool density_by_tiles(const wc_ctx* c) { return c->tile_ok && c->density_variant == wc::tile_variant(); }
@@ -621,6 +621,7 @@ int create_context(const wc_params* scenes, uint32_t num, wc_ctx** out) {
         return fail(WC_ERR_HIP, "buffer initialisation failed: %s", hipGetErrorString(e));
     }
     rc = upload_tables(c);
+    if (!rc && prepare_tiles(c) != hipSuccess) rc = fail(WC_ERR_HIP, "tile buffers");
     if (rc) {
         destroy_ctx(c);
         return rc;
@@ -1238,12 +1239,18 @@ WC_API int wc_set_tuning(wc_ctx* c, const wc_tuning* t) {
         const int ra = ensure_neighbour_lists(c);
         if (ra) return ra;
     }
-    if (!t->neighbour_list) WC_HIP(refresh_lists(c, false));
+    const bool release = c->tile_mem && t->density_variant != wc::tile_variant();
+    if (!t->neighbour_list || release) WC_HIP(refresh_lists(c, false));
     c->density_variant = t->density_variant;
     c->update_variant = t->update_variant;
     c->neighbour_list = t->neighbour_list != 0;
     c->tile_refused = false;
     drop_graph(c);
+    if (release) {
+        WC_HIP(hipStreamSynchronize(c->stream));
+        release_tiles(c);
+    }
+    WC_HIP(prepare_tiles(c));
     return WC_OK;
 }
 
