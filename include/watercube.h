@@ -278,8 +278,9 @@ WC_API const char* wc_pass_name(int k);
  * bit-identical results, only speed differs.  Contexts of 50,000 particles and more, and of 20,000 a
  * scene, start with the last variant if at rest density boxes fit LDS and lists hold the neighbours,
  * others with variant 2: the parameters alone decide, so a state far from rest (a thin gas, say) may
- * be faster by what wc_tune finds for it.  Only
- * contexts tuned to the last variant hold its buffers (2 KB a particle and more).  No reference counterpart: the reference dispatches
+ * be faster by what wc_tune finds for it.  Only contexts that run the last variant hold its buffers
+ * (2 KB a particle and more); tuned to another, one gives them back in the next call that waits for
+ * it (wc_synchronize, an upload or download).  No reference counterpart: the reference dispatches
  * fixed 128-invocation work groups (src/core/util.h:18). */
 typedef struct wc_tuning {
     int32_t density_variant;

@@ -434,3 +434,28 @@ def test_parameters_that_change_the_box_shape(oracle):
             f.synchronize()
             got = f.particles(1)
             assert np.array_equal(got.view(np.uint32), st.buf1.view(np.uint32)), f"ratio {ratio}"
+
+
+@pytest.mark.parametrize("n_side", [(40, 40, 40), (20, 20, 20)])
+def test_steps_captured_before_the_buffers_go(n_side):
+    """A context tuned away from the tile passes gives their buffers back when it next waits; steps captured before that,
+    and after, hold no address of them.  The same bits as a context that never had them."""
+    p, parts = scaled_block(n_side, 0.0175, 1)
+    tile = L.lib().wc_num_variants() - 1
+    with Fluid(p, parts) as a, Fluid(p, parts) as b:
+        print(f"case buffers given back, {len(parts)} particles", flush=True)
+        b.set_tuning(2, 2, 1)
+        a.set_tuning(tile, tile, 1)
+        a.step(2e-5, 3)
+        a.set_tuning(2, 2, 1)
+        a.step(2e-5, 9)   # captured with the buffers there
+        b.step(2e-5, 12)
+        a.synchronize()   # gives them back
+        a.step(2e-5, 9)   # replayed or captured again
+        a.synchronize()
+        a.set_tuning(tile, tile, 0)
+        a.step(2e-5, 9)
+        b.step(2e-5, 18)
+        a.synchronize()
+        b.synchronize()
+        assert a.particles(1).tobytes() == b.particles(1).tobytes()

@@ -381,7 +381,9 @@ int ensure_neighbour_lists(wc_ctx* c) {
     return WC_OK;
 }
 
+// Frees the tile passes' buffers; the caller has waited for the stream.  Captured graphs go first: they hold addresses.
 void release_tiles(wc_ctx* c) {
+    drop_graph(c);
     if (c->tile_mem) (void)hipFree(c->tile_mem);
     c->tile_mem = nullptr;
     c->b.tiles = nullptr;
@@ -389,9 +391,9 @@ void release_tiles(wc_ctx* c) {
     c->tile_ok = c->tiles_ok = c->llist_ok = c->lists_owed = false;
 }
 
-// The tile passes' buffers: allocated when a context starts with those passes or is tuned to them, not under capture and
-// not by its first step (0.1 to 0.4 ms); again if a change of parameters asks for more; given back when it is tuned to
-// other passes.  tile_ok says whether they are there.
+// The tile passes' buffers: allocated when a context starts with those passes or is tuned to them (not by its first step:
+// that takes 0.1 to 0.4 ms), and again if a change of parameters asks for more.  Not under capture.  tile_ok says whether
+// they are there.
 hipError_t ensure_tiles(wc_ctx* c) {
     c->tile_ok = false;
     if (!c->tile_fit || c->tile_refused) return hipSuccess;
@@ -403,7 +405,6 @@ hipError_t ensure_tiles(wc_ctx* c) {
     if (c->tile_ok) return hipSuccess;
     hipError_t e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return e;
-    drop_graph(c);
     release_tiles(c);
     // Only with room left for what a caller may ask for later, about 1 KB a particle (neighbour lists, a learned step's
     // workspace): else the context keeps the per-particle passes.
@@ -437,6 +438,10 @@ hipError_t ensure_tiles(wc_ctx* c) {
 }
 // ... if the current tuning runs those passes.  Before a sort is queued: parameters may have changed.
 hipError_t prepare_tiles(wc_ctx* c) { return c->density_variant == wc::tile_variant() ? ensure_tiles(c) : hipSuccess; }
+// Gives back the buffers of a context that is tuned to other passes, in a call that has waited for its stream (0.3 ms).
+void release_idle_tiles(wc_ctx* c) {
+    if (c->tile_mem && c->density_variant != wc::tile_variant() && !c->lists_owed) release_tiles(c);
+}
 
 bool density_by_tiles(const wc_ctx* c) { return c->tile_ok && c->density_variant == wc::tile_variant(); }
 bool update_by_tiles(const wc_ctx* c) { return density_by_tiles(c) && c->update_variant == wc::tile_variant(); }
@@ -458,7 +463,7 @@ void note_step(wc_ctx* c) {
 // The kernels of a sort, in order, each followed by after(k) (k-th of the passes wc_pass_name names).
 template <typename After>
 hipError_t launch_sort(wc_ctx* c, bool tiles, After after) {
-    hipError_t e = wc::launch_hash(c->b, c->stream);
+    hipError_t e = wc::launch_hash(c->b, tiles, c->stream);
     if (e == hipSuccess) e = after(0);
     if (e == hipSuccess) e = wc::launch_scan(c->b, c->stream);
     if (e == hipSuccess) e = after(1);
@@ -712,6 +717,7 @@ int copy_records_in(wc_ctx* c, uint32_t first, const wc_particle* host, uint32_t
     c->tiles_ok = c->llist_ok = c->nlist_ok = c->lists_owed = false;
     WC_HIP(wc::launch_invalidate(c->b, c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
+    release_idle_tiles(c);
     return WC_OK;
 }
 
@@ -725,6 +731,7 @@ int copy_records_out(wc_ctx* c, int which, uint32_t first, wc_particle* host, ui
     WC_HIP(hipMemcpyAsync(host, c->staging + first, (size_t)n * sizeof(wc_particle), hipMemcpyDeviceToHost,
                           c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
+    release_idle_tiles(c);
     return WC_OK;
 }
 
@@ -1084,7 +1091,7 @@ WC_API int wc_step_noalloc(const wc_params* p, float dt, void* posrho, void* vel
     v.blocks128 = tables[3];
     v.blocks256 = tables[5];
     WC_HIP(wc::launch_noalloc_setup(d, tables, d_desc, d_tables, b.counts, (uint32_t)ncells, b.error_flag, s));
-    WC_HIP(wc::launch_hash(b, s));
+    WC_HIP(wc::launch_hash(b, false, s));
     WC_HIP(wc::launch_scan(b, s));
     WC_HIP(wc::launch_place(b, nullptr, s));
     WC_HIP(wc::launch_gather(b, nullptr, s));
@@ -1110,6 +1117,7 @@ WC_API int wc_synchronize(wc_ctx* c) {
     int rc = set_device(c);
     if (rc) return rc;
     WC_HIP(hipStreamSynchronize(c->stream));
+    release_idle_tiles(c);
     uint32_t flag = 0;
     WC_HIP(hipMemcpy(&flag, c->b.error_flag, 4, hipMemcpyDeviceToHost));
     if (flag) return fail(WC_ERR_DEVICE_FAULT, "scan look-back exceeded its bounded wait (flag %u)", flag);
@@ -1239,17 +1247,12 @@ WC_API int wc_set_tuning(wc_ctx* c, const wc_tuning* t) {
         const int ra = ensure_neighbour_lists(c);
         if (ra) return ra;
     }
-    const bool release = c->tile_mem && t->density_variant != wc::tile_variant();
-    if (!t->neighbour_list || release) WC_HIP(refresh_lists(c, false));
+    if (!t->neighbour_list) WC_HIP(refresh_lists(c, false));
     c->density_variant = t->density_variant;
     c->update_variant = t->update_variant;
     c->neighbour_list = t->neighbour_list != 0;
     c->tile_refused = false;
     drop_graph(c);
-    if (release) {
-        WC_HIP(hipStreamSynchronize(c->stream));
-        release_tiles(c);
-    }
     WC_HIP(prepare_tiles(c));
     return WC_OK;
 }
@@ -1369,16 +1372,13 @@ WC_API int wc_tune(wc_ctx* c, float dt, uint32_t reps, wc_tuning* chosen, double
         restore();
         use(err == hipSuccess ? pick : before);
         drop_graph(c);
-        if (err == hipSuccess && c->tile_mem && c->density_variant != wc::tile_variant()) {
-            err = hipStreamSynchronize(c->stream);
-            release_tiles(c);
-        }
         if (err == hipSuccess) err = launch_sort(c, density_by_tiles(c), [](int) { return hipSuccess; });
         if (err == hipSuccess)
             err = density_by_tiles(c) ? launch_density_pass(c, true)
                                       : wc::launch_density(c->b, particle_variant(c->density_variant), true, c->stream);
         c->nlist_ok = err == hipSuccess;
         if (err == hipSuccess) err = hipStreamSynchronize(c->stream);
+        if (err == hipSuccess) release_idle_tiles(c);
         (void)hipFree(save_pos);
         (void)hipFree(save_vel);
         if (save_ids) (void)hipFree(save_ids);

@@ -206,7 +206,8 @@ constexpr size_t kTileTableBytes = 1824;     // cell table of a box
 inline uint64_t tile_capacity(uint64_t tiles, uint64_t particles) { return tiles + particles / 4 + 64; }
 
 // Kernel launchers (wc_kernels.hip).  Each enqueues on `stream` and returns the launch status.
-hipError_t launch_hash(const DeviceBuffers& b, hipStream_t stream);
+// `tiles`: the sort feeds the tile passes, whose counters the hash resets; others hold no address of their buffers.
+hipError_t launch_hash(const DeviceBuffers& b, bool tiles, hipStream_t stream);
 hipError_t launch_scan(const DeviceBuffers& b, hipStream_t stream);
 // With `tiles`, the two also form the tile passes' work list and tables for that shape.
 hipError_t launch_place(const DeviceBuffers& b, const TileShape* tiles, hipStream_t stream);

@@ -2766,14 +2766,15 @@ inline unsigned blocks_for(size_t n, unsigned per) { return (unsigned)((n + per 
 
 }  // namespace
 
-hipError_t launch_hash(const DeviceBuffers& b, hipStream_t s) {
+hipError_t launch_hash(const DeviceBuffers& b, bool tiles, hipStream_t s) {
     const Scenes& S = b.sc;
     size_t blocks = S.blocks256;
     const size_t reset = blocks_for(S.total_tiles > S.num_scenes ? S.total_tiles : S.num_scenes, kHashBlock);
     if (reset > blocks) blocks = reset;
     if (blocks == 0) blocks = 1;  // still resets the step clock
     hipLaunchKernelGGL(k_hash, dim3((unsigned)blocks), dim3(kHashBlock), 0, s, S, b.posrho[0], b.key, b.rank,
-                       b.counts, b.scan_status, b.scene_done, b.step_start, b.rho_max, b.crowd_count, b.tile_count);
+                       b.counts, b.scan_status, b.scene_done, b.step_start, b.rho_max, b.crowd_count,
+                       tiles ? b.tile_count : nullptr);
     return hipGetLastError();
 }
 
