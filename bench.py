@@ -181,8 +181,14 @@ def scale_section(steps: int, warmup: int = 5) -> dict:
     return {"workload": "block_sphere_17m", "particles": n, "grid_res": int(p.grid_res), "steps": steps,
             "value": n * steps / elapsed, "unit": "particle-steps/s", "ms_per_step": elapsed * 1e3 / steps,
             "pass_ms": {k: v / 5 for k, v in prof.items()},
-            "tuning": [tuning["variants"][tuning["density_variant"]], tuning["variants"][tuning["update_variant"]],
+            "tuning": [variant_text(tuning, "density_variant"), variant_text(tuning, "update_variant"),
                        tuning["neighbour_list"]]}
+
+
+def variant_text(tuning: dict, which: str):
+    """The picked variant's description; the last one is no particle per lane."""
+    v = tuning["variants"][tuning[which]]
+    return list(v) if any(v) else "boxes of cells"
 
 
 def learned_section(p, parts, dt, weights: Path, horizon: int = 500, reps: int = 20) -> dict:
@@ -311,8 +317,8 @@ def main() -> int:
 
     with Fluid(p, parts) as f:
         tuning = f.tune(dt, reps=5)  # untimed: picks the fastest variant of each neighbour pass
-        print(f"# tuned variants: density {tuning['variants'][tuning['density_variant']]} "
-              f"update {tuning['variants'][tuning['update_variant']]} neighbour lists {tuning['neighbour_list']}",
+        print(f"# tuned variants: density {variant_text(tuning, 'density_variant')} "
+              f"update {variant_text(tuning, 'update_variant')} neighbour lists {tuning['neighbour_list']}",
               file=sys.stderr, flush=True)
         print("# variant ms density: " + " ".join(f"{x:.4f}" for x in tuning["density_ms"]) +
               " | update: " + " ".join(f"{x:.4f}" for x in tuning["update_ms"]), file=sys.stderr, flush=True)
@@ -392,8 +398,8 @@ def main() -> int:
         "data": "synthetic",
         "config": {"workload": WORKLOAD, "particles": n, "grid_res": int(p.grid_res), "dt": dt,
                    "method": "plain", "kernel_radius": float(p.kernel_radius),
-                   "tuning": {"density": tuning["variants"][tuning["density_variant"]],
-                              "update": tuning["variants"][tuning["update_variant"]],
+                   "tuning": {"density": variant_text(tuning, "density_variant"),
+                              "update": variant_text(tuning, "update_variant"),
                               "neighbour_list": tuning["neighbour_list"]}},
         "simulated_s_per_s": dt * args.steps / elapsed,
         "pass_ms": per_launch_ms,

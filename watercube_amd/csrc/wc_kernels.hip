@@ -1451,7 +1451,7 @@ __global__ __launch_bounds__(BLOCK) void k_update(Scenes S, const float4* __rest
 //
 // Measured against those (us, density + force): the 80,000-particle scene 120 + 202 -> 92 + 64, 192,089
 // particles 90 + 125 -> 84 + 57, the million-particle block 265 + 217 -> 163 + 117, 17.8 million
-// 3,582 + 3,762 -> 2,107 + 1,710; the work list and tables cost the sort 17 us of the million's step.
+// 3,582 + 3,762 -> 2,107 + 1,710; the work list and tables cost the sort 20 us of the million's step.
 //
 // The density pass is bound by VALU issue and, below 4 boxes a CU, by its chain of dependent loads; the force
 // pass by LDS reads (32 bytes a neighbour) and arithmetic.  512 threads and 1,920 records let three density
