@@ -1,5 +1,5 @@
-// wc_choose.hpp -- choices by size and density, as plain functions of numbers: the box shape of the tile passes and
-// whether a context starts with them.  Host code without HIP.
+// wc_choose.hpp -- choices by size, density and times, as plain functions of numbers: the box shape of the tile passes,
+// whether a context starts with them, which boxes are thin, and the tuner's candidates.  Host code without HIP.
 #pragma once
 
 #include <stddef.h>
@@ -49,7 +49,7 @@ inline SceneFill scene_fill(uint32_t n, int grid_res, double bin, double h, doub
 // 4x3x4 / 4x2x4 / 2x2x4 (us): 91,125 particles 141 / 130 / 104, 125,000 126 / 137 / 137, 262,144 141 / 158 / 176: the
 // first from 300 boxes of it.  At 12 a cell, where it does not fit, by 4x2x4 / 2x2x4: 125,000 182 / 135, 192,089 (once
 // spread, three at once) 94 / 111, 2,048,000 1,087 / 1,109: the second from 450 boxes.  Up to 16 a cell 2x2x4
-// otherwise. Above, where a box of it has more particles than threads, by 2x2x4 / 2x2x2: 59,319 (20 a cell) 192 / 143,
+// otherwise.  Above, where a box of it has more particles than threads, by 2x2x4 / 2x2x2: 59,319 (20 a cell) 192 / 143,
 // 125,000 (20) 249 / 234, 343,000 (19) 553 / 542, 704,969 (17) 969 / 1,071, 1,000,000 (19) 1,321 / 1,388, 4,492,125
 // (19) 5,762 / 6,093: 2x2x2 below 2,000 boxes of 2x2x4.
 inline TileShape choose_tile_shape(const std::vector<SceneFill>& scenes) {

@@ -170,13 +170,12 @@ struct PassVariant {
 int num_variants();
 PassVariant variant(int v);
 
-int tile_variant();
-// What the sort forms for them.
+int tile_variant();  // the last: the tile passes (TileShape, wc_choose.hpp)
+// What the sort forms for the tile passes.
 struct TileWork {
     uint4* tiles;     // work list
     // its entries; [1]: slots in `sparse` of a single scene; [kListCount]: list chunks; with several scenes,
-    // [kSceneSparse + s]: scene s's slots in `sparse` (from its first particle on), [kSceneSparse - 1]: entries of
-    // those
+    // [kSceneSparse + s]: scene s's slots in `sparse` (from its first particle on), [kSceneSparse - 1]: their entries
     uint32_t* count;
     uint32_t cap;
     uint32_t rec_cap;  // records a box may stage
